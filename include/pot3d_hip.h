@@ -145,15 +145,16 @@ enum {
                                 the mixed-precision recurrence (x rounded to
                                 float, the result in float); 0 FP64 */
   P3D_OPT_FUSE_RESIDUAL = 17, /* FP32 recurrence with the register-tile ILU
-                                sweeps (P3D_OPT_TILE_STAGE 2): 1 folds the
+                                sweeps (P3D_OPT_TILE_STAGE 2) or the column
+                                sweeps (P3D_OPT_COLUMN): 1 folds the
                                 residual update r -= alpha Ap into the
                                 forward sweep, 0 runs it on its own; -1
-                                (default) 1 when N >= 2^26 unknowns (the
-                                sweeps are then bandwidth-bound and the
-                                fold saves a pass; below, they are
-                                latency-bound and it costs).  Same values
-                                bit for bit. */
-  P3D_OPT_BLOCK_SWEEP = 18   /* block-Jacobi ILU on register tiles
+                                (default) 1 with the column sweeps and when
+                                N >= 2^26 unknowns (the tiles are then
+                                bandwidth-bound and the fold saves a pass;
+                                below, they are latency-bound and it
+                                costs).  Same values bit for bit. */
+  P3D_OPT_BLOCK_SWEEP = 18,  /* block-Jacobi ILU on register tiles
                                 (P3D_OPT_TILE_STAGE 2 with a cut): 1 runs
                                 each sweep as one launch, a workgroup per
                                 block marching the block's tile diagonals;
@@ -163,6 +164,14 @@ enum {
                                 launch per diagonal over all blocks; -1
                                 (default) 1 below 2^26 unknowns, else 0.
                                 Same values bit for bit. */
+  P3D_OPT_COLUMN = 19        /* 8x8 columns of one wave: 1 runs each ILU sweep
+                                as one launch, a workgroup per column of
+                                points marching all planes and handing its
+                                faces to the next columns as it goes; 0 the
+                                tile schedules above; -1 (default) 1, but 0
+                                while P3D_OPT_BLOCK_SWEEP is not -1 and for
+                                block-Jacobi register tiles of 2^22 to 2^25
+                                unknowns.  Same values bit for bit. */
 };
 
 /* Creates a solver for one rank's grid (nr,nt,np include the boundary /

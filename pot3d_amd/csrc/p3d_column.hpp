@@ -1,0 +1,60 @@
+// D-ILU triangular solves by columns, one launch per sweep (p3d_column.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "p3d_internal.hpp"
+
+namespace p3d {
+
+// LDS of one column at most (beyond about 5000 planes: the tile schedules)
+constexpr size_t kColLdsMax = 64 * 1024;
+
+struct ColArgs {
+  int NI = 0, NJ = 0, c = 0;  // columns of 8x8 points, planes
+  int tk_log2 = 0, planes = 0;  // tile-major placement of r and z (TileMap)
+  int rounds = 0;               // rounds of 32 steps
+  int rows_alloc = 0;           // rows of a column in dinv_s and y_s
+  int face_rows = 0;            // rows of a column's faces
+  int pf_n = 0;                 // entries of the phi-factor tables
+  int skip = 0;                 // steps before the backward sweep's first plane
+  int mode = 0;                 // phi factors: by plane, equal but for the cut, equal
+  float u_d = 0.f, u_k = 0.f;   // the equal FDPH, FDPL = FDPU
+  IluBlocks bl{};
+  const int* order = nullptr;      // columns by anti-diagonal inside their block
+  const float* dinv_s = nullptr;   // [column][row][lane]: plane row - 32 - ii - 2 jj
+  float* y_s = nullptr;            // the forward result, placed as dinv_s
+  unsigned long long* face_i = nullptr;  // [column][row][8]: {value, stamp} of the step row - 8
+  unsigned long long* face_j = nullptr;
+  const float2* pf_lo = nullptr;  // (FDPH, FDPL) by plane + 21, zero outside
+  const float2* pf_up = nullptr;  // (FDPH, FDPU) from plane c + skip - 1 downwards, likewise
+  unsigned* ctr = nullptr;        // stamps of the next forward, backward sweep; failure flag
+  void* dummy = nullptr;          // where rows outside the vectors are stored
+};
+
+struct ColumnPlan {
+  int ready = 0;
+  ColArgs a;
+  int* order = nullptr;
+  float *dinv_s = nullptr, *y_s = nullptr;
+  unsigned long long* face = nullptr;
+  float2* pf = nullptr;
+  unsigned* ctr = nullptr;
+  void* dummy = nullptr;
+};
+
+// dinv: the D-ILU's inverse pivots in natural order; tk_log2: planes per
+// tile of the r and z placement.  Returns 0 when the sweeps can run.
+int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
+                      int tk_log2, const float* dinv);
+void free_column_plan(ColumnPlan& plan);
+
+// z = (LU)^-1 r on tile-major r and z, two launches.  ap (FP32, with guard):
+// r -= alpha ap first, alpha from guard.
+template <typename T>
+void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g, T* r, T* z,
+                         const CgState* guard, const float* ap, hipStream_t s);
+
+// Device word that is not 0 once a wait of a column sweep ran into its bound.
+const unsigned* column_failure_flag(const ColumnPlan& plan);
+
+}  // namespace p3d

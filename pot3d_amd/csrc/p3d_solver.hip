@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/pot3d_hip.h"
+#include "p3d_column.hpp"
 #include "p3d_kernels.hpp"
 #include "p3d_sweep.hpp"
 
@@ -102,6 +103,8 @@ struct p3d_solver {
   int eG = 0;
   SweepPlan sweep;
   bool sweep_ready = false;
+  ColumnPlan col;
+  bool col_tried = false;  // col is the current plan, or there is none
   // options
   int stop_mode = 0;
   int mixed = 0;
@@ -115,6 +118,7 @@ struct p3d_solver {
   int apply_fp32 = 0;  // p3d_apply_A with the FP32 operator
   int fuse_rupd = -1;  // P3D_OPT_FUSE_RESIDUAL
   int blk_sweep = -1;  // P3D_OPT_BLOCK_SWEEP
+  int column = -1;     // P3D_OPT_COLUMN
   IluBlocks blocks{0, 0, 0, 1};  // block-Jacobi cut of the ILU (none by default)
   int nblk[3] = {1, 1, 1};       // blocks per axis (r, theta, phi)
   // graphs: [0] FP64, [1] FP32, [2] FP32 recurrence with the FP64 solution
@@ -224,6 +228,41 @@ static int read_state(p3d_solver* s) {
 }
 
 // ---------------------------------------------------------------------------
+// The column sweeps are to run instead of the tile schedules.  By themselves
+// (P3D_OPT_COLUMN -1) wherever they apply, unless P3D_OPT_BLOCK_SWEEP asks for
+// a tile schedule, or the register tiles of a block-Jacobi cut run
+// block-persistent between 2^22 and 2^25 unknowns: FP32 apply, tiles against
+// columns, 64 and 51 us at 0.8 M unknowns, 72 and 73 at 6.4 M (a whole FP64
+// solve 164 and 170 ms), 94 and 100 at 13.6 M, 183 and 199 at 26.8 M, 366 and
+// 361 at 46.4 M, 1429 and 1423 at 214.7 M.  Without a cut the tiles' one
+// launch per diagonal is never near: FP64 apply, tiles and columns, 350 and
+// 100 us at 0.8 M, 1383 and 410 at 26.8 M, 4977 and 1864 at 214.7 M.
+static bool columns_wanted(const p3d_solver* s) {
+  if (s->ifprec != PREC_ILU || s->sweep_mode != 0 || !s->tm.on) return false;
+  if (s->column >= 0) return s->column != 0;
+  if (s->blk_sweep >= 0) return false;
+  const bool tiles_win = s->sweep.blocked && s->sweep.stage_one == 2 && s->g.N >= (1u << 22) &&
+                         s->g.N < (1u << 25);
+  return !tiles_win;
+}
+static bool columns_on(const p3d_solver* s) { return columns_wanted(s) && s->col.ready; }
+
+// Builds the column sweeps' plan for the current pivots, cut and placement
+// before a call that applies the ILU (every option that changes one of them
+// drops it).  Without a plan (no memory for it, too many planes) the tile
+// schedules run.
+static void ensure_columns(p3d_solver* s) {
+  if (!columns_wanted(s) || s->col_tried) return;
+  s->col_tried = true;
+  build_column_plan(s->col, s->m, s->g, s->blocks, s->tm.tk_log2, s->dinv);
+}
+
+// Whether the FP32 ILU apply can take the residual update (see cg_iteration).
+static bool fuse_rupd_available(const p3d_solver* s) {
+  return columns_on(s) ||
+         (s->sweep_mode == 0 && s->sweep_ready && dilu_tiles_fuse_rupd(s->sweep));
+}
+
 // Preconditioner application r -> z (+ fused dots with epilogue).
 // ap_upd (FP32 register tiles, guard set): the residual update r -= alpha ap
 // is folded into the forward sweep (r is written).
@@ -232,7 +271,9 @@ static void prec_and_dot(p3d_solver* s, const T* r, T* z, Epi epi, double* out, 
                          const float* ap_upd = nullptr) {
   if (s->ifprec == PREC_ILU) {
     const CgState* gd = guard ? s->st : nullptr;
-    if (s->sweep_mode == 0 && s->sweep_ready) {
+    if (columns_on(s)) {
+      launch_dilu_columns<T>(s->col, s->m, s->g, const_cast<T*>(r), z, gd, ap_upd, s->stream);
+    } else if (s->sweep_mode == 0 && s->sweep_ready) {
       if constexpr (sizeof(T) == 4) {
         if (ap_upd)
           launch_dilu_tiles_rupd(s->sweep, s->m, s->g, const_cast<float*>(r), ap_upd, z, gd,
@@ -275,8 +316,9 @@ static void cg_iteration(p3d_solver* s, Vecs<T> v, int t) {
                             0, EPI_PAP, nullptr, true, s->stream, s->tm);
       // r -= alpha ap, in the forward sweep of the register tiles where they
       // run, else on its own; then z = M^-1 r and r.z, r.r together
-      const bool fused = (s->fuse_rupd == 1 || (s->fuse_rupd < 0 && s->g.N >= (1u << 26))) &&
-                         s->sweep_mode == 0 && s->sweep_ready && dilu_tiles_fuse_rupd(s->sweep);
+      const bool fused = (s->fuse_rupd == 1 ||
+                          (s->fuse_rupd < 0 && (columns_on(s) || s->g.N >= (1u << 26)))) &&
+                         fuse_rupd_available(s);
       if (!fused) launch_r_update(s->gt.N, s->Lt, v.r, v.ap, s->st, s->stream);
       prec_and_dot<float>(s, v.r, v.z, EPI_RITER, nullptr, true, fused ? v.ap : nullptr);
       launch_p_update_x(s->g, s->L, t, v.pb, v.z, s->st, s->stream, s->tm, v.xs, v.xscale,
@@ -402,6 +444,28 @@ static void print_history(p3d_solver* s, int ncghist) {
   fflush(stdout);
 }
 
+// Whether a column sweep gave up waiting (two threads' sweeps that crowd each
+// other out of the device can do that): its results are void, and the call
+// starts over with the tile schedules (kStartOver).  copy_column_flag goes with the other copies of a
+// result to the host, check_columns after the stream has been waited for.
+static constexpr int kStartOver = -1;
+static void copy_column_flag(p3d_solver* s) {
+  unsigned* f = (unsigned*)(s->out_host + 6);
+  *f = 0;
+  if (columns_on(s))
+    (void)hipMemcpyAsync(f, column_failure_flag(s->col), sizeof *f, hipMemcpyDeviceToHost,
+                         s->stream);
+}
+static int check_columns(p3d_solver* s) {
+  if (*(const unsigned*)(s->out_host + 6) == 0) return P3D_OK;
+  for (int q = 0; q < 3; q++) {
+    if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
+    s->gexec[q] = nullptr;
+  }
+  free_column_plan(s->col);
+  return kStartOver;
+}
+
 static int true_residual(p3d_solver* s, double* rr, double* bb) {
   // ap = b - A x (FP64), reductions into out[0] (r.r), out[2] (b.b)
   launch_pole_sums<double>(s->m, s->g, s->x, s->pole_part, s->stream);
@@ -411,10 +475,11 @@ static int true_residual(p3d_solver* s, double* rr, double* bb) {
                       s->out + 2, false, s->stream);
   HIPCHK(hipMemcpyAsync(s->out_host, s->out, 4 * sizeof(double), hipMemcpyDeviceToHost,
                         s->stream));
+  copy_column_flag(s);
   HIPCHK(hipStreamSynchronize(s->stream));
   *rr = s->out_host[0];
   *bb = s->out_host[2];
-  return P3D_OK;
+  return check_columns(s);
 }
 
 static int status_rc(int done) {
@@ -612,6 +677,7 @@ static int solve_mixed_ru(p3d_solver* s, double epscg, int ncgmax) {
 static int solve_core(p3d_solver* s, double epscg, int ncgmax, int ncghist) {
   int rc;
   auto t0 = std::chrono::steady_clock::now();
+  ensure_columns(s);
   memset(&s->stats, 0, sizeof s->stats);
   if (s->guess_check) {
     // a proposed guess that is worse than the reference's zero guess is
@@ -724,6 +790,7 @@ int p3d_destroy(p3d_solver* s) {
   for (float* b : s->p32b)
     if (b) hipFree(b);
   free_sweep_plan(s->sweep);
+  free_column_plan(s->col);
   if (s->st_host) hipHostFree(s->st_host);
   if (s->out_host) hipHostFree(s->out_host);
   if (s->stream) hipStreamDestroy(s->stream);
@@ -732,6 +799,11 @@ int p3d_destroy(p3d_solver* s) {
 }
 
 static int block_sweep_on(const p3d_solver* s);
+
+static void drop_columns(p3d_solver* s) {
+  free_column_plan(s->col);
+  s->col_tried = false;
+}
 
 int p3d_create(p3d_solver** out, int nr, int nt, int np, const double* r, const double* dr,
                const double* rh, const double* drh, const double* st, const double* dt,
@@ -971,6 +1043,7 @@ static IluBlocks ilu_blocks(const p3d_solver* s) {
 // current tile shape and block-Jacobi cut.
 static int rebuild_ilu(p3d_solver* s, bool refactor) {
   HIPCHK(hipStreamSynchronize(s->stream));
+  drop_columns(s);
   for (int t = 0; t < 3; t++) {
     if (s->gexec[t]) hipGraphExecDestroy(s->gexec[t]);
     s->gexec[t] = nullptr;
@@ -1077,6 +1150,20 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       }
       break;
     }
+    case P3D_OPT_COLUMN: {
+      const int v = (int)value;
+      if (v < -1 || v > 1) return fail(P3D_EINVAL, "P3D_OPT_COLUMN must be -1, 0 or 1");
+      if (v != s->column) {
+        // captured iterations hold the other launch sequence
+        HIPCHK(hipStreamSynchronize(s->stream));
+        for (int q = 0; q < 3; q++) {
+          if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
+          s->gexec[q] = nullptr;
+        }
+        s->column = v;
+      }
+      break;
+    }
     case P3D_OPT_TILE_K:
     case P3D_OPT_TILE_WAVES:
     case P3D_OPT_TILE_STAGE: {
@@ -1158,13 +1245,15 @@ int p3d_solve_dev(p3d_solver* s, double* x_dev, double* rhs_dev, double epscg, i
   if (!(epscg > 0)) return fail(P3D_EINVAL, "epscg must be positive");
   const size_t nb = sizeof(double) * s->g.N;
   int rc;
-  if (rhs_dev) {
-    HIPCHK(hipMemcpyAsync(s->b, rhs_dev, nb, hipMemcpyDeviceToDevice, s->stream));
-  } else if ((rc = make_rhs(s, s->b))) {
-    return rc;
-  }
-  HIPCHK(hipMemcpyAsync(s->x, x_dev, nb, hipMemcpyDeviceToDevice, s->stream));
-  rc = solve_core(s, epscg, ncgmax, 0);
+  do {
+    if (rhs_dev) {
+      HIPCHK(hipMemcpyAsync(s->b, rhs_dev, nb, hipMemcpyDeviceToDevice, s->stream));
+    } else if ((rc = make_rhs(s, s->b))) {
+      return rc;
+    }
+    HIPCHK(hipMemcpyAsync(s->x, x_dev, nb, hipMemcpyDeviceToDevice, s->stream));
+    rc = solve_core(s, epscg, ncgmax, 0);
+  } while (rc == kStartOver);
   HIPCHK(hipMemcpyAsync(x_dev, s->x, nb, hipMemcpyDeviceToDevice, s->stream));
   if (rhs_dev) {
     // the final residual: FP64 recurrence r (natural order via ap), or the
@@ -1184,13 +1273,15 @@ int p3d_solve(p3d_solver* s, double* x, double* rhs, double epscg, int ncgmax, i
   if (!(epscg > 0)) return fail(P3D_EINVAL, "epscg must be positive");
   const size_t nb = sizeof(double) * s->g.N;
   int rc;
-  if (rhs) {
-    HIPCHK(hipMemcpyAsync(s->b, rhs, nb, hipMemcpyHostToDevice, s->stream));
-  } else if ((rc = make_rhs(s, s->b))) {
-    return rc;
-  }
-  HIPCHK(hipMemcpyAsync(s->x, x, nb, hipMemcpyHostToDevice, s->stream));
-  rc = solve_core(s, epscg, ncgmax, ncghist);
+  do {
+    if (rhs) {
+      HIPCHK(hipMemcpyAsync(s->b, rhs, nb, hipMemcpyHostToDevice, s->stream));
+    } else if ((rc = make_rhs(s, s->b))) {
+      return rc;
+    }
+    HIPCHK(hipMemcpyAsync(s->x, x, nb, hipMemcpyHostToDevice, s->stream));
+    rc = solve_core(s, epscg, ncgmax, ncghist);
+  } while (rc == kStartOver);
   HIPCHK(hipMemcpyAsync(x, s->x, nb, hipMemcpyDeviceToHost, s->stream));
   if (rhs) {
     if (!s->mixed) launch_copy<double>(s->g, s->L, s->ap, s->r, s->stream, s->tm, 0);
@@ -1324,12 +1415,17 @@ int p3d_apply_A(p3d_solver* s, const double* x, double* y) {
 int p3d_apply_prec(p3d_solver* s, double* x) {
   if (!s || !x) return fail(P3D_EINVAL, "null argument");
   const size_t nb = sizeof(double) * s->g.N;
-  // x -> r and z -> x through the natural-order staging vector ap
-  HIPCHK(hipMemcpyAsync(s->ap, x, nb, hipMemcpyHostToDevice, s->stream));
-  launch_copy<double>(s->g, s->L, s->r, s->ap, s->stream, s->tm, 1);
-  prec_and_dot<double>(s, s->r, s->z, EPI_NONE, nullptr, false);
-  launch_copy<double>(s->g, s->L, s->ap, s->z, s->stream, s->tm, 0);
-  HIPCHK(hipGetLastError());
+  ensure_columns(s);
+  do {
+    // x -> r and z -> x through the natural-order staging vector ap
+    HIPCHK(hipMemcpyAsync(s->ap, x, nb, hipMemcpyHostToDevice, s->stream));
+    launch_copy<double>(s->g, s->L, s->r, s->ap, s->stream, s->tm, 1);
+    prec_and_dot<double>(s, s->r, s->z, EPI_NONE, nullptr, false);
+    launch_copy<double>(s->g, s->L, s->ap, s->z, s->stream, s->tm, 0);
+    HIPCHK(hipGetLastError());
+    copy_column_flag(s);
+    HIPCHK(hipStreamSynchronize(s->stream));
+  } while (check_columns(s) == kStartOver);
   HIPCHK(hipMemcpyAsync(x, s->ap, nb, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
   return P3D_OK;
@@ -1344,12 +1440,13 @@ int p3d_ilu_dinv(p3d_solver* s, float* dinv) {
 
 int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   if (!s || !avg_ms || reps <= 0) return fail(P3D_EINVAL, "bad argument");
+  ensure_columns(s);
   if (which == 2 && s->ifprec != 2) return fail(P3D_ESTATE, "no ILU preconditioner");
   if ((which == 7 || which == 11) && s->ifprec != 2)
     return fail(P3D_ESTATE, "no ILU preconditioner");
   if ((which == 8 || which == 9 || which == 10 || which == 11) && !s->tm.on)
     return fail(P3D_ESTATE, "no tile-major placement (single-wave ILU tile sweeps)");
-  if (which == 11 && !(s->sweep_mode == 0 && s->sweep_ready && dilu_tiles_fuse_rupd(s->sweep)))
+  if (which == 11 && !fuse_rupd_available(s))
     return fail(P3D_ESTATE, "no register-tile ILU sweeps (P3D_OPT_TILE_STAGE 2)");
   if (which == 1 || which == 3 || which >= 7) {
     int rc = ensure_mixed(s);
@@ -1447,7 +1544,12 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
                            EPI_NONE, nullptr, false, s->stream);
         break;
       case 11:  // FP32 ILU apply with the residual update in its forward sweep
-        launch_dilu_tiles_rupd(s->sweep, s->m, s->g, s->r32, s->ap32, s->z32, s->st, s->stream);
+        if (columns_on(s))
+          launch_dilu_columns<float>(s->col, s->m, s->g, s->r32, s->z32, s->st, s->ap32,
+                                     s->stream);
+        else
+          launch_dilu_tiles_rupd(s->sweep, s->m, s->g, s->r32, s->ap32, s->z32, s->st,
+                                 s->stream);
         break;
       default:
         break;
