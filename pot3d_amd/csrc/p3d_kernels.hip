@@ -48,6 +48,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// v of lane l (wave-uniform l).
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)u, l);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // Block reduction of NV doubles, in two levels so that no single counter
 // takes an atomic from every workgroup (thousands of same-address atomics
 // serialise at the L2 and cost hundreds of microseconds per reduction).
@@ -57,7 +65,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 // slot's global counter; the last group sums the group partials in order,
 // runs the epilogue and re-arms the counters.  The result is deterministic
 // for a given launch shape.
-//   counter: the slot's kRedCounters counters ([0] global, [1 + group]);
+//   counter: the slot's kRedCounters counters, kRedStride words apart ([0]
+//   global, [1 + group]);
 //   partial: NV*G block partials, then NV*ngroups group partials.
 // Counts a block in at a reduction counter after its partial sums (agent-
 // scope atomic stores, coherent by themselves) have completed.  A release
@@ -69,6 +78,23 @@ __device__ __forceinline__ unsigned arrive(unsigned* counter) {
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A plain count-in of G blocks, one thread of each: true for the last one,
+// which re-arms the counters.
+__device__ __forceinline__ bool count_in(unsigned* counter, int G) {
+  const int grp = (int)blockIdx.x / kRedGroup;
+  const int gn = min(kRedGroup, G - grp * kRedGroup), ngrp = (G + kRedGroup - 1) / kRedGroup;
+  unsigned* gc = counter + (1 + grp) * kRedStride;
+  if (__hip_atomic_fetch_add(gc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+      (unsigned)gn - 1)
+    return false;
+  __hip_atomic_store(gc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+      (unsigned)ngrp - 1)
+    return false;
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
 }
 
 template <int BS, int NV>
@@ -93,12 +119,14 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
       for (int ww = 0; ww < BS / 64; ww++) s += sh[q][ww];
       __hip_atomic_store(&partial[q * G + Lb], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const unsigned prev = arrive(counter + 1 + grp);
+    const unsigned prev = arrive(counter + (1 + grp) * kRedStride);
     amlast = (prev == (unsigned)gn - 1);
   }
   __syncthreads();
   if (!amlast) return;
-  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  // the partials are read by agent-scope loads after the count-in returned:
+  // nothing stale can be seen, so no fence (which would drop the L2's lines)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
   // last block of the group: the group partial
 #pragma unroll
   for (int q = 0; q < NV; q++) {
@@ -110,29 +138,40 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
     if (lane == 0) sh[q][w] = s;
   }
   __syncthreads();
+  CgState c;  // for the epilogue, loaded while the count-in is under way
   if (threadIdx.x == 0) {
+    if (st) c = *st;
 #pragma unroll
     for (int q = 0; q < NV; q++) {
       double s = 0.0;
       for (int ww = 0; ww < BS / 64; ww++) s += sh[q][ww];
       __hip_atomic_store(&gpart[q * ngrp + grp], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __hip_atomic_store(counter + 1 + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(counter + (1 + grp) * kRedStride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned prev = arrive(counter);
     amlast = (prev == (unsigned)ngrp - 1);
   }
   __syncthreads();
-  if (!amlast || threadIdx.x != 0) return;
-  __atomic_thread_fence(__ATOMIC_ACQUIRE);
-  // last group: the total, in group order
-  double tot[NV];
+  if (!amlast || w != 0) return;
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  // last group: the total, in group order.  One wave loads the group partials
+  // side by side and adds them in order out of its lanes; one lane loading
+  // them in turn cost about 0.7 us each, 20 us of every reduction of 2048
+  // blocks.
+  double tot[NV] = {};
+  for (int gb = 0; gb < ngrp; gb += 64) {
+    double v[NV];
 #pragma unroll
-  for (int q = 0; q < NV; q++) {
-    double s = 0.0;
-    for (int gi = 0; gi < ngrp; gi++)
-      s += __hip_atomic_load(&gpart[q * ngrp + gi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    tot[q] = s;
+    for (int q = 0; q < NV; q++)
+      v[q] = gb + lane < ngrp ? __hip_atomic_load(&gpart[q * ngrp + gb + lane], __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0.0;
+    const int n = min(64, ngrp - gb);
+    for (int l = 0; l < n; l++)
+#pragma unroll
+      for (int q = 0; q < NV; q++) tot[q] += lane_value(v[q], l);
   }
+  if (lane != 0) return;
   if (NV == 3) {
     if (out) {
       out[0] = tot[0];
@@ -140,7 +179,7 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
       out[2] = tot[NV > 2 ? 2 : 0];
     }
   } else {
-    cg_epilogue(st, epi, tot[0], NV > 1 ? tot[NV > 1 ? 1 : 0] : 0.0, out);
+    cg_epilogue(st, c, epi, tot[0], NV > 1 ? tot[NV > 1 ? 1 : 0] : 0.0, out);
   }
   __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -870,7 +909,7 @@ static void launch_stencil_lds(const Metric& m, const Grid3& g, const T* x, T* y
   const int nseg = stencil_lds_segments<T, C>(g);
   const int G = stencil_lds_blocks<T, C>(g);
   k_stencil_lds<T, C><<<G, kBlock, 0, s>>>(m, g, nseg, x, y, pole_part, st, red.partial,
-                                            red.counter + (size_t)slot * kRedCounters, epi, out,
+                                            red.counter + (size_t)slot * kRedSlotWords, epi, out,
                                             guard ? 1 : 0, want, tm);
 }
 
@@ -936,7 +975,7 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
     const int G = stencil_rows_blocks(g);
     k_stencil_rows<T><<<G, kBlock, 0, s>>>(m, g, nseg, x, y, b, mode, pole_part, st,
                                             red.partial,
-                                            red.counter + (size_t)slot * kRedCounters, epi, out,
+                                            red.counter + (size_t)slot * kRedSlotWords, epi, out,
                                             guard ? 1 : 0, want, tm);
     return;
   }
@@ -944,7 +983,7 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
   const int G0 = stencil_col_blocks(g, tm) * nseg;
   const int G = (G0 + 7) / 8 * 8;
   k_stencil_march<T><<<G, kBlock, 0, s>>>(m, g, nseg, x, y, b, mode, pole_part, st,
-                                           red.partial, red.counter + (size_t)slot * kRedCounters,
+                                           red.partial, red.counter + (size_t)slot * kRedSlotWords,
                                            epi, out, guard ? 1 : 0, want, tm);
 }
 
@@ -1044,7 +1083,7 @@ void launch_cg_update(const Metric& m, const Grid3& g, const Launch& L, int prec
     CH = L.CHcg;
   }
   k_cg_update<T><<<G, kBlock, 0, s>>>(m, g, G, CH, prec, x, r, p, ap, st, red.partial,
-                                       red.counter + (size_t)slot * kRedCounters, xs, xscale, tm);
+                                       red.counter + (size_t)slot * kRedSlotWords, xs, xscale, tm);
 }
 
 // The residual update of the FP32 recurrence with the FP64 solution, one
@@ -1143,17 +1182,10 @@ __global__ void __launch_bounds__(kBlock)
     }
   }
   if (do_x) {
-    __shared__ int amlast;
+    // only the reads of x_ncg must precede its update
     __syncthreads();
-    // only the reads of x_ncg must precede its update: a plain count-in
-    if (threadIdx.x == 0)
-      amlast = (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                (unsigned)G - 1);
-    __syncthreads();
-    if (amlast && threadIdx.x == 0) {
+    if (threadIdx.x == 0 && count_in(counter, G))
       __hip_atomic_store(&st->x_ncg, ncg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
   }
 }
 
@@ -1238,17 +1270,10 @@ __global__ void __launch_bounds__(kBlock)
     }
   }
   if (flush) {
-    __shared__ int amlast;
+    // only the reads of x_ncg must precede its update
     __syncthreads();
-    // only the reads of x_ncg must precede its update: a plain count-in
-    if (threadIdx.x == 0)
-      amlast = (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                (unsigned)G - 1);
-    __syncthreads();
-    if (amlast && threadIdx.x == 0) {
+    if (threadIdx.x == 0 && count_in(counter, G))
       __hip_atomic_store(&st->x_ncg, ncg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
   }
 }
 
@@ -1331,7 +1356,7 @@ void launch_dot2(const Grid3& g, const Launch& L, const T* x, const T* y, const 
                  bool guard, hipStream_t s, const TileMap& tm) {
   const int G = sizeof(T) == 8 && L.Gd2 > 0 ? L.Gd2 : L.G;
   k_dot2<T><<<G, kBlock, 0, s>>>(g, G, L.CH, x, y, u, v, st, red.partial,
-                                  red.counter + (size_t)slot * kRedCounters, epi, out,
+                                  red.counter + (size_t)slot * kRedSlotWords, epi, out,
                                   guard ? 1 : 0, tm);
 }
 
@@ -1362,7 +1387,7 @@ void launch_point_prec(const Metric& m, const Grid3& g, const Launch& L, int pre
                        T* z, CgState* st, Reduce red, int slot, Epi epi, double* out,
                        hipStream_t s) {
   k_point_prec<T><<<L.G, kBlock, 0, s>>>(m, g, L.G, L.CH, prec, r, z, st, red.partial,
-                                          red.counter + (size_t)slot * kRedCounters, epi, out);
+                                          red.counter + (size_t)slot * kRedSlotWords, epi, out);
 }
 
 template <typename T>

@@ -22,24 +22,30 @@ enum Epi {
 };
 
 // ---------------------------------------------------------------------------
-// CG scalar logic (cgsolve/ernorm), run by one thread after a reduction.
-__device__ inline void cg_check(CgState* st) {
-  const double epssq = st->rdotr / st->bdotb;
+// CG scalar logic (cgsolve/ernorm), run by one thread after a reduction; c is
+// the state before it, read in one go (its fields one by one, as the logic
+// comes to them, would be so many memory round trips).
+__device__ inline int cg_check(CgState* st, const CgState& c, double rdotr, double rr) {
+  const double epssq = rdotr / c.bdotb;
   const double epsn = copysign(1.0, epssq) * sqrt(fabs(epssq));
+  const double relres = sqrt(rr / c.bb);
   st->epsn = epsn;
-  st->relres = sqrt(st->rr / st->bb);
-  if (st->hist && st->ncg < st->hist_cap) st->hist[st->ncg] = epsn;
-  const double crit = st->stop_mode == 0 ? epsn : st->relres;
-  if (!isfinite(epsn) || !isfinite(st->relres)) {
-    st->done = 3;
-  } else if (crit < st->epscg) {
-    st->done = 1;
-  } else if (st->ncg >= st->ncgmax) {
-    st->done = 2;
-  }
+  st->relres = relres;
+  if (c.hist && c.ncg < c.hist_cap) c.hist[c.ncg] = epsn;
+  const double crit = c.stop_mode == 0 ? epsn : relres;
+  int done = 0;
+  if (!isfinite(epsn) || !isfinite(relres))
+    done = 3;
+  else if (crit < c.epscg)
+    done = 1;
+  else if (c.ncg >= c.ncgmax)
+    done = 2;
+  if (done) st->done = done;
+  return done;
 }
 
-__device__ inline void cg_epilogue(CgState* st, Epi epi, double s0, double s1, double* out) {
+__device__ inline void cg_epilogue(CgState* st, const CgState& c, Epi epi, double s0, double s1,
+                                   double* out) {
   switch (epi) {
     case EPI_BDOTB:
       st->bdotb = s0;
@@ -49,30 +55,29 @@ __device__ inline void cg_epilogue(CgState* st, Epi epi, double s0, double s1, d
     case EPI_RINIT:
       st->rdotr = s0;
       st->rr = s1;
-      cg_check(st);
+      cg_check(st, c, s0, s1);
       break;
     case EPI_PAP:
-      st->ncg += 1;
+      st->ncg = c.ncg + 1;
       st->pdotap = s0;
-      st->alpha = st->rdotr / s0;
+      st->alpha = c.rdotr / s0;
       break;
     case EPI_RR:
       st->rr = s1;
       break;
     case EPI_RITER:
     case EPI_RZITER:
-      st->rdotr_old = st->rdotr;
+      st->rdotr_old = c.rdotr;
       st->rdotr = s0;
       if (epi == EPI_RITER) st->rr = s1;
-      cg_check(st);
-      if (!st->done) st->beta = st->rdotr / st->rdotr_old;
+      if (!cg_check(st, c, s0, epi == EPI_RITER ? s1 : c.rr)) st->beta = s0 / c.rdotr;
       break;
     case EPI_REPLACE:
       // the recurrence stopped with rdotr_old = r.z of its last direction;
       // the replaced residual continues the same Krylov recurrence
       st->rdotr = s0;
       st->rr = s1;
-      st->beta = s0 / st->rdotr_old;
+      st->beta = s0 / c.rdotr_old;
       break;
     case EPI_STORE:
       if (out) {
@@ -108,6 +113,11 @@ constexpr int kBlock = 256;
 // ([0] global + one per group), so at most kRedGroup*(kRedCounters-1) blocks
 constexpr int kRedGroup = 128;
 constexpr int kRedCounters = 256;
+// words from one counter to the next: counters that share a 256-byte piece of
+// memory take their atomics one after the other (10 ns each, 20 us for the
+// 2048 blocks of a reduction whose counters were neighbours)
+constexpr int kRedStride = 64;
+constexpr int kRedSlotWords = kRedCounters * kRedStride;  // of one reduction site
 constexpr int kRedSlots = 16;
 constexpr int kUnroll = 4;  // points per thread in flight in the streaming kernels
 constexpr int kPoleSegs = 16;

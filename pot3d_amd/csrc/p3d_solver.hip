@@ -322,7 +322,7 @@ static void cg_iteration(p3d_solver* s, Vecs<T> v, int t) {
       if (!fused) launch_r_update(s->gt.N, s->Lt, v.r, v.ap, s->st, s->stream);
       prec_and_dot<float>(s, v.r, v.z, EPI_RITER, nullptr, true, fused ? v.ap : nullptr);
       launch_p_update_x(s->g, s->L, t, v.pb, v.z, s->st, s->stream, s->tm, v.xs, v.xscale,
-                        s->red.counter + 5 * kRedCounters);
+                        s->red.counter + 5 * kRedSlotWords);
       return;
     }
   }
@@ -985,9 +985,9 @@ int p3d_create(p3d_solver** out, int nr, int nt, int np, const double* r, const 
   if ((rc = dalloc((void**)&s->red.partial,
                    sizeof(double) * 3 * (s->red.max_blocks + kRedCounters))))
     return bail(rc);
-  if ((rc = dalloc((void**)&s->red.counter, sizeof(unsigned) * kRedSlots * kRedCounters)))
+  if ((rc = dalloc((void**)&s->red.counter, sizeof(unsigned) * kRedSlots * kRedSlotWords)))
     return bail(rc);
-  hipMemset(s->red.counter, 0, sizeof(unsigned) * kRedSlots * kRedCounters);
+  hipMemset(s->red.counter, 0, sizeof(unsigned) * kRedSlots * kRedSlotWords);
   hipMemset(s->x, 0, nb);
   hipMemset(s->b, 0, nb);
   hipMemset(s->pole_part, 0, sizeof(double) * 2 * kPoleSegs * a);
@@ -1349,7 +1349,7 @@ int p3d_energy(p3d_solver* s, const double* phi, double* w, double* br, double* 
     if ((rc = dalloc((void**)&s->e_partial, sizeof(double) * 3 * (s->eG + kRedCounters))))
       return rc;
   }
-  launch_energy(s->em, nr, nt, np, s->phi, s->e_partial, s->red.counter + 8 * kRedCounters,
+  launch_energy(s->em, nr, nt, np, s->phi, s->e_partial, s->red.counter + 8 * kRedSlotWords,
                 s->out, s->eG,
                 s->stream);
   HIPCHK(hipGetLastError());
@@ -1533,7 +1533,7 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
         (void)hipMemsetAsync(&s->st->x_ncg, 0, sizeof(int), s->stream);  // checked below
         for (int t = 0; t < kXBatch; t++)
           launch_p_update_x(s->g, s->L, t, pb, s->z32, s->st, s->stream, s->tm, s->x,
-                            s->out + 4, s->red.counter + 5 * kRedCounters);
+                            s->out + 4, s->red.counter + 5 * kRedSlotWords);
         break;
       }
       case 9:  // residual update of the FP32 recurrence (tile-major r, ap)
