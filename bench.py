@@ -116,13 +116,18 @@ def cpu_baseline(workload, family: str, cores: int, sample_iters: int, n_iter_es
 
 # (name, time_kernel id, algorithmic bytes per unknown, padded-array bytes per point)
 KERNELS = [
-    ("pcg_iteration_fp64 (graph replay)", 3, 136, 8),
+    # operator 8 + 8 (padded), forward sweep with r -= alpha Ap 32, backward
+    # sweep 16, r.z with r.r 16, p update with x 34
+    ("pcg_iteration_fp64 (graph replay)", 3, 106, 8),
     ("stencil_fp64 (k_stencil_lds<double>)", 0, 8, 8),
     ("stencil_fp32 (k_stencil_lds<float>)", 1, 4, 4),
     ("ilu_apply_fp64 (k_tile_fwd+k_tile_bwd<double>)", 2, 32, 0),
     ("ilu_apply_fp32 (k_tile_fwd+k_tile_bwd<float>)", 7, 24, 0),
-    ("cg_update_fp64 (k_cg_update<double>)", 4, 48, 0),
-    ("p_update_fp64 (k_p_update<double>)", 5, 24, 0),
+    # r, ap read, r written (runs where the sweeps do not take it)
+    ("cg_update_fp64 (k_cg_update<double>)", 4, 24, 0),
+    # p, z read, p written, and the solution once per 4 iterations:
+    # (4*24 + 16 + 24) / 4
+    ("p_update_fp64 (k_p_update_x<double>, x every 4 iterations)", 5, 34, 0),
     ("copy_fp64 (k_copy<double>)", 6, 16, 0),
 ]
 

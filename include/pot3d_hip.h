@@ -98,7 +98,8 @@ enum {
                              its residual is replaced by the FP64 b-Ax
                              whenever it has fallen 1000-fold */
   P3D_OPT_INNER_TOL = 3,  /* inner relative tolerance (default 1e-5) */
-  P3D_OPT_CHUNK = 4,      /* CG iterations per captured graph (default auto) */
+  P3D_OPT_CHUNK = 4,      /* CG iterations per captured graph, rounded up to
+                             groups of 4 (default auto) */
   P3D_OPT_GRAPH = 5,      /* 1: replay iterations as a hipGraph (default) */
   P3D_OPT_SWEEP = 6,      /* ILU triangular-solve schedule: 0 tile diagonals
                              (8x8x32 tiles, one launch per anti-diagonal;
@@ -134,8 +135,10 @@ enum {
                                 i from the adjacent lanes; 2 64 x 4WJ (r,
                                 theta) patches staged plane by plane in LDS,
                                 WJ = 8 when that still makes 2048 or more
-                                workgroups, else 4; 3 and 4 the same with
-                                WJ = 8 and WJ = 4; -1 (default) 2.  The LDS
+                                workgroups (FP32: and from 2^25 unknowns),
+                                else 4; 3 and 4 the same with WJ = 8 and
+                                WJ = 4; -1 (default) 2, below 2^22 unknowns
+                                0.  The LDS
                                 kernels apply A x; b - A x and outputs of
                                 2^32 bytes or more take 1 (FP32 operator
                                 whose 62-lane waves cover the r extent to
@@ -273,8 +276,9 @@ int p3d_history(p3d_solver* s, double* hist, int n);
 /* Kernel timing with HIP events on the solver's stream: `which` =
  * 0 FP64 operator, 1 FP32 operator (output placed as in the FP32
  * recurrence), 2 ILU apply (FP64 in/out), 3 one FP64 PCG iteration
- * (replayed through the solve's captured graph), 4 FP64 CG vector update,
- * 5 FP64 p update, 6 plain copy of N doubles (bandwidth reference), 7 ILU
+ * (replayed through the solve's captured graph), 4 FP64 CG residual update
+ * with its dot products, 5 FP64 p update with the solution update (per
+ * iteration of a group of 4), 6 plain copy of N doubles (bandwidth reference), 7 ILU
  * apply in FP32; with the single-wave ILU tile sweeps (tile-major vectors,
  * else P3D_ESTATE) the FP32 recurrence's 8 p update with the FP64 solution
  * update, 9 residual update, 10 r.z with r.r, and with the register tiles

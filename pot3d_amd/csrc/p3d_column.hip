@@ -98,6 +98,13 @@ __device__ __forceinline__ uint32_t tm_row(const ColArgs& ca, int col, int k) {
   return ((tile << ca.tk_log2) + (uint32_t)(k & ((1 << ca.tk_log2) - 1))) * 64u;
 }
 
+__device__ __forceinline__ float neg_fma(float a, float b, float c) {
+  return __builtin_fmaf(-a, b, c);
+}
+__device__ __forceinline__ double neg_fma(double a, double b, double c) {
+  return __builtin_fma(-a, b, c);
+}
+
 template <int P>
 using Phase = std::integral_constant<int, P>;
 
@@ -309,12 +316,12 @@ __device__ __forceinline__ void col_lds_init(const ColArgs& ca, ColLds& sh, floa
 }
 
 // ---------------------------------------------------------------------------
-// Forward sweep, y = L^-1 r.  With kUpd (FP32 recurrence) r -= alpha ap
-// first, r written back (the same fmaf as k_r_update).
+// Forward sweep, y = L^-1 r.  With kUpd r -= alpha ap first, r written back
+// (the same fused multiply-add as k_r_update and k_cg_update).
 template <typename T, bool kUpd, int kMode>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
     k_col_fwd(Metric m, Grid3 g, ColArgs ca, T* __restrict__ r, const CgState* guard,
-              const float* __restrict__ ap) {
+              const T* __restrict__ ap) {
   extern __shared__ char lds[];
   ColLds& sh = *(ColLds*)lds;
   float2* pf = (float2*)(lds + sizeof(ColLds));
@@ -323,36 +330,46 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
   if (x.wave == 1) {
     const int kmax = ca.planes;  // planes of the tile-major vectors
     const int last = ca.rounds * kCP - 1;
-    T rv[kCP][kCU];
-    float av[kUpd ? kCP : 1][kUpd ? kCU : 1], dv[kCP][kCU];
+    // ap in FP64 comes two chunks ahead only: registers for three waves per SIMD
+    constexpr int kAP = !kUpd ? 1 : (sizeof(T) == 8 ? 2 : kCP);
+    T rv[kCP][kCU], av[kAP][kCU];
+    float dv[kCP][kCU];
+    // past the vector's planes: its last ones (pivot 0 there, not used)
+    auto row = [&](int n) { return tm_row(ca, x.col, min(n * kCU, kmax - kCU)); };
     auto load = [&](int p, int n) {
-      // past the vector's planes: its last ones (pivot 0 there, not used)
-      const uint32_t o = tm_row(ca, x.col, min(n * kCU, kmax - kCU));
-      const T* rb = r + o;
+      const T* rb = r + row(n);
       const float* d = ca.dinv_s + x.sk + (size_t)min(n, last) * (kCU * 64);
 #pragma unroll
       for (int u = 0; u < kCU; u++) {
         rv[p][u] = rb[u * 64 + lane];
-        if constexpr (kUpd) av[p][u] = (ap + o)[u * 64 + lane];
         dv[p][u] = d[u * 64 + lane];
       }
     };
+    auto load_a = [&](int p, int n) {
+      const T* ab = ap + row(n);
+#pragma unroll
+      for (int u = 0; u < kCU; u++) av[p][u] = ab[u * 64 + lane];
+    };
 #pragma unroll
     for (int p = 0; p < kCP; p++) load(p, p);
-    const float alpha = kUpd ? (float)st_load(&guard->alpha) : 0.f;
+    if constexpr (kUpd) {
+#pragma unroll
+      for (int p = 0; p < kAP; p++) load_a(p, p);
+    }
+    const T alpha = kUpd ? (T)st_load(&guard->alpha) : (T)0;
     col_lds_init(ca, sh, pf, ca.pf_lo, lane);
     if (guard && st_done(guard)) return;
     // chunk n's inputs to LDS (n = phase p mod kCP): row q of r to step q + dl
     auto put = [&](auto pc, int n) {
       constexpr int p = decltype(pc)::value;
-      float v[kCU];
+      T v[kCU];
       float2* d = &sh.v[(n & 7) * kCU][lane];
       const int o = (n & 7) * kCU + x.dl;
 #pragma unroll
       for (int u = 0; u < kCU; u++) {
-        v[u] = (float)rv[p][u];
-        if constexpr (kUpd) v[u] = __builtin_fmaf(-alpha, av[p][u], v[u]);
-        sh.v[(o + u) & (kRing - 1)][lane].x = v[u];
+        v[u] = rv[p][u];
+        if constexpr (kUpd) v[u] = neg_fma(alpha, av[p % kAP][u], v[u]);
+        sh.v[(o + u) & (kRing - 1)][lane].x = (float)v[u];
         d[u * 64].y = dv[p][u];
       }
       if constexpr (kUpd) {
@@ -360,6 +377,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
         T* ro = (in ? r : (T*)ca.dummy) + (in ? tm_row(ca, x.col, n * kCU) : 0u);
 #pragma unroll
         for (int u = 0; u < kCU; u++) ro[u * 64 + lane] = v[u];
+        load_a(p % kAP, n + kAP);
       }
       load(p, n + kCP);
     };
@@ -525,17 +543,13 @@ size_t col_lds(const ColArgs& ca) {
 
 template <typename T, int kMode>
 void launch_columns(const ColArgs& ca, const Metric& m, const Grid3& g, T* r, T* z,
-                    const CgState* guard, const float* ap, hipStream_t s) {
+                    const CgState* guard, const T* ap, hipStream_t s) {
   const size_t lds = col_lds(ca);
   const int nb = ca.NI * ca.NJ;
-  if constexpr (sizeof(T) == 4) {
-    if (ap)
-      k_col_fwd<T, true, kMode><<<nb, kThreads, lds, s>>>(m, g, ca, r, guard, ap);
-    else
-      k_col_fwd<T, false, kMode><<<nb, kThreads, lds, s>>>(m, g, ca, r, guard, nullptr);
-  } else {
+  if (ap)
+    k_col_fwd<T, true, kMode><<<nb, kThreads, lds, s>>>(m, g, ca, r, guard, ap);
+  else
     k_col_fwd<T, false, kMode><<<nb, kThreads, lds, s>>>(m, g, ca, r, guard, nullptr);
-  }
   k_col_bwd<T, kMode><<<nb, kThreads, lds, s>>>(m, g, ca, z, guard);
 }
 
@@ -640,7 +654,7 @@ void free_column_plan(ColumnPlan& plan) {
 
 template <typename T>
 void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g, T* r, T* z,
-                         const CgState* guard, const float* ap, hipStream_t s) {
+                         const CgState* guard, const T* ap, hipStream_t s) {
   const ColArgs& ca = plan.a;
   if (ca.mode == kPhiUniform)
     launch_columns<T, kPhiUniform>(ca, m, g, r, z, guard, ap, s);
@@ -653,7 +667,7 @@ void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g
 const unsigned* column_failure_flag(const ColumnPlan& plan) { return plan.ctr + 2; }
 
 template void launch_dilu_columns<double>(const ColumnPlan&, const Metric&, const Grid3&, double*,
-                                          double*, const CgState*, const float*, hipStream_t);
+                                          double*, const CgState*, const double*, hipStream_t);
 template void launch_dilu_columns<float>(const ColumnPlan&, const Metric&, const Grid3&, float*,
                                          float*, const CgState*, const float*, hipStream_t);
 

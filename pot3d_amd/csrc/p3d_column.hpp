@@ -48,11 +48,11 @@ int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const I
                       int tk_log2, const float* dinv);
 void free_column_plan(ColumnPlan& plan);
 
-// z = (LU)^-1 r on tile-major r and z, two launches.  ap (FP32, with guard):
-// r -= alpha ap first, alpha from guard.
+// z = (LU)^-1 r on tile-major r and z, two launches.  ap (tile-major, with
+// guard): r -= alpha ap first, alpha from guard.
 template <typename T>
 void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g, T* r, T* z,
-                         const CgState* guard, const float* ap, hipStream_t s);
+                         const CgState* guard, const T* ap, hipStream_t s);
 
 // Device word that is not 0 once a wait of a column sweep ran into its bound.
 const unsigned* column_failure_flag(const ColumnPlan& plan);

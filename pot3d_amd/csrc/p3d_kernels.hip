@@ -331,6 +331,14 @@ __host__ __device__ inline int stencil_col_blocks(const Grid3& g, const TileMap&
   return (int)((g.ab + kBlock - 1) / kBlock);
 }
 
+// The tile map that shapes the march: the FP64 sums keep the natural column
+// order whatever the placement of the output, so that an FP64 solve does not
+// depend on the ILU schedule.
+template <typename T>
+__host__ __device__ inline TileMap march_shape(const TileMap& tm) {
+  return sizeof(T) == 4 ? tm : TileMap{};
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     k_stencil_march(Metric m, Grid3 g, int nseg, const T* __restrict__ x, T* __restrict__ y,
@@ -340,16 +348,16 @@ __global__ void __launch_bounds__(kBlock)
   if (guard && st_done(st)) return;
   const int G = gridDim.x;
   const int Lb = logical_block(G);
-  const int ncol_blocks = stencil_col_blocks(g, tm);
+  const int ncol_blocks = stencil_col_blocks(g, march_shape<T>(tm));
   const int cb = Lb % ncol_blocks, seg = Lb / ncol_blocks;
   const int kper = (g.c + nseg - 1) / nseg;
   const int k0 = seg * kper, k1 = min(g.c, k0 + kper);
-  // the columns of a wave: 64 consecutive mcol = i + a j, or, with the
+  // the columns of a wave: 64 consecutive mcol = i + a j, or, with the FP32
   // tile-major output, one 8x8 (i, j) patch, so that a wave writes whole
   // 256-byte tile planes
   int i, j;
   bool col_ok;
-  if (tm.on) {
+  if (march_shape<T>(tm).on) {
     const int t = cb * (kBlock / 64) + (int)(threadIdx.x >> 6);
     const int lane = (int)(threadIdx.x & 63);
     i = (t % tm.TNI) * 8 + (lane & 7);
@@ -895,10 +903,13 @@ static int stencil_lds_blocks_max(const Grid3& g) {
                    stencil_lds_blocks<float, LdsCfg<float, false>>(g)});
 }
 
-// The tall patches when they still make about 8 workgroups per CU.
+// The tall patches when they still make about 8 workgroups per CU; in FP32
+// from 2^25 points (short and tall: 60 and 67 us at 26.8 M points, 192 and 188
+// at 67.2 M, 520 and 470 at 214.7 M).
 template <typename T>
 static bool stencil_lds_tall(const Grid3& g) {
-  return stencil_lds_blocks<T, LdsCfg<T, true>>(g) >= 8 * 256;
+  return stencil_lds_blocks<T, LdsCfg<T, true>>(g) >= 8 * 256 &&
+         (sizeof(T) == 8 || g.N >= (1u << 25));
 }
 
 template <typename T, typename C>
@@ -959,7 +970,11 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
                   (double)(((g.c + (1 << tm.tk_log2) - 1) >> tm.tk_log2) << tm.tk_log2)
             : (double)g.N;
   const bool lds_ok = mode == 0 && nout * sizeof(T) < (double)kDropStore;
-  if (lds_ok && (L.stencil < 0 || L.stencil >= 2)) {
+  // below 2^22 points the launch is all latency, and the column march has the
+  // shortest chain (LDS patches and march, FP64: 14.2 and 8.3 us at 0.8 M
+  // points, 21 and 18 at 3.4 M, 28 and 27 at 6.4 M, 36 and 51 at 13.6 M)
+  const bool small = L.stencil < 0 && g.N < (1u << 22);
+  if (lds_ok && !small && (L.stencil < 0 || L.stencil >= 2)) {
     const bool tall = L.stencil == 3 || ((L.stencil < 0 || L.stencil == 2) &&
                                          stencil_lds_tall<T>(g));
     if (tall)
@@ -970,7 +985,7 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
                                               guard, want, s, tm);
     return;
   }
-  if (L.stencil == 1 || (L.stencil < 0 && stencil_rows_chosen(g, sizeof(T)))) {
+  if (L.stencil == 1 || (L.stencil < 0 && !small && stencil_rows_chosen(g, sizeof(T)))) {
     const int nseg = stencil_rows_segments(g);
     const int G = stencil_rows_blocks(g);
     k_stencil_rows<T><<<G, kBlock, 0, s>>>(m, g, nseg, x, y, b, mode, pole_part, st,
@@ -979,8 +994,8 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
                                             guard ? 1 : 0, want, tm);
     return;
   }
-  const int nseg = stencil_segments(g, tm);
-  const int G0 = stencil_col_blocks(g, tm) * nseg;
+  const int nseg = stencil_segments(g, march_shape<T>(tm));
+  const int G0 = stencil_col_blocks(g, march_shape<T>(tm)) * nseg;
   const int G = (G0 + 7) / 8 * 8;
   k_stencil_march<T><<<G, kBlock, 0, s>>>(m, g, nseg, x, y, b, mode, pole_part, st,
                                            red.partial, red.counter + (size_t)slot * kRedSlotWords,
@@ -994,27 +1009,33 @@ __device__ __forceinline__ float diag_inv(const Metric& m, int i, int j, int k) 
   return (float)(1.0 / cf.a4);
 }
 
-template <typename T>
-__device__ __forceinline__ T apply_point_prec(const Metric& m, const Grid3& g, int prec,
-                                              uint32_t n, T r) {
-  if (prec == PREC_DIAG) {
-    int i, j, k;
-    unflatten(g, n, i, j, k);
-    const float ai = diag_inv(m, i, j, k);
-    return (T)((T)ai * r);
-  }
-  return r;
+// The diagonal preconditioner's factors: FP32 as in the reference, formed once
+// (10 table loads and an FP64 division per point, which the CG update and the
+// p update had to do in every iteration: at 55x181x361 the two took 38 + 32 us
+// and, with the grouped solution update below, take 20 + 21).
+__global__ void k_diag_inv(Metric m, Grid3 g, float* __restrict__ d) {
+  const uint32_t n = blockIdx.x * kBlock + threadIdx.x;
+  if (n >= g.N) return;
+  int i, j, k;
+  unflatten(g, n, i, j, k);
+  d[n] = diag_inv(m, i, j, k);
 }
 
-// x += alpha p ; r -= alpha ap ; (DIAG/NONE) z = M^-1 r with s0=r.z, s1=r.r
-// (cgsolve :4340-4351).  For ILU only s1=r.r is reduced here.  With xs != nullptr (FP32 recurrence, FP64 solution) the
+void launch_diag_inv(const Metric& m, const Grid3& g, float* d, hipStream_t s) {
+  k_diag_inv<<<(g.N + kBlock - 1) / kBlock, kBlock, 0, s>>>(m, g, d);
+}
+
+// r -= alpha ap ; (DIAG/NONE) z = M^-1 r with s0=r.z, s1=r.r (cgsolve
+// :4340-4351).  For ILU only s1=r.r is reduced here.  kX: also x += alpha p;
+// else the solution is updated once per group of iterations with the p update
+// (k_p_update_x).  With xs != nullptr (kX; FP32 recurrence, FP64 solution) the
 // update goes to the double vector xs instead of x: xs += (alpha scale) p,
 // scale = *xscale being the factor of the scaled FP32 system.  Accumulating
 // the solution in FP32 would leave its true residual at about
 // eps32*cond(A) of the start, whatever the recurrence says.
-template <typename T>
+template <typename T, bool kX>
 __global__ void __launch_bounds__(kBlock)
-    k_cg_update(Metric m, Grid3 g, int G, int CH, int prec, T* __restrict__ x,
+    k_cg_update(Grid3 g, int G, int CH, int prec, const float* __restrict__ dg, T* __restrict__ x,
                 T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ ap, CgState* st,
                 double* partial, unsigned* counter, double* __restrict__ xs,
                 const double* __restrict__ xscale, TileMap tm) {
@@ -1024,44 +1045,54 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t n1 = min(g.N, n0 + (uint32_t)CH);
   const double alpha_d = st_load(&st->alpha);
   const T alpha = (T)alpha_d;
-  const double alpha_x = xs ? alpha_d * *xscale : 0.0;
+  const double alpha_x = kX && xs ? alpha_d * *xscale : 0.0;
+  const bool diag = prec == PREC_DIAG;
   double s0 = 0.0, s1 = 0.0;
-  // blocks of kUnroll points per thread, all loads issued first; the sums
-  // keep the point order of the plain loop (one chunk per workgroup:
-  // measured 5% faster here than the grid-stride of the FP32 streams)
-  for (uint32_t nb = n0 + threadIdx.x; nb < n1; nb += kUnroll * kBlock) {
-    T xv[kUnroll], pv[kUnroll], rv[kUnroll], av[kUnroll];
-    double xd[kUnroll];
-    uint32_t tr[kUnroll];  // position of point n in r
+  // blocks of kU points per thread, all loads issued first; the sums keep the
+  // point order of the plain loop (one chunk per workgroup: measured 5%
+  // faster here than the grid-stride of the FP32 streams)
+  constexpr int kU = kX ? kUnroll : 2 * kUnroll;
+  for (uint32_t nb = n0 + threadIdx.x; nb < n1; nb += kU * kBlock) {
+    T xv[kU], pv[kU], rv[kU], av[kU];
+    double xd[kU];
+    float dv[kU];
+    uint32_t tr[kU];  // position of point n in r
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
+    for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
       xv[u] = pv[u] = rv[u] = av[u] = (T)0;
       xd[u] = 0.0;
+      dv[u] = 0.f;
       tr[u] = 0;
       if (n < n1) {
         tr[u] = tmap(tm, g, n);
-        if (xs)
-          xd[u] = xs[n];
-        else
-          xv[u] = x[n];
-        pv[u] = p[n];
+        if constexpr (kX) {
+          if (xs)
+            xd[u] = xs[n];
+          else
+            xv[u] = x[n];
+          pv[u] = p[n];
+        }
         rv[u] = r[tr[u]];
         av[u] = ap[n];
+        if (diag) dv[u] = dg[n];
       }
     }
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
+    for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
       if (n < n1) {
-        if (xs)
-          xs[n] = xd[u] + alpha_x * (double)pv[u];
-        else
-          x[n] = xv[u] + alpha * pv[u];
-        const T rn = rv[u] - alpha * av[u];
+        if constexpr (kX) {
+          if (xs)
+            xs[n] = xd[u] + alpha_x * (double)pv[u];
+          else
+            x[n] = xv[u] + alpha * pv[u];
+        }
+        const T rn = sizeof(T) == 8 ? (T)__builtin_fma(-(double)alpha, (double)av[u], (double)rv[u])
+                                    : (T)__builtin_fmaf(-(float)alpha, (float)av[u], (float)rv[u]);
         r[tr[u]] = rn;
         if (prec != PREC_ILU) {
-          const T z = apply_point_prec<T>(m, g, prec, n, rn);
+          const T z = diag ? (T)dv[u] * rn : rn;
           s0 += (double)rn * (double)z;
         }
         s1 += (double)rn * (double)rn;
@@ -1074,7 +1105,7 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 template <typename T>
-void launch_cg_update(const Metric& m, const Grid3& g, const Launch& L, int prec, T* x, T* r,
+void launch_cg_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* x, T* r,
                       const T* p, const T* ap, CgState* st, Reduce red, int slot,
                       hipStream_t s, double* xs, const double* xscale, const TileMap& tm) {
   int G = L.G, CH = L.CH;
@@ -1082,8 +1113,13 @@ void launch_cg_update(const Metric& m, const Grid3& g, const Launch& L, int prec
     G = L.Gcg;
     CH = L.CHcg;
   }
-  k_cg_update<T><<<G, kBlock, 0, s>>>(m, g, G, CH, prec, x, r, p, ap, st, red.partial,
-                                       red.counter + (size_t)slot * kRedSlotWords, xs, xscale, tm);
+  unsigned* c = red.counter + (size_t)slot * kRedSlotWords;
+  if (x || xs)
+    k_cg_update<T, true><<<G, kBlock, 0, s>>>(g, G, CH, prec, dg, x, r, p, ap, st, red.partial, c,
+                                              xs, xscale, tm);
+  else
+    k_cg_update<T, false><<<G, kBlock, 0, s>>>(g, G, CH, prec, dg, x, r, p, ap, st, red.partial,
+                                               c, xs, xscale, tm);
 }
 
 // The residual update of the FP32 recurrence with the FP64 solution, one
@@ -1130,7 +1166,7 @@ void launch_r_update(uint32_t n_all, const Launch& Lt, float* r, const float* ap
 // p = beta p + z  (:4361-4363)
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    k_p_update(Metric m, Grid3 g, int G, int CH, int prec, T* __restrict__ p,
+    k_p_update(Grid3 g, int G, int prec, const float* __restrict__ dg, T* __restrict__ p,
                const T* __restrict__ r, const T* __restrict__ z, CgState* st, TileMap tm,
                double* __restrict__ xs, const double* __restrict__ xscale,
                unsigned* counter) {
@@ -1143,8 +1179,8 @@ __global__ void __launch_bounds__(kBlock)
   const int ncg = xs ? st_load_int(&st->ncg) : 0;
   const bool do_x = xs && st_load_int(&st->x_ncg) < ncg;
   if (done && !do_x) return;
-  const int Lb = logical_block(G);
   const uint32_t n1 = g.N;
+  const bool diag = prec == PREC_DIAG;
   const T beta = (T)st_load(&st->beta);
   const double alpha_x = do_x ? st_load(&st->alpha) * *xscale : 0.0;
   // 16 points per thread in flight, and the p and solution streams read
@@ -1158,12 +1194,15 @@ __global__ void __launch_bounds__(kBlock)
        nb += (uint32_t)G * (kU * kBlock)) {
     T pv[kU], zv[kU];
     double xv[kU];
+    float dv[kU];
 #pragma unroll
     for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
       pv[u] = zv[u] = (T)0;
       xv[u] = 0.0;
+      dv[u] = 0.f;
       if (n < n1) {
+        if (diag) dv[u] = dg[n];
         pv[u] = __builtin_nontemporal_load(p + n);
         if (do_x) xv[u] = __builtin_nontemporal_load(xs + n);
         if (!done) zv[u] = (prec == PREC_ILU) ? z[tmap(tm, g, n)] : r[n];
@@ -1175,7 +1214,7 @@ __global__ void __launch_bounds__(kBlock)
       if (n < n1) {
         if (do_x) __builtin_nontemporal_store(xv[u] + alpha_x * (double)pv[u], xs + n);
         if (!done) {
-          const T zn = (prec == PREC_ILU) ? zv[u] : apply_point_prec<T>(m, g, prec, n, zv[u]);
+          const T zn = diag ? (T)dv[u] * zv[u] : zv[u];
           p[n] = beta * pv[u] + zn;
         }
       }
@@ -1189,21 +1228,24 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// The p update of the FP32 recurrence with the FP64 solution, the
-// solution updated once per group of kXBatch iterations: iteration t of a
-// group reads its direction p_t from pb.p[t] and writes p_(t+1) = z + beta
-// p_t to pb.p[(t+1) % kXBatch]; at the group's last iteration, or when the
-// recurrence has stopped, the solution takes the group's pending updates
-// x += (alpha_u scale) p_u in iteration order -- the arithmetic, in the
-// order, of one update per iteration (explicit fused multiply-adds), with
-// the solution read and written once instead of kXBatch times.  The
-// directions of earlier iterations are still in their buffers: p_(t+1)
-// overwrites p_(t+1-kXBatch), read first for the flush.
-template <int T_>
+// The p update with the solution updated once per group of kXBatch
+// iterations: iteration t of a group reads its direction p_t from pb.p[t] and
+// writes p_(t+1) = z + beta p_t to pb.p[(t+1) % kXBatch]; at the group's last
+// iteration, or when the recurrence has stopped, the solution takes the
+// group's pending updates x += (alpha_u scale) p_u in iteration order -- the
+// arithmetic, in the order, of one update per iteration (explicit fused
+// multiply-adds), with the solution read and written once instead of kXBatch
+// times: 10 bytes per unknown and iteration in FP64 where the CG update took
+// 24.  The directions of earlier iterations are still in their buffers:
+// p_(t+1) overwrites p_(t+1-kXBatch), read first for the flush.
+// T float: the FP32 recurrence with the FP64 solution (scale *xscale); double:
+// the FP64 one (xscale null: 1).  z: ILU, M^-1 r placed by tm; DIAG (dg) and
+// NONE, r itself.
+template <typename T, int T_, int kPrec>
 __global__ void __launch_bounds__(kBlock)
-    k_p_update_x(Grid3 g, int G, int CH, PBuf pb, const float* __restrict__ z, CgState* st,
-                 TileMap tm, double* __restrict__ xs, const double* __restrict__ xscale,
-                 unsigned* counter) {
+    k_p_update_x(Grid3 g, int G, PBuf<T> pb, const T* __restrict__ z,
+                 const float* __restrict__ dg, CgState* st, TileMap tm, double* __restrict__ xs,
+                 const double* __restrict__ xscale, unsigned* counter) {
   const int done = st_done(st);
   const int ncg = st_load_int(&st->ncg);
   const int pending = ncg - st_load_int(&st->x_ncg);  // iterations not in x yet
@@ -1217,8 +1259,8 @@ __global__ void __launch_bounds__(kBlock)
   }
   if (done && !flush) return;
   const uint32_t n1 = g.N;
-  const float beta = (float)st_load(&st->beta);
-  const double sc = *xscale;
+  const T beta = (T)st_load(&st->beta);
+  const double sc = xscale ? *xscale : 1.0;
   double ax[kXBatch];
   bool use[kXBatch];
 #pragma unroll
@@ -1226,22 +1268,25 @@ __global__ void __launch_bounds__(kBlock)
     use[u] = flush && u <= T_ && u >= T_ + 1 - pending;
     ax[u] = u == T_ ? st_load(&st->alpha) * sc : (use[u] ? st_load(&st->alpha_hist[u]) * sc : 0.0);
   }
-  const float* __restrict__ pin = pb.p[T_];
-  float* __restrict__ pout = pb.p[(T_ + 1) % kXBatch];
-  constexpr int kU = 8;  // (16 measured 4% slower: half the resident waves)
+  const T* __restrict__ pin = pb.p[T_];
+  T* __restrict__ pout = pb.p[(T_ + 1) % kXBatch];
+  // (16 for float measured 4% slower: half the resident waves)
+  constexpr int kU = sizeof(T) == 4 ? 8 : 4;
   // grid-stride over runs of kU kBlock points in dispatch order: the
   // workgroups in flight stream one window of the vectors together
   for (uint32_t nb = blockIdx.x * (kU * kBlock) + threadIdx.x; nb < n1;
        nb += (uint32_t)G * (kU * kBlock)) {
-    float pv[kU], zv[kU], pold[kXBatch][kU];
+    T pv[kU], zv[kU], pold[kXBatch][kU];
     double xv[kU];
+    float dv[kU];
 #pragma unroll
     for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
-      pv[u] = zv[u] = 0.f;
+      pv[u] = zv[u] = (T)0;
       xv[u] = 0.0;
+      dv[u] = 0.f;
 #pragma unroll
-      for (int q = 0; q < kXBatch; q++) pold[q][u] = 0.f;
+      for (int q = 0; q < kXBatch; q++) pold[q][u] = (T)0;
       if (n < n1) {
         pv[u] = __builtin_nontemporal_load(pin + n);
         if (flush) {
@@ -1250,7 +1295,10 @@ __global__ void __launch_bounds__(kBlock)
           for (int q = 0; q < T_; q++)
             if (use[q]) pold[q][u] = __builtin_nontemporal_load(pb.p[q] + n);
         }
-        if (!done) zv[u] = z[tmap(tm, g, n)];
+        if (!done) {
+          zv[u] = kPrec == PREC_ILU ? z[tmap(tm, g, n)] : z[n];
+          if constexpr (kPrec == PREC_DIAG) dv[u] = dg[n];
+        }
       }
     }
 #pragma unroll
@@ -1265,7 +1313,7 @@ __global__ void __launch_bounds__(kBlock)
           x = __builtin_fma(ax[T_], (double)pv[u], x);
           __builtin_nontemporal_store(x, xs + n);
         }
-        if (!done) pout[n] = beta * pv[u] + zv[u];
+        if (!done) pout[n] = beta * pv[u] + (kPrec == PREC_DIAG ? (T)dv[u] * zv[u] : zv[u]);
       }
     }
   }
@@ -1277,33 +1325,45 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-void launch_p_update_x(const Grid3& g, const Launch& L, int t, const PBuf& pb, const float* z,
-                       CgState* st, hipStream_t s, const TileMap& tm, double* xs,
-                       const double* xscale, unsigned* counter) {
-  const int G = L.Gpx[t & 3] > 0 ? L.Gpx[t & 3] : L.G;
+template <typename T, int kPrec>
+static void launch_p_update_x_t(const Grid3& g, const Launch& L, int t, const PBuf<T>& pb,
+                                const T* z, const float* dg, CgState* st, hipStream_t s,
+                                const TileMap& tm, double* xs, const double* xscale,
+                                unsigned* counter) {
+  const int* gp = sizeof(T) == 4 ? L.Gpx : L.Gpx64;
+  const int G = gp[t & 3] > 0 ? gp[t & 3] : L.G;
+  auto go = [&](auto tc) {
+    k_p_update_x<T, decltype(tc)::value, kPrec>
+        <<<G, kBlock, 0, s>>>(g, G, pb, z, dg, st, tm, xs, xscale, counter);
+  };
   switch (t) {
-    case 0:
-      k_p_update_x<0><<<G, kBlock, 0, s>>>(g, G, L.CH, pb, z, st, tm, xs, xscale, counter);
-      break;
-    case 1:
-      k_p_update_x<1><<<G, kBlock, 0, s>>>(g, G, L.CH, pb, z, st, tm, xs, xscale, counter);
-      break;
-    case 2:
-      k_p_update_x<2><<<G, kBlock, 0, s>>>(g, G, L.CH, pb, z, st, tm, xs, xscale, counter);
-      break;
-    default:
-      k_p_update_x<3><<<G, kBlock, 0, s>>>(g, G, L.CH, pb, z, st, tm, xs, xscale, counter);
-      break;
+    case 0: go(std::integral_constant<int, 0>{}); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    default: go(std::integral_constant<int, 3>{}); break;
   }
 }
 
+template <typename T>
+void launch_p_update_x(const Grid3& g, const Launch& L, int prec, int t, const PBuf<T>& pb,
+                       const T* z, const float* dg, CgState* st, hipStream_t s,
+                       const TileMap& tm, double* xs, const double* xscale, unsigned* counter) {
+  if (prec == PREC_ILU) {
+    launch_p_update_x_t<T, PREC_ILU>(g, L, t, pb, z, dg, st, s, tm, xs, xscale, counter);
+  } else if constexpr (sizeof(T) == 8) {
+    if (prec == PREC_DIAG)
+      launch_p_update_x_t<T, PREC_DIAG>(g, L, t, pb, z, dg, st, s, tm, xs, xscale, counter);
+    else
+      launch_p_update_x_t<T, PREC_NONE>(g, L, t, pb, z, dg, st, s, tm, xs, xscale, counter);
+  }
+}
 
 template <typename T>
-void launch_p_update(const Metric& m, const Grid3& g, const Launch& L, int prec, T* p,
+void launch_p_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* p,
                      const T* r, const T* z, CgState* st, hipStream_t s, const TileMap& tm,
                      double* xs, const double* xscale, unsigned* counter) {
   const int G = sizeof(T) == 8 && L.Gp > 0 ? L.Gp : L.G;
-  k_p_update<T><<<G, kBlock, 0, s>>>(m, g, G, L.CH, prec, p, r, z, st, tm, xs, xscale, counter);
+  k_p_update<T><<<G, kBlock, 0, s>>>(g, G, prec, dg, p, r, z, st, tm, xs, xscale, counter);
 }
 
 // s0 = x.y, s1 = u.v
@@ -1315,6 +1375,7 @@ __global__ void __launch_bounds__(kBlock)
   if (guard && st_done(st)) return;
   const int Lb = logical_block(G);
   const uint32_t n1 = g.N;
+  const bool own = u == x && v == x;  // x.y and x.x: x is read once
   double s0 = 0.0, s1 = 0.0;
   // 8 points per thread in flight; x and y read non-temporally (streams);
   // grid-stride over runs of kU kBlock points in dispatch order: the
@@ -1331,7 +1392,7 @@ __global__ void __launch_bounds__(kBlock)
         const uint32_t t = tmap(tm, g, n);
         xv[q] = __builtin_nontemporal_load(x + t);
         yv[q] = __builtin_nontemporal_load(y + t);
-        if (u) {
+        if (u && !own) {
           uv[q] = u[t];
           vv[q] = v[t];
         }
@@ -1342,7 +1403,7 @@ __global__ void __launch_bounds__(kBlock)
       const uint32_t n = nb + q * kBlock;
       if (n < n1) {
         s0 += (double)xv[q] * (double)yv[q];
-        if (u) s1 += (double)uv[q] * (double)vv[q];
+        if (u) s1 += own ? (double)xv[q] * (double)xv[q] : (double)uv[q] * (double)vv[q];
       }
     }
   }
@@ -1363,8 +1424,8 @@ void launch_dot2(const Grid3& g, const Launch& L, const T* x, const T* y, const 
 // z = M^-1 r (DIAG/NONE), reductions s0=r.z, s1=r.r.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    k_point_prec(Metric m, Grid3 g, int G, int CH, int prec, const T* __restrict__ r,
-                 T* __restrict__ z, CgState* st, double* partial, unsigned* counter, Epi epi,
+    k_point_prec(Grid3 g, int G, int CH, int prec, const float* __restrict__ dg,
+                 const T* __restrict__ r, T* __restrict__ z, CgState* st, double* partial, unsigned* counter, Epi epi,
                  double* out) {
   const int Lb = logical_block(G);
   const uint32_t n0 = (uint32_t)Lb * (uint32_t)CH;
@@ -1372,7 +1433,7 @@ __global__ void __launch_bounds__(kBlock)
   double s0 = 0.0, s1 = 0.0;
   for (uint32_t n = n0 + threadIdx.x; n < n1; n += kBlock) {
     const T rn = r[n];
-    const T zn = apply_point_prec<T>(m, g, prec, n, rn);
+    const T zn = prec == PREC_DIAG ? (T)dg[n] * rn : rn;
     z[n] = zn;
     s0 += (double)rn * (double)zn;
     s1 += (double)rn * (double)rn;
@@ -1383,10 +1444,10 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 template <typename T>
-void launch_point_prec(const Metric& m, const Grid3& g, const Launch& L, int prec, const T* r,
+void launch_point_prec(const Grid3& g, const Launch& L, int prec, const float* dg, const T* r,
                        T* z, CgState* st, Reduce red, int slot, Epi epi, double* out,
                        hipStream_t s) {
-  k_point_prec<T><<<L.G, kBlock, 0, s>>>(m, g, L.G, L.CH, prec, r, z, st, red.partial,
+  k_point_prec<T><<<L.G, kBlock, 0, s>>>(g, L.G, L.CH, prec, dg, r, z, st, red.partial,
                                           red.counter + (size_t)slot * kRedSlotWords, epi, out);
 }
 
@@ -1887,16 +1948,19 @@ void launch_getb(const EnergyMesh& em, int nr, int nt, int np, const double* phi
   template void launch_stencil<T>(const Metric&, const Grid3&, const Launch&, const T*, T*,     \
                                   const T*, int, const double*, CgState*, Reduce, int, Epi,     \
                                   double*, bool, hipStream_t, const TileMap&);                  \
-  template void launch_cg_update<T>(const Metric&, const Grid3&, const Launch&, int, T*, T*,    \
+  template void launch_cg_update<T>(const Grid3&, const Launch&, int, const float*, T*, T*,     \
                                     const T*, const T*, CgState*, Reduce, int, hipStream_t,     \
                                     double*, const double*, const TileMap&);                    \
-  template void launch_p_update<T>(const Metric&, const Grid3&, const Launch&, int, T*,         \
+  template void launch_p_update_x<T>(const Grid3&, const Launch&, int, int, const PBuf<T>&,     \
+                                     const T*, const float*, CgState*, hipStream_t,             \
+                                     const TileMap&, double*, const double*, unsigned*);        \
+  template void launch_p_update<T>(const Grid3&, const Launch&, int, const float*, T*,          \
                                    const T*, const T*, CgState*, hipStream_t, const TileMap&,   \
                                    double*, const double*, unsigned*);                          \
   template void launch_dot2<T>(const Grid3&, const Launch&, const T*, const T*, const T*,       \
                                const T*, CgState*, Reduce, int, Epi, double*, bool,             \
                                hipStream_t, const TileMap&);                                    \
-  template void launch_point_prec<T>(const Metric&, const Grid3&, const Launch&, int, const T*, \
+  template void launch_point_prec<T>(const Grid3&, const Launch&, int, const float*, const T*,  \
                                      T*, CgState*, Reduce, int, Epi, double*, hipStream_t);     \
   template void launch_sub<T>(const Grid3&, const Launch&, T*, const T*, hipStream_t,           \
                               const TileMap&);                                                  \
@@ -1927,17 +1991,21 @@ void size_stream_grids(Launch& L, int ncu, uint32_t N) {
     const int G = nb * ncu / 8 * 8;
     return G >= 8 && G < L.G ? G : 0;
   };
-  L.Gcg = fit(k_cg_update<double>);
+  L.Gcg = fit(k_cg_update<double, false>);
   if (L.Gcg > 0) {
     const uint32_t ch = (N + (uint32_t)L.Gcg - 1) / (uint32_t)L.Gcg;
     L.CHcg = (int)((ch + kBlock - 1) / kBlock * kBlock);
   }
   L.Gp = fit(k_p_update<double>);
   L.Gd2 = fit(k_dot2<double>);
-  L.Gpx[0] = fit(k_p_update_x<0>);
-  L.Gpx[1] = fit(k_p_update_x<1>);
-  L.Gpx[2] = fit(k_p_update_x<2>);
-  L.Gpx[3] = fit(k_p_update_x<3>);
+  L.Gpx[0] = fit(k_p_update_x<float, 0, PREC_ILU>);
+  L.Gpx[1] = fit(k_p_update_x<float, 1, PREC_ILU>);
+  L.Gpx[2] = fit(k_p_update_x<float, 2, PREC_ILU>);
+  L.Gpx[3] = fit(k_p_update_x<float, 3, PREC_ILU>);
+  L.Gpx64[0] = fit(k_p_update_x<double, 0, PREC_ILU>);
+  L.Gpx64[1] = fit(k_p_update_x<double, 1, PREC_ILU>);
+  L.Gpx64[2] = fit(k_p_update_x<double, 2, PREC_ILU>);
+  L.Gpx64[3] = fit(k_p_update_x<double, 3, PREC_ILU>);
   L.Gru = fit(k_r_update);
 }
 

@@ -98,10 +98,11 @@ struct Launch {
   // patches (3 tall, 4 short), -1 the LDS-staged patches where they apply
   int stencil = -1;
   // grid-stride kernels whose registers allow fewer than G resident
-  // workgroups (the grouped p update, t = 0..3, and the FP32 r update):
+  // workgroups (the grouped p update in FP32 and FP64,
+  // t = 0..3, and the FP32 r update):
   // as many workgroups as the device holds at once (0: G), so that no
   // second wave of workgroups streams its share alone at the end
-  int Gpx[4] = {0, 0, 0, 0};
+  int Gpx[4] = {0, 0, 0, 0}, Gpx64[4] = {0, 0, 0, 0};
   int Gru = 0;
   // the same for the FP64 CG update (chunks of CHcg points), p update and
   // dot products
@@ -151,22 +152,26 @@ void launch_stencil(const Metric& m, const Grid3& g, const Launch& L, const T* x
 void launch_r_update(uint32_t n_all, const Launch& Lt, float* r, const float* ap,
                      const CgState* st, hipStream_t s);
 
-// CG update x += alpha p, r -= alpha ap, and for PREC_DIAG/NONE the reduction
-// of r.z and r.r with epilogue EPI_RITER; for PREC_ILU only r.r (EPI_RR).
-// With xs non-null the solution update goes to the FP64 vector xs instead:
-// xs += (alpha * *xscale) p (x is not touched).
+// The diagonal preconditioner's factors (N floats), dg below.
+void launch_diag_inv(const Metric& m, const Grid3& g, float* d, hipStream_t s);
+
+// CG update r -= alpha ap, and for PREC_DIAG/NONE the reduction of r.z and r.r
+// with epilogue EPI_RITER; for PREC_ILU only r.r (EPI_RR).  With x non-null
+// also x += alpha p; with xs non-null the solution update goes to the FP64
+// vector xs instead: xs += (alpha * *xscale) p (x is not touched).
 template <typename T>
-void launch_cg_update(const Metric& m, const Grid3& g, const Launch& L, int prec, T* x, T* r,
+void launch_cg_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* x, T* r,
                       const T* p, const T* ap, CgState* st, Reduce red, int slot,
                       hipStream_t s, double* xs = nullptr, const double* xscale = nullptr,
                       const TileMap& tm = TileMap{});
 
-// p update of the FP32 recurrence at iteration t of a group of kXBatch,
-// with the group's FP64 solution updates at its last iteration (or when the
-// recurrence has stopped): k_p_update_x in p3d_kernels.hip.
-void launch_p_update_x(const Grid3& g, const Launch& L, int t, const PBuf& pb, const float* z,
-                       CgState* st, hipStream_t s, const TileMap& tm, double* xs,
-                       const double* xscale, unsigned* counter);
+// p update at iteration t of a group of kXBatch, with the group's FP64
+// solution updates at its last iteration (or when the recurrence has stopped):
+// k_p_update_x in p3d_kernels.hip.  T float: PREC_ILU only.
+template <typename T>
+void launch_p_update_x(const Grid3& g, const Launch& L, int prec, int t, const PBuf<T>& pb,
+                       const T* z, const float* dg, CgState* st, hipStream_t s,
+                       const TileMap& tm, double* xs, const double* xscale, unsigned* counter);
 
 // p = z + beta p (z = M^-1 r computed in place for DIAG/NONE, read for ILU).
 // tm: placement of r (cg_update) and z (p_update) (natural by default).
@@ -174,7 +179,7 @@ void launch_p_update_x(const Grid3& g, const Launch& L, int t, const PBuf& pb, c
 // solution update xs += (alpha * *xscale) p, once per iteration
 // (CgState::x_ncg; counter: a reduction slot's counter).
 template <typename T>
-void launch_p_update(const Metric& m, const Grid3& g, const Launch& L, int prec, T* p,
+void launch_p_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* p,
                      const T* r, const T* z, CgState* st, hipStream_t s,
                      const TileMap& tm = TileMap{}, double* xs = nullptr,
                      const double* xscale = nullptr, unsigned* counter = nullptr);
@@ -188,7 +193,7 @@ void launch_dot2(const Grid3& g, const Launch& L, const T* x, const T* y, const 
 
 // z = M^-1 r for DIAG/NONE (r,z may alias), with optional s0=r.z, s1=r.r.
 template <typename T>
-void launch_point_prec(const Metric& m, const Grid3& g, const Launch& L, int prec, const T* r,
+void launch_point_prec(const Grid3& g, const Launch& L, int prec, const float* dg, const T* r,
                        T* z, CgState* st, Reduce red, int slot, Epi epi, double* out,
                        hipStream_t s);
 

@@ -57,9 +57,10 @@ struct Vecs {
   T *x, *r, *p, *ap, *z;
   double* xs = nullptr;             // FP64 solution updated instead of x (FP32 recurrence)
   const double* xscale = nullptr;  // scale of the FP32 system (device)
-  // FP32 recurrence with the FP64 solution on tile-major r, ap, z: the
-  // kXBatch rotating direction buffers (pb.p[0] = p), x updated per group
-  PBuf pb{};
+  // the kXBatch rotating direction buffers (pb.p[0] = p) when x is updated
+  // once per group of iterations: the FP64 recurrence, and the FP32 one with
+  // the FP64 solution on tile-major r, ap, z
+  PBuf<T> pb{};
 };
 
 struct p3d_solver {
@@ -82,7 +83,10 @@ struct p3d_solver {
   float* yv = nullptr;
   float* dinv = nullptr;
   float *x32 = nullptr, *r32 = nullptr, *p32 = nullptr, *ap32 = nullptr, *z32 = nullptr;
-  float* p32b[kXBatch - 1] = {};  // the other direction buffers of the grouped x updates
+  // the other direction buffers of the grouped x updates
+  float* p32b[kXBatch - 1] = {};
+  double* pb64[kXBatch - 1] = {};
+  bool pb64_tried = false;
   // r, z (and r32, z32) hold nvec >= N entries: with the single-wave tile
   // sweeps they are tile-major (tm.on), every other vector is natural
   size_t nvec = 0;
@@ -144,13 +148,30 @@ __global__ void k_convert(uint32_t n, const A* __restrict__ src, B* __restrict__
   if (q < n) dst[q] = (B)src[q];
 }
 
+// Memory the FP64 recurrence can do without (its x is then updated in every
+// iteration) is given back before an allocation that cannot fails.
+static int dalloc_or_yield(p3d_solver* s, void** p, size_t bytes) {
+  if (hipMalloc(p, bytes) == hipSuccess) return P3D_OK;
+  (void)hipGetLastError();
+  (void)hipStreamSynchronize(s->stream);
+  for (double*& b : s->pb64) {
+    if (b) hipFree(b);
+    b = nullptr;
+  }
+  if (s->gexec[0]) hipGraphExecDestroy(s->gexec[0]);
+  s->gexec[0] = nullptr;
+  return dalloc(p, bytes);
+}
+
 static int ensure_mixed(p3d_solver* s) {
   if (s->x32) return P3D_OK;
   const size_t nb = (size_t)s->g.N * sizeof(float), nv = s->nvec * sizeof(float);
   int rc;
-  if ((rc = dalloc((void**)&s->x32, nb)) || (rc = dalloc((void**)&s->r32, nv)) ||
-      (rc = dalloc((void**)&s->p32, nb)) || (rc = dalloc((void**)&s->ap32, nv)) ||
-      (rc = dalloc((void**)&s->z32, nv)))
+  if ((rc = dalloc_or_yield(s, (void**)&s->x32, nb)) ||
+      (rc = dalloc_or_yield(s, (void**)&s->r32, nv)) ||
+      (rc = dalloc_or_yield(s, (void**)&s->p32, nb)) ||
+      (rc = dalloc_or_yield(s, (void**)&s->ap32, nv)) ||
+      (rc = dalloc_or_yield(s, (void**)&s->z32, nv)))
     return rc;
   HIPCHK(hipMemsetAsync(s->r32, 0, nv, s->stream));
   HIPCHK(hipMemsetAsync(s->z32, 0, nv, s->stream));
@@ -163,9 +184,35 @@ static int ensure_mixed(p3d_solver* s) {
 static int ensure_pbuf(p3d_solver* s) {
   int rc;
   for (int q = 0; q < kXBatch - 1; q++)
-    if (!s->p32b[q] && (rc = dalloc((void**)&s->p32b[q], (size_t)s->g.N * sizeof(float))))
+    if (!s->p32b[q] &&
+        (rc = dalloc_or_yield(s, (void**)&s->p32b[q], (size_t)s->g.N * sizeof(float))))
       return rc;
   return P3D_OK;
+}
+
+// The FP64 recurrence's vectors; with its direction buffers (natural order, N
+// doubles each) x is updated once per group of iterations.  Without memory
+// for them x is updated in every iteration.
+static Vecs<double> fp64_vecs(p3d_solver* s) {
+  Vecs<double> v{s->x, s->r, s->p, s->ap, s->z};
+  if (!s->pb64_tried) {
+    s->pb64_tried = true;
+    bool ok = true;
+    for (double*& b : s->pb64)
+      ok = ok && hipMalloc((void**)&b, (size_t)s->g.N * sizeof(double)) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      for (double*& b : s->pb64) {
+        if (b) hipFree(b);
+        b = nullptr;
+      }
+    }
+  }
+  if (s->pb64[0]) {
+    v.pb.p[0] = s->p;
+    for (int q = 1; q < kXBatch; q++) v.pb.p[q] = s->pb64[q - 1];
+  }
+  return v;
 }
 
 // Placement of r and z: tile-major exactly when the single-wave tile
@@ -264,18 +311,18 @@ static bool fuse_rupd_available(const p3d_solver* s) {
 }
 
 // Preconditioner application r -> z (+ fused dots with epilogue).
-// ap_upd (FP32 register tiles, guard set): the residual update r -= alpha ap
-// is folded into the forward sweep (r is written).
+// ap_upd (FP32 register tiles or columns, guard set): the residual update
+// r -= alpha ap is folded into the forward sweep (r is written).
 template <typename T>
 static void prec_and_dot(p3d_solver* s, const T* r, T* z, Epi epi, double* out, bool guard,
-                         const float* ap_upd = nullptr) {
+                         const T* ap_upd = nullptr) {
   if (s->ifprec == PREC_ILU) {
     const CgState* gd = guard ? s->st : nullptr;
     if (columns_on(s)) {
       launch_dilu_columns<T>(s->col, s->m, s->g, const_cast<T*>(r), z, gd, ap_upd, s->stream);
     } else if (s->sweep_mode == 0 && s->sweep_ready) {
       if constexpr (sizeof(T) == 4) {
-        if (ap_upd)
+        if (ap_upd)  // (FP64 folds it only with the columns)
           launch_dilu_tiles_rupd(s->sweep, s->m, s->g, const_cast<float*>(r), ap_upd, z, gd,
                                  s->stream);
         else
@@ -296,55 +343,69 @@ static void prec_and_dot(p3d_solver* s, const T* r, T* z, Epi epi, double* out, 
                        s->tm);
     }
   } else {
-    launch_point_prec<T>(s->m, s->g, s->L, s->ifprec, r, z, s->st, s->red, 1, epi, out,
+    launch_point_prec<T>(s->g, s->L, s->ifprec, s->dinv, r, z, s->st, s->red, 1, epi, out,
                          s->stream);
   }
 }
 
+// The FP64 recurrence with the column sweeps: r -= alpha ap goes with the
+// forward sweep, as in the FP32 one (ap is then tile-major like r).
+static bool fp64_folds_rupd(const p3d_solver* s) { return columns_on(s) && s->fuse_rupd != 0; }
+
 // One CG iteration; t is its place in the group of kXBatch iterations of
-// the FP32 recurrence's grouped solution updates (unused otherwise).
+// the grouped solution updates (unused otherwise).
 template <typename T>
 static void cg_iteration(p3d_solver* s, Vecs<T> v, int t) {
-  if constexpr (sizeof(T) == 4) {
-    if (v.xs && s->tm.on && v.pb.p[0]) {
-      // FP32 recurrence with the FP64 solution and tile-major r, ap, z:
-      // every pass contiguous except the p update's read of z; direction
-      // p_t in buffer t of the group, the FP64 x updated once per group
-      float* p = v.pb.p[t];
-      launch_pole_sums<float>(s->m, s->g, p, s->pole_part, s->stream);
-      launch_stencil<float>(s->m, s->g, s->L, p, v.ap, nullptr, 0, s->pole_part, s->st, s->red,
-                            0, EPI_PAP, nullptr, true, s->stream, s->tm);
-      // r -= alpha ap, in the forward sweep of the register tiles where they
-      // run, else on its own; then z = M^-1 r and r.z, r.r together
-      const bool fused = (s->fuse_rupd == 1 ||
-                          (s->fuse_rupd < 0 && (columns_on(s) || s->g.N >= (1u << 26)))) &&
-                         fuse_rupd_available(s);
-      if (!fused) launch_r_update(s->gt.N, s->Lt, v.r, v.ap, s->st, s->stream);
-      prec_and_dot<float>(s, v.r, v.z, EPI_RITER, nullptr, true, fused ? v.ap : nullptr);
-      launch_p_update_x(s->g, s->L, t, v.pb, v.z, s->st, s->stream, s->tm, v.xs, v.xscale,
-                        s->red.counter + 5 * kRedSlotWords);
-      return;
+  if (v.pb.p[0]) {
+    // direction p_t in buffer t of the group, the solution updated once per
+    // group
+    T* p = v.pb.p[t];
+    launch_pole_sums<T>(s->m, s->g, p, s->pole_part, s->stream);
+    // FP32 (tile-major r, ap, z): every pass contiguous except the p update's
+    // read of z.  r -= alpha ap in the forward sweep where it runs there,
+    // else on its own; then z = M^-1 r and r.z, r.r together
+    const bool f32 = sizeof(T) == 4;
+    const bool fused = f32 ? (s->fuse_rupd == 1 ||
+                              (s->fuse_rupd < 0 && (columns_on(s) || s->g.N >= (1u << 26)))) &&
+                                 fuse_rupd_available(s)
+                           : fp64_folds_rupd(s);
+    launch_stencil<T>(s->m, s->g, s->L, p, v.ap, nullptr, 0, s->pole_part, s->st, s->red, 0,
+                      EPI_PAP, nullptr, true, s->stream, f32 || fused ? s->tm : TileMap{});
+    if (f32 || fused) {
+      if constexpr (sizeof(T) == 4)
+        if (!fused) launch_r_update(s->gt.N, s->Lt, v.r, v.ap, s->st, s->stream);
+      prec_and_dot<T>(s, v.r, v.z, EPI_RITER, nullptr, true, fused ? v.ap : nullptr);
+    } else {
+      launch_cg_update<T>(s->g, s->L, s->ifprec, s->dinv, nullptr, v.r, p, v.ap, s->st, s->red, 2,
+                          s->stream, nullptr, nullptr, s->tm);
+      if (s->ifprec == PREC_ILU) prec_and_dot<T>(s, v.r, v.z, EPI_RZITER, nullptr, true);
     }
+    launch_p_update_x<T>(s->g, s->L, s->ifprec, t, v.pb, s->ifprec == PREC_ILU ? v.z : v.r,
+                         s->dinv, s->st, s->stream, s->tm, f32 ? v.xs : (double*)v.x, v.xscale,
+                         s->red.counter + 5 * kRedSlotWords);
+    return;
   }
   launch_pole_sums<T>(s->m, s->g, v.p, s->pole_part, s->stream);
   launch_stencil<T>(s->m, s->g, s->L, v.p, v.ap, nullptr, 0, s->pole_part, s->st, s->red, 0,
                     EPI_PAP, nullptr, true, s->stream);
-  launch_cg_update<T>(s->m, s->g, s->L, s->ifprec, v.x, v.r, v.p, v.ap, s->st, s->red, 2,
+  launch_cg_update<T>(s->g, s->L, s->ifprec, s->dinv, v.x, v.r, v.p, v.ap, s->st, s->red, 2,
                       s->stream, v.xs, v.xscale, s->tm);
   if (s->ifprec == PREC_ILU) prec_and_dot<T>(s, v.r, v.z, EPI_RZITER, nullptr, true);
-  launch_p_update<T>(s->m, s->g, s->L, s->ifprec, v.p, v.r, v.z, s->st, s->stream, s->tm);
+  launch_p_update<T>(s->g, s->L, s->ifprec, s->dinv, v.p, v.r, v.z, s->st, s->stream, s->tm);
 }
 
 template <typename T>
 static int chunk_size(p3d_solver* s) {
-  if (s->chunk > 0) return s->chunk;
+  // whole groups of the grouped solution updates
+  if (s->chunk > 0) return (s->chunk + kXBatch - 1) / kXBatch * kXBatch;
   if (s->ifprec == PREC_ILU) {
-    const int per = (s->sweep_mode == 0 && s->sweep_ready) ? 2 * s->sweep.ndiag + 6
-                                                           : 2 * (s->g.a + s->g.b + s->g.c);
+    const int per = columns_on(s) ? 8
+                    : (s->sweep_mode == 0 && s->sweep_ready)
+                        ? 2 * s->sweep.ndiag + 6
+                        : 2 * (s->g.a + s->g.b + s->g.c);
     int k = 4096 / per;
     if (k > 32) k = 32;
-    // whole groups of the FP32 recurrence's grouped solution updates
-    if (sizeof(T) == 4) k = k / kXBatch * kXBatch;
+    k = k / kXBatch * kXBatch;
     return k < kXBatch ? kXBatch : k;
   }
   return 32;
@@ -428,6 +489,10 @@ static int pcg(p3d_solver* s, Vecs<T> v, double epscg, int ncgmax, int stop_mode
   launch_sub<T>(s->g, s->L, v.r, v.ap, s->stream, s->tm);
   prec_and_dot<T>(s, v.r, v.z, EPI_RINIT, nullptr, false);
   launch_copy<T>(s->g, s->L, v.p, v.z, s->stream, s->tm, 0);
+  // with the residual update in the forward sweep ap is tile-major from here
+  // on: nothing but zero outside the grid (r takes it over there)
+  if (sizeof(T) == 8 && v.pb.p[0] && fp64_folds_rupd(s))
+    HIPCHK(hipMemsetAsync(v.ap, 0, s->nvec * sizeof(T), s->stream));
   if ((rc = read_state(s))) return rc;
   return run_until_done<T>(s, v);
 }
@@ -665,7 +730,8 @@ static int solve_mixed_ru(p3d_solver* s, double epscg, int ncgmax) {
       HIPCHK(hipMemcpyAsync(&s->st->p_cur, &s->st_host->p_cur, sizeof(int),
                             hipMemcpyHostToDevice, s->stream));
     }
-    launch_p_update<float>(s->m, s->g, s->L, s->ifprec, v.p, v.r, v.z, s->st, s->stream, s->tm);
+    launch_p_update<float>(s->g, s->L, s->ifprec, s->dinv, v.p, v.r, v.z, s->st, s->stream,
+                           s->tm);
     if ((rc = read_state(s))) return rc;
   }
   s->stats.relres = s->stats.true_relres = relres;
@@ -712,8 +778,7 @@ static int solve_core(p3d_solver* s, double epscg, int ncgmax, int ncghist) {
     HIPCHK(hipStreamSynchronize(s->stream));
   } else {
     launch_copy<double>(s->g, s->L, s->r, s->b, s->stream, s->tm, 1);
-    Vecs<double> v{s->x, s->r, s->p, s->ap, s->z};
-    if ((rc = pcg<double>(s, v, epscg, ncgmax, s->stop_mode))) return rc;
+    if ((rc = pcg<double>(s, fp64_vecs(s), epscg, ncgmax, s->stop_mode))) return rc;
     print_history(s, ncghist);
     s->stats.ncg = s->st_host->ncg;
     s->stats.status = s->st_host->done;
@@ -788,6 +853,8 @@ int p3d_destroy(p3d_solver* s) {
   for (void* b : bufs)
     if (b) hipFree(b);
   for (float* b : s->p32b)
+    if (b) hipFree(b);
+  for (double* b : s->pb64)
     if (b) hipFree(b);
   free_sweep_plan(s->sweep);
   free_column_plan(s->col);
@@ -958,7 +1025,7 @@ int p3d_create(p3d_solver** out, int nr, int nt, int np, const double* r, const 
   }
   const size_t nbv = s->nvec * sizeof(double);
   if ((rc = dalloc((void**)&s->x, nb)) || (rc = dalloc((void**)&s->r, nbv)) ||
-      (rc = dalloc((void**)&s->p, nb)) || (rc = dalloc((void**)&s->ap, nb)) ||
+      (rc = dalloc((void**)&s->p, nb)) || (rc = dalloc((void**)&s->ap, nbv)) ||
       (rc = dalloc((void**)&s->z, nbv)) || (rc = dalloc((void**)&s->b, nb)))
     return bail(rc);
   hipMemset(s->r, 0, nbv);
@@ -991,6 +1058,12 @@ int p3d_create(p3d_solver** out, int nr, int nt, int np, const double* r, const 
   hipMemset(s->x, 0, nb);
   hipMemset(s->b, 0, nb);
   hipMemset(s->pole_part, 0, sizeof(double) * 2 * kPoleSegs * a);
+  if (ifprec == PREC_DIAG) {
+    if ((rc = dalloc((void**)&s->dinv, N * sizeof(float)))) return bail(rc);
+    launch_diag_inv(s->m, s->g, s->dinv, s->stream);
+    if (hipStreamSynchronize(s->stream) != hipSuccess)
+      return bail(fail(P3D_EHIP, "diagonal preconditioner failed"));
+  }
   if (ifprec == 2) {
     auto t0 = std::chrono::steady_clock::now();
     if ((rc = dalloc((void**)&s->yv, N * sizeof(float))) ||
@@ -1463,14 +1536,17 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   init.bb = 1.0;
   init.epscg = 0.0;
   init.ncgmax = 1 << 30;
-  init.ncg = which == 8 ? kXBatch : 1;
+  const Vecs<double> v = fp64_vecs(s);
+  const bool grouped = which == 8 || (which == 5 && v.pb.p[0]);
+  init.ncg = grouped ? kXBatch : 1;
   *s->st_host = init;
   s->out_host[4] = 1.0;
   HIPCHK(hipMemcpyAsync(s->out + 4, s->out_host + 4, sizeof(double), hipMemcpyHostToDevice,
                         s->stream));
   HIPCHK(hipMemcpyAsync(s->st, s->st_host, sizeof(CgState), hipMemcpyHostToDevice, s->stream));
-  Vecs<double> v{s->x, s->r, s->p, s->ap, s->z};
   if (which == 3) {
+    if (v.pb.p[0] && fp64_folds_rupd(s))
+      HIPCHK(hipMemsetAsync(v.ap, 0, s->nvec * sizeof(double), s->stream));
     // one genuine PCG run (r0 = p0 = 1, x0 = 0, never converging) replayed
     // through the captured graph: milliseconds per iteration
     launch_fill(s->x, 0.0, (size_t)s->g.N, s->stream);
@@ -1510,12 +1586,22 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
         prec_and_dot<double>(s, s->r, s->z, EPI_NONE, nullptr, false);
         break;
       case 4:
-        launch_cg_update<double>(s->m, s->g, s->L, s->ifprec, s->x, s->r, s->p, s->ap, s->st,
-                                 s->red, 2, s->stream, nullptr, nullptr, s->tm);
+        launch_cg_update<double>(s->g, s->L, s->ifprec, s->dinv, v.pb.p[0] ? nullptr : s->x, s->r,
+                                 s->p, s->ap, s->st, s->red, 2, s->stream, nullptr, nullptr,
+                                 s->tm);
         break;
       case 5:
-        launch_p_update<double>(s->m, s->g, s->L, s->ifprec, s->p, s->r, s->z, s->st,
-                                s->stream, s->tm);
+        if (!v.pb.p[0]) {
+          launch_p_update<double>(s->g, s->L, s->ifprec, s->dinv, s->p, s->r, s->z, s->st,
+                                  s->stream, s->tm);
+          break;
+        }
+        (void)hipMemsetAsync(&s->st->x_ncg, 0, sizeof(int), s->stream);  // checked below
+        for (int t = 0; t < kXBatch; t++)
+          launch_p_update_x<double>(s->g, s->L, s->ifprec, t, v.pb,
+                                    s->ifprec == PREC_ILU ? s->z : s->r, s->dinv, s->st,
+                                    s->stream, s->tm, s->x, nullptr,
+                                    s->red.counter + 5 * kRedSlotWords);
         break;
       case 6:  // plain copy of N doubles: the bandwidth reference
         launch_copy<double>(s->g, s->L, s->ap, s->p, s->stream);
@@ -1527,13 +1613,13 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
         // last with the FP64 solution update of the whole group; x_ncg cleared
         // so that it applies kXBatch pending updates; alpha = 0 leaves x);
         // timed per iteration
-        PBuf pb{};
+        PBuf<float> pb{};
         pb.p[0] = s->p32;
         for (int q = 1; q < kXBatch; q++) pb.p[q] = s->p32b[q - 1];
         (void)hipMemsetAsync(&s->st->x_ncg, 0, sizeof(int), s->stream);  // checked below
         for (int t = 0; t < kXBatch; t++)
-          launch_p_update_x(s->g, s->L, t, pb, s->z32, s->st, s->stream, s->tm, s->x,
-                            s->out + 4, s->red.counter + 5 * kRedSlotWords);
+          launch_p_update_x<float>(s->g, s->L, PREC_ILU, t, pb, s->z32, s->dinv, s->st, s->stream,
+                                   s->tm, s->x, s->out + 4, s->red.counter + 5 * kRedSlotWords);
         break;
       }
       case 9:  // residual update of the FP32 recurrence (tile-major r, ap)
@@ -1565,7 +1651,7 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   hipEventDestroy(e0);
   hipEventDestroy(e1);
   HIPCHK(hipGetLastError());
-  *avg_ms = (double)ms / reps / (which == 8 ? kXBatch : 1);
+  *avg_ms = (double)ms / reps / (grouped ? kXBatch : 1);
   if (which > 11 || which < 0) return fail(P3D_EINVAL, "unknown kernel id %d", which);
   return P3D_OK;
 }
