@@ -26,6 +26,15 @@
 // call over with the tile schedules.
 //
 // Per-point arithmetic and order are those of p3d_sweep.hip: the same bits.
+//
+// Stored couplings (the legacy CSR input, any values): the same march on x in
+// natural order, the three couplings of a point and its pivot inverse as one
+// 16-byte word per step and lane, laid out in marching order for each
+// direction (32 bytes per unknown instead of the 12 that the couplings and
+// dinv take once in natural order, but one coalesced load of 1 KB per step).
+// What bounds it: the chain, as above.  One call of the drop-in interface,
+// tiles and columns: 333 and 85 us at 20x31x60, 1429 and 167 us at 51x91x181,
+// 3448 and 368 us at 101x181x361, 7.06 and 0.87 ms at 151x301x601.
 #include <type_traits>
 #include <vector>
 
@@ -88,8 +97,15 @@ struct ColLds {
   float2 f[2][kCU][16];
 };
 
-// Phi factors of the couplings (ColArgs::mode).
-enum { kPhiAny = 0, kPhiCut = 1, kPhiUniform = 2 };
+// With stored couplings, those of 32 steps besides: (k, j) and i.  Written two
+// chunks and read one chunk ahead, so four chunks of rows do.
+struct ColLdsStored : ColLds {
+  float2 ckj[kCS][64];
+  float ci[kCS][64];
+};
+
+// Phi factors of the couplings (ColArgs::mode), or the couplings themselves.
+enum { kPhiAny = 0, kPhiCut = 1, kPhiUniform = 2, kStored = 3 };
 
 // Offset of plane k of column col in a tile-major vector (TileMap); 32 bits
 // hold it (build_column_plan).
@@ -128,7 +144,7 @@ struct ColCtx {
   size_t fbase, sk;  // this column's faces; its row kFront of dinv_s and y_s
 };
 
-template <bool kFwd>
+template <bool kFwd, bool kSt = false>
 __device__ __forceinline__ ColCtx col_ctx(const Metric& m, const Grid3& g, const ColArgs& ca) {
   ColCtx x;
   x.lane = threadIdx.x & 63;
@@ -141,8 +157,11 @@ __device__ __forceinline__ ColCtx col_ctx(const Metric& m, const Grid3& g, const
   x.J = x.col / ca.NI;
   const int i = x.I * 8 + x.ii, j = x.J * 8 + x.jj;
   x.act = i < g.a && j < g.b;
-  x.cp = kFwd ? sweep_coup_lower(m, x.act ? i : 0, x.act ? j : 0)
-              : sweep_coup_upper(m, x.act ? i : 0, x.act ? j : 0);
+  if constexpr (kSt)
+    x.cp = SweepCoup{};
+  else
+    x.cp = kFwd ? sweep_coup_lower(m, x.act ? i : 0, x.act ? j : 0)
+                : sweep_coup_upper(m, x.act ? i : 0, x.act ? j : 0);
   x.stamp = __hip_atomic_load(ca.ctr + (kFwd ? 0 : 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   x.fbase = (size_t)x.col * ca.face_rows * 8;
   x.sk = ((size_t)x.col * ca.rows_alloc + kFront) * 64;
@@ -159,24 +178,38 @@ __device__ __forceinline__ ColCtx col_ctx(const Metric& m, const Grid3& g, const
 template <bool kFwd, int kMode>
 __device__ __forceinline__ void march(const Metric& m, const ColArgs& ca, const ColCtx& x,
                                       ColLds& sh, const float2* pf) {
+  constexpr bool kTable = kMode == kPhiAny || kMode == kPhiCut;
+  const ColLdsStored& st = (const ColLdsStored&)sh;  // (with kStored only)
   const int lane = x.lane, dly = kFwd ? x.dl : kDelay - x.dl;
   const int nbr = (kFwd ? (lane - 8) & 63 : (lane + 8) & 63) << 2;
   const bool edge_i = x.ii == (kFwd ? 0 : 7), edge_j = x.jj == (kFwd ? 0 : 7);
   // the lane's face entry: its row's for i, its column's for j, the lane on
   // both edges entry 0 (the j faces are numbered from that lane)
   const int fe = edge_i ? (kFwd ? x.jj : 7 - x.jj) : 8 + (kFwd ? x.ii : 7 - x.ii);
-  const float wc = ca.bl.wrap ? x.cp.k * (kFwd ? m.FDPU[m.c - 1] : m.FDPL[0]) : 0.f;
+  // coupling of the phi wrap
+  float wc = 0.f;
+  if constexpr (kMode == kStored) {
+    if (x.act && ca.bl.wrap)
+      wc = (kFwd ? ca.wrap_lo : ca.wrap_up)[x.I * 8 + x.ii + m.a * (x.J * 8 + x.jj)];
+  } else {
+    if (ca.bl.wrap) wc = x.cp.k * (kFwd ? m.FDPU[m.c - 1] : m.FDPL[0]);
+  }
   // first and last plane of the grid, counted in marching order
   const int q_first = kFwd ? 0 : ca.skip, q_last = q_first + ca.c - 1;
   const float2* pfl = pf + (kDelay - dly);
   const float ck0 = x.cp.k * ca.u_k, cj0 = x.cp.j * ca.u_d, ci0 = x.cp.i * ca.u_d;
   float t = 0.f, t_w = 0.f, nj[kJ] = {};  // nj: from the j neighbour, oldest first
   float2 rd[2][kCU], cf[2][kCU];
+  float cg[2][kCU];
   lds_barrier();
 #pragma unroll
   for (int u = 0; u < kCU; u++) {
     rd[0][u] = sh.v[u][lane];
-    if constexpr (kMode != kPhiUniform) cf[0][u] = pfl[u];
+    if constexpr (kTable) cf[0][u] = pfl[u];
+    if constexpr (kMode == kStored) {
+      cf[0][u] = st.ckj[u][lane];
+      cg[0][u] = st.ci[u][lane];
+    }
   }
   rounds(ca.rounds, [&](auto pc, int n) {
     constexpr int p = decltype(pc)::value, q = p & 1;
@@ -200,6 +233,10 @@ __device__ __forceinline__ void march(const Metric& m, const ColArgs& ca, const 
           ck = x.cp.k * cf[q][u].y;
           cj = x.cp.j * cf[q][u].x;
           ci = x.cp.i * cf[q][u].x;
+        } else if constexpr (kMode == kStored) {
+          ck = cf[q][u].x;
+          cj = cf[q][u].y;
+          ci = cg[q][u];
         } else if constexpr (kMode == kPhiCut) {
           ck = cf[q][u].y == 0.f ? 0.f : ck0;
         }
@@ -224,7 +261,11 @@ __device__ __forceinline__ void march(const Metric& m, const ColArgs& ca, const 
         nj[kJ - 1] = bperm(nbr, t);
         v[u * 64].x = y;
         rd[1 - q][u] = vn[u * 64];
-        if constexpr (kMode != kPhiUniform) cf[1 - q][u] = pn[u];
+        if constexpr (kTable) cf[1 - q][u] = pn[u];
+        if constexpr (kMode == kStored) {
+          cf[1 - q][u] = st.ckj[((p + 1) % kCP) * kCU + u][lane];
+          cg[1 - q][u] = st.ci[((p + 1) % kCP) * kCU + u][lane];
+        }
       }
     };
     if (s0 <= kDelay + q_first || s0 + kCU >= q_last)
@@ -311,8 +352,42 @@ __device__ __forceinline__ void col_lds_init(const ColArgs& ca, ColLds& sh, floa
                                              const float2* src, int lane) {
 #pragma unroll
   for (int t = 0; t < kRing; t++) sh.v[t][lane] = make_float2(0.f, 0.f);
-  if (ca.mode != kPhiUniform)
+  if (ca.mode == kPhiAny || ca.mode == kPhiCut)
     for (int q = lane; q < ca.pf_n; q += 64) pf[q] = src[q];
+}
+
+// Wave 2, forward: the march's results, to the next columns and to y_s.
+__device__ __forceinline__ void forward_out(const ColArgs& ca, const ColCtx& x, ColLds& sh) {
+  const int lane = x.lane;
+  u64* oi = ca.face_i + x.fbase + lane;
+  u64* oj = ca.face_j + x.fbase + lane;
+  float* ys = ca.y_s + x.sk;
+  const int fu = lane >> 3, fe = lane & 7;  // this lane's face row and entry
+  // chunk n - 1's results: the faces first, then the rows
+  auto out = [&](int n) {
+    const int b = ((n - 1) & 7) * kCU;
+    const float2 vi = sh.v[b + fu][7 + 8 * fe], vj = sh.v[b + fu][56 + fe];
+    float y[kCU];
+#pragma unroll
+    for (int u = 0; u < kCU; u++) y[u] = sh.v[b + u][lane].x;
+    word_store(oi + (size_t)n * (kCU * 8), vi.y * vi.x, x.stamp);
+    word_store(oj + (size_t)n * (kCU * 8), vj.y * vj.x, x.stamp);
+    float* yo = ys + (ptrdiff_t)(n - 1) * (kCU * 64);
+#pragma unroll
+    for (int u = 0; u < kCU; u++) yo[u * 64 + lane] = y[u];
+  };
+  lds_barrier();
+  rounds(ca.rounds, [&](auto, int n) {
+    out(n);
+    lds_barrier();
+  });
+  const int end = ca.rounds * kCP;
+  out(end);
+  // the rows that a reader's last steps ask for lie behind the grid
+  for (int n = end + 1; n <= end + (7 * kJ + kCU - 1) / kCU; n++) {
+    word_store(oi + (size_t)n * (kCU * 8), 0.f, x.stamp);
+    word_store(oj + (size_t)n * (kCU * 8), 0.f, x.stamp);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -399,35 +474,40 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
   } else if (x.wave == 3) {
     faces<true>(ca, x, sh);
   } else {
-    u64* oi = ca.face_i + x.fbase + lane;
-    u64* oj = ca.face_j + x.fbase + lane;
-    float* ys = ca.y_s + x.sk;
-    const int fu = lane >> 3, fe = lane & 7;  // this lane's face row and entry
-    // chunk n - 1's results: the faces first, then the rows
-    auto out = [&](int n) {
-      const int b = ((n - 1) & 7) * kCU;
-      const float2 vi = sh.v[b + fu][7 + 8 * fe], vj = sh.v[b + fu][56 + fe];
-      float y[kCU];
+    forward_out(ca, x, sh);
+  }
+}
+
+// Wave 2, backward: the march's results to the next columns, and the planes
+// that a chunk completes, k downwards (lane dl finished plane top - s at step
+// s - dl), to store(k, values); what lies outside the grid stays zero.
+template <typename F>
+__device__ __forceinline__ void backward_out(const ColArgs& ca, const ColCtx& x, ColLds& sh,
+                                             F&& store) {
+  const int lane = x.lane, top = ca.c + ca.skip + kDelay - 1;
+  u64* oi = ca.face_i + x.fbase + lane;
+  u64* oj = ca.face_j + x.fbase + lane;
+  const int fu = lane >> 3, fe = lane & 7;
+  auto out = [&](int n) {
+    const int b = ((n - 1) & 7) * kCU;
+    const float ti = sh.v[b + fu][8 * fe].x, tj = sh.v[b + fu][fe].x;
+    float y[kCU];
 #pragma unroll
-      for (int u = 0; u < kCU; u++) y[u] = sh.v[b + u][lane].x;
-      word_store(oi + (size_t)n * (kCU * 8), vi.y * vi.x, x.stamp);
-      word_store(oj + (size_t)n * (kCU * 8), vj.y * vj.x, x.stamp);
-      float* yo = ys + (ptrdiff_t)(n - 1) * (kCU * 64);
-#pragma unroll
-      for (int u = 0; u < kCU; u++) yo[u * 64 + lane] = y[u];
-    };
+    for (int u = 0; u < kCU; u++) y[u] = sh.v[(b + u - x.dl) & (kRing - 1)][lane].x;
+    word_store(oi + (size_t)n * (kCU * 8), ti, x.stamp);
+    word_store(oj + (size_t)n * (kCU * 8), tj, x.stamp);
+    store(top - (n - 1) * kCU, y);
+  };
+  lds_barrier();
+  rounds(ca.rounds, [&](auto, int n) {
+    out(n);
     lds_barrier();
-    rounds(ca.rounds, [&](auto, int n) {
-      out(n);
-      lds_barrier();
-    });
-    const int end = ca.rounds * kCP;
-    out(end);
-    // the rows that a reader's last steps ask for lie behind the grid
-    for (int n = end + 1; n <= end + (7 * kJ + kCU - 1) / kCU; n++) {
-      word_store(oi + (size_t)n * (kCU * 8), 0.f, x.stamp);
-      word_store(oj + (size_t)n * (kCU * 8), 0.f, x.stamp);
-    }
+  });
+  const int end = ca.rounds * kCP;
+  out(end);
+  for (int n = end + 1; n <= end + (7 * kJ + kCU - 1) / kCU; n++) {
+    word_store(oi + (size_t)n * (kCU * 8), 0.f, x.stamp);
+    word_store(oj + (size_t)n * (kCU * 8), 0.f, x.stamp);
   }
 }
 
@@ -465,8 +545,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     auto put = [&](auto pc, int n) {
       constexpr int p = decltype(pc)::value;
       float2* d = &sh.v[(n & 7) * kCU][lane];
+      // y_s outside the grid is whatever the march made of what it met there
+      // (a NaN, next to an overflow)
+      const int k0 = top - n * kCU - x.dl;
 #pragma unroll
-      for (int u = 0; u < kCU; u++) d[u * 64] = make_float2(yv[p][u], dv[p][u]);
+      for (int u = 0; u < kCU; u++)
+        d[u * 64] = make_float2(x.act && (unsigned)(k0 - u) < (unsigned)ca.c ? yv[p][u] : 0.f,
+                                dv[p][u]);
       load(p, n + kCP);
     };
     put(Phase<0>{}, 0);
@@ -487,37 +572,153 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
   } else if (x.wave == 3) {
     faces<false>(ca, x, sh);
   } else {
-    u64* oi = ca.face_i + x.fbase + lane;
-    u64* oj = ca.face_j + x.fbase + lane;
-    const int fu = lane >> 3, fe = lane & 7;
-    // chunk n - 1's results: its faces, and the planes that it completes, k
-    // downwards (lane dl finished plane top - s at step s - dl); what lies
-    // outside the grid stays zero
-    auto out = [&](int n) {
-      const int b = ((n - 1) & 7) * kCU, k = top - (n - 1) * kCU;
-      const float ti = sh.v[b + fu][8 * fe].x, tj = sh.v[b + fu][fe].x;
-      float y[kCU];
-#pragma unroll
-      for (int u = 0; u < kCU; u++) y[u] = sh.v[(b + u - x.dl) & (kRing - 1)][lane].x;
-      word_store(oi + (size_t)n * (kCU * 8), ti, x.stamp);
-      word_store(oj + (size_t)n * (kCU * 8), tj, x.stamp);
+    backward_out(ca, x, sh, [&](int k, const float* y) {
       const bool in = k >= 0 && k < ca.planes;
       T* zo = (in ? z : (T*)ca.dummy) + (in ? tm_row(ca, x.col, k - (kCU - 1)) : 0u);
 #pragma unroll
       for (int u = 0; u < kCU; u++)
         zo[(kCU - 1 - u) * 64 + lane] = (T)(x.act && k - u < ca.c ? y[u] : 0.f);
+    });
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The sweeps with stored couplings: x in natural order, solved in place.
+// lo_s and up_s hold {k, j, i coupling, dinv} by step of the direction's own
+// march.  The forward sweep keeps the right-hand side as it uses it (FP32,
+// natural order): what the tile schedule starts from when a wait runs out.
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+    k_col_fwd_stored(Grid3 g, ColArgs ca, const double* __restrict__ xv, float* __restrict__ r32) {
+  extern __shared__ char lds[];
+  ColLdsStored& sh = *(ColLdsStored*)lds;
+  Metric m{};
+  m.a = g.a;
+  const ColCtx x = col_ctx<true, true>(m, g, ca);
+  if (x.wave == 1) {
+    const int lane = x.lane, last = ca.rounds * kCP - 1;
+    const size_t base = x.act ? (size_t)(x.I * 8 + x.ii) + (size_t)g.a * (x.J * 8 + x.jj) : 0;
+    const float4* cs = ca.lo_s + (size_t)x.col * ca.rounds * (kCS * 64) + lane;
+    constexpr int kAP = 2;  // chunks of couplings in flight: registers
+    double rv[kCP][kCU];
+    float4 cv[kAP][kCU];
+    auto load = [&](int p, int n) {
+#pragma unroll
+      for (int u = 0; u < kCU; u++)
+        rv[p][u] = xv[base + (size_t)g.ab * (size_t)min(n * kCU + u, ca.c - 1)];
     };
+    auto load_c = [&](int p, int n) {
+      const float4* c = cs + (size_t)min(n, last) * (kCU * 64);
+#pragma unroll
+      for (int u = 0; u < kCU; u++) cv[p][u] = c[u * 64];
+    };
+#pragma unroll
+    for (int p = 0; p < kCP; p++) load(p, p);
+#pragma unroll
+    for (int p = 0; p < kAP; p++) load_c(p, p);
+    col_lds_init(ca, sh, nullptr, nullptr, lane);
+    auto put = [&](auto pc, int n) {
+      constexpr int p = decltype(pc)::value;
+      const int o = (n & 7) * kCU + x.dl;
+#pragma unroll
+      for (int u = 0; u < kCU; u++) {
+        const int k = n * kCU + u;
+        const bool in = x.act && k < ca.c;
+        const float v = in ? (float)rv[p][u] : 0.f;
+        sh.v[(o + u) & (kRing - 1)][lane].x = v;
+        if (in) r32[base + (size_t)g.ab * k] = v;
+        const float4 c = cv[p % kAP][u];
+        sh.v[(n & 7) * kCU + u][lane].y = c.w;
+        sh.ckj[p * kCU + u][lane] = make_float2(c.x, c.y);
+        sh.ci[p * kCU + u][lane] = c.z;
+      }
+      load_c(p % kAP, n + kAP);
+      load(p, n + kCP);
+    };
+    put(Phase<0>{}, 0);
+    put(Phase<1>{}, 1);
     lds_barrier();
-    rounds(ca.rounds, [&](auto, int n) {
-      out(n);
+    rounds(ca.rounds, [&](auto pc, int n) {
+      put(Phase<(decltype(pc)::value + 2) % kCP>{}, n + 2);
       lds_barrier();
     });
-    const int end = ca.rounds * kCP;
-    out(end);
-    for (int n = end + 1; n <= end + (7 * kJ + kCU - 1) / kCU; n++) {
-      word_store(oi + (size_t)n * (kCU * 8), 0.f, x.stamp);
-      word_store(oj + (size_t)n * (kCU * 8), 0.f, x.stamp);
-    }
+  } else if (x.wave == 0) {
+    // the backward sweep's stamp (no workgroup of this launch reads it)
+    if (blockIdx.x == 0 && x.lane == 0)
+      __hip_atomic_store(ca.ctr + 1, x.stamp + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    march<true, kStored>(m, ca, x, sh, nullptr);
+  } else if (x.wave == 3) {
+    faces<true>(ca, x, sh);
+  } else {
+    forward_out(ca, x, sh);
+  }
+}
+
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+    k_col_bwd_stored(Grid3 g, ColArgs ca, double* __restrict__ xv) {
+  extern __shared__ char lds[];
+  ColLdsStored& sh = *(ColLdsStored*)lds;
+  Metric m{};
+  m.a = g.a;
+  const ColCtx x = col_ctx<false, true>(m, g, ca);
+  const int top = ca.c + ca.skip + kDelay - 1;  // row of step 0
+  if (x.wave == 1) {
+    const int lane = x.lane, last = ca.rounds * kCP - 1;
+    const float4* cs = ca.up_s + (size_t)x.col * ca.rounds * (kCS * 64) + lane;
+    const float* ys = ca.y_s + x.sk + (size_t)top * 64 + lane;
+    constexpr int kAP = 2;
+    float yv[kCP][kCU];
+    float4 cv[kAP][kCU];
+    auto load = [&](int p, int n) {
+      const float* y = ys - (ptrdiff_t)min(n, last) * (kCU * 64);
+#pragma unroll
+      for (int u = 0; u < kCU; u++) yv[p][u] = y[-u * 64];
+    };
+    auto load_c = [&](int p, int n) {
+      const float4* c = cs + (size_t)min(n, last) * (kCU * 64);
+#pragma unroll
+      for (int u = 0; u < kCU; u++) cv[p][u] = c[u * 64];
+    };
+#pragma unroll
+    for (int p = 0; p < kCP; p++) load(p, p);
+#pragma unroll
+    for (int p = 0; p < kAP; p++) load_c(p, p);
+    col_lds_init(ca, sh, nullptr, nullptr, lane);
+    auto put = [&](auto pc, int n) {
+      constexpr int p = decltype(pc)::value;
+      const int k0 = top - n * kCU - x.dl;
+#pragma unroll
+      for (int u = 0; u < kCU; u++) {
+        const bool in = x.act && (unsigned)(k0 - u) < (unsigned)ca.c;
+        const float4 c = cv[p % kAP][u];
+        sh.v[(n & 7) * kCU + u][lane] = make_float2(in ? yv[p][u] : 0.f, c.w);
+        sh.ckj[p * kCU + u][lane] = make_float2(c.x, c.y);
+        sh.ci[p * kCU + u][lane] = c.z;
+      }
+      load_c(p % kAP, n + kAP);
+      load(p, n + kCP);
+    };
+    put(Phase<0>{}, 0);
+    put(Phase<1>{}, 1);
+    lds_barrier();
+    rounds(ca.rounds, [&](auto pc, int n) {
+      put(Phase<(decltype(pc)::value + 2) % kCP>{}, n + 2);
+      lds_barrier();
+    });
+  } else if (x.wave == 0) {
+    // the next forward sweep's stamp
+    if (blockIdx.x == 0 && x.lane == 0)
+      __hip_atomic_store(ca.ctr, x.stamp + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    march<false, kStored>(m, ca, x, sh, nullptr);
+  } else if (x.wave == 3) {
+    faces<false>(ca, x, sh);
+  } else {
+    const size_t base = x.act ? (size_t)(x.I * 8 + x.ii) + (size_t)g.a * (x.J * 8 + x.jj) : 0;
+    backward_out(ca, x, sh, [&](int k, const float* y) {
+#pragma unroll
+      for (int u = 0; u < kCU; u++)
+        if (x.act && (unsigned)(k - u) < (unsigned)ca.c)
+          xv[base + (size_t)g.ab * (size_t)(k - u)] = (double)y[u];
+    });
   }
 }
 
@@ -537,7 +738,32 @@ __global__ void k_col_gather(Grid3 g, int NI, int rows_alloc, size_t n,
                : 0.f;
 }
 
+// The couplings and dinv of one direction by step of its march: entry s of
+// column (I, J) belongs to the plane that lane (ii, jj) handles at step s,
+// zero where no point of the grid lies (and for what the point does not have).
+__global__ void k_col_gather_stored(Grid3 g, int NI, int steps, int top, size_t n,
+                                    const float* __restrict__ ck, const float* __restrict__ cj,
+                                    const float* __restrict__ ci, const float* __restrict__ dinv,
+                                    int fwd, float4* __restrict__ dst) {
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n) return;
+  const int lane = (int)(t & 63);
+  const size_t cr = t >> 6;
+  const int s = (int)(cr % (size_t)steps), col = (int)(cr / (size_t)steps);
+  const int i = (col % NI) * 8 + (lane & 7), j = (col / NI) * 8 + (lane >> 3);
+  const int dl = (lane & 7) + kJ * (lane >> 3), k = fwd ? s - dl : top - s - dl;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (i < g.a && j < g.b && k >= 0 && k < g.c) {
+    const size_t q = (size_t)i + (size_t)g.a * j + (size_t)g.ab * k;
+    v = make_float4((fwd ? k > 0 : k < g.c - 1) ? ck[q] : 0.f,
+                    (fwd ? j > 0 : j < g.b - 1) ? cj[q] : 0.f,
+                    (fwd ? i > 0 : i < g.a - 1) ? ci[q] : 0.f, dinv[q]);
+  }
+  dst[t] = v;
+}
+
 size_t col_lds(const ColArgs& ca) {
+  if (ca.mode == kStored) return sizeof(ColLdsStored);
   return sizeof(ColLds) + (ca.mode == kPhiUniform ? 0 : ca.pf_n * sizeof(float2));
 }
 
@@ -555,16 +781,17 @@ void launch_columns(const ColArgs& ca, const Metric& m, const Grid3& g, T* r, T*
 
 }  // namespace
 
-int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
-                      int tk_log2, const float* dinv) {
-  free_column_plan(plan);
+namespace {
+
+// What both kinds of plan share: the columns and steps of the grid, and the
+// device memory that does not depend on where the couplings come from.
+// Returns 0, or 1 when a buffer cannot be had (the caller frees the plan).
+int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int planes) {
   ColArgs& ca = plan.a;
   ca.NI = (g.a + 7) / 8;
   ca.NJ = (g.b + 7) / 8;
   ca.c = g.c;
-  ca.tk_log2 = tk_log2;
-  const int TK = 1 << tk_log2;
-  ca.planes = (g.c + TK - 1) / TK * TK;
+  ca.planes = planes;
   ca.bl = bl;
   ca.skip = (kCU - 1 - (g.c + kDelay - 1)) & (kCU - 1);
   ca.rounds = (g.c + ca.skip + kDelay + kCS - 1) / kCS;
@@ -572,21 +799,55 @@ int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const I
   ca.face_rows = (ca.rounds * kCP + kCP + 6) * kCU;  // from chunk -1 on
   ca.pf_n = ca.rounds * kCS + kCU + kDelay;
   const int ncol = ca.NI * ca.NJ;
-  if ((uint64_t)ncol * ca.planes * 64 >= (1ull << 32)) return 1;
   const size_t nsk = (size_t)ncol * ca.rows_alloc * 64, nf = (size_t)ncol * ca.face_rows * 8;
   // columns by anti-diagonal inside their block (blocks are independent)
   const int bI = bl.bi < g.a ? bl.bi / 8 : ca.NI, bJ = bl.bj < g.b ? bl.bj / 8 : ca.NJ;
-  if ((bl.bi < g.a && bl.bi % 8) || (bl.bj < g.b && bl.bj % 8)) return 2;
   std::vector<int> order;
   order.reserve(ncol);
   for (int L = 0; L <= bI + bJ - 2; L++)
     for (int J = 0; J < ca.NJ; J++)
       for (int I = 0; I < ca.NI; I++)
         if (I % bI + J % bJ == L) order.push_back(I + ca.NI * J);
+  const unsigned ctr[4] = {1u, 2u, 0u, 0u};
+  const bool ok =
+      hipMalloc((void**)&plan.order, ncol * sizeof(int)) == hipSuccess &&
+      hipMalloc((void**)&plan.y_s, nsk * sizeof(float)) == hipSuccess &&
+      hipMalloc((void**)&plan.face, 2 * nf * sizeof(u64)) == hipSuccess &&
+      hipMalloc((void**)&plan.ctr, sizeof ctr) == hipSuccess &&
+      hipMalloc((void**)&plan.dummy, kCU * 64 * sizeof(double)) == hipSuccess &&
+      hipMemset(plan.y_s, 0, nsk * sizeof(float)) == hipSuccess &&
+      hipMemset(plan.face, 0, 2 * nf * sizeof(u64)) == hipSuccess &&
+      hipMemcpy(plan.order, order.data(), ncol * sizeof(int), hipMemcpyHostToDevice) ==
+          hipSuccess &&
+      hipMemcpy(plan.ctr, ctr, sizeof ctr, hipMemcpyHostToDevice) == hipSuccess;
+  ca.order = plan.order;
+  ca.y_s = plan.y_s;
+  ca.face_i = plan.face;
+  ca.face_j = plan.face + nf;
+  ca.ctr = plan.ctr;
+  ca.dummy = plan.dummy;
+  return ok ? 0 : 1;
+}
+
+int no_plan(ColumnPlan& plan) {
+  free_column_plan(plan);
+  (void)hipGetLastError();  // a failed allocation: the tile schedules run
+  return 1;
+}
+
+}  // namespace
+
+int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
+                      int tk_log2, const float* dinv) {
+  free_column_plan(plan);
+  ColArgs& ca = plan.a;
+  ca.tk_log2 = tk_log2;
+  const int TK = 1 << tk_log2, planes = (g.c + TK - 1) / TK * TK;
+  if ((uint64_t)((g.a + 7) / 8) * ((g.b + 7) / 8) * planes * 64 >= (1ull << 32)) return 1;
+  if ((bl.bi < g.a && bl.bi % 8) || (bl.bj < g.b && bl.bj % 8)) return 2;
   // phi factors by plane, zero outside the grid; a coupling that the
   // block-Jacobi cut drops has a zero factor
   std::vector<float> dph(g.c), dpl(g.c), dpu(g.c);
-  std::vector<float2> lo(ca.pf_n, make_float2(0.f, 0.f)), up(lo);
   if (hipMemcpy(dph.data(), m.FDPH, g.c * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess ||
       hipMemcpy(dpl.data(), m.FDPL, g.c * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess ||
       hipMemcpy(dpu.data(), m.FDPU, g.c * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
@@ -599,54 +860,62 @@ int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const I
   ca.mode = !uniform ? kPhiAny : (bl.bk < g.c ? kPhiCut : kPhiUniform);
   ca.u_d = dph[0];
   ca.u_k = dpl[0];
-  if (col_lds(ca) > kColLdsMax) return 1;
+  if (plan_columns(plan, g, bl, planes) != 0) return no_plan(plan);
+  if (col_lds(ca) > kColLdsMax) return no_plan(plan);
+  std::vector<float2> lo(ca.pf_n, make_float2(0.f, 0.f)), up(lo);
   for (int k = 0; k < g.c; k++) {
     lo[kDelay + k] = make_float2(dph[k], k > 0 && k % bl.bk ? dpl[k] : 0.f);
-    up[kDelay + ca.skip + g.c - 1 - k] = make_float2(dph[k], k < g.c - 1 && (k + 1) % bl.bk ? dpu[k] : 0.f);
+    up[kDelay + ca.skip + g.c - 1 - k] =
+        make_float2(dph[k], k < g.c - 1 && (k + 1) % bl.bk ? dpu[k] : 0.f);
   }
-  const unsigned ctr[4] = {1u, 2u, 0u, 0u};
-  bool ok = hipMalloc((void**)&plan.order, ncol * sizeof(int)) == hipSuccess &&
-            hipMalloc((void**)&plan.dinv_s, nsk * sizeof(float)) == hipSuccess &&
-            hipMalloc((void**)&plan.y_s, nsk * sizeof(float)) == hipSuccess &&
-            hipMalloc((void**)&plan.face, 2 * nf * sizeof(u64)) == hipSuccess &&
-            hipMalloc((void**)&plan.pf, 2 * ca.pf_n * sizeof(float2)) == hipSuccess &&
-            hipMalloc((void**)&plan.ctr, sizeof ctr) == hipSuccess &&
-            hipMalloc((void**)&plan.dummy, kCU * 64 * sizeof(double)) == hipSuccess;
-  if (ok) {
-    k_col_gather<<<(unsigned)((nsk + 255) / 256), 256>>>(g, ca.NI, ca.rows_alloc, nsk, dinv,
-                                                         plan.dinv_s);
-    ok = hipGetLastError() == hipSuccess &&
-         hipMemset(plan.y_s, 0, nsk * sizeof(float)) == hipSuccess &&
-         hipMemset(plan.face, 0, 2 * nf * sizeof(u64)) == hipSuccess &&
-         hipMemcpy(plan.order, order.data(), ncol * sizeof(int), hipMemcpyHostToDevice) ==
-             hipSuccess &&
-         hipMemcpy(plan.pf, lo.data(), ca.pf_n * sizeof(float2), hipMemcpyHostToDevice) ==
-             hipSuccess &&
-         hipMemcpy(plan.pf + ca.pf_n, up.data(), ca.pf_n * sizeof(float2),
-                   hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(plan.ctr, ctr, sizeof ctr, hipMemcpyHostToDevice) == hipSuccess &&
-         hipDeviceSynchronize() == hipSuccess;
-  }
-  if (!ok) {
-    free_column_plan(plan);
-    (void)hipGetLastError();  // a failed allocation: the tile schedules run
-    return 1;
-  }
-  ca.order = plan.order;
+  const size_t nsk = (size_t)ca.NI * ca.NJ * ca.rows_alloc * 64;
+  if (hipMalloc((void**)&plan.dinv_s, nsk * sizeof(float)) != hipSuccess ||
+      hipMalloc((void**)&plan.pf, 2 * ca.pf_n * sizeof(float2)) != hipSuccess)
+    return no_plan(plan);
+  k_col_gather<<<(unsigned)((nsk + 255) / 256), 256>>>(g, ca.NI, ca.rows_alloc, nsk, dinv,
+                                                       plan.dinv_s);
+  if (hipGetLastError() != hipSuccess ||
+      hipMemcpy(plan.pf, lo.data(), ca.pf_n * sizeof(float2), hipMemcpyHostToDevice) !=
+          hipSuccess ||
+      hipMemcpy(plan.pf + ca.pf_n, up.data(), ca.pf_n * sizeof(float2), hipMemcpyHostToDevice) !=
+          hipSuccess ||
+      hipDeviceSynchronize() != hipSuccess)
+    return no_plan(plan);
   ca.dinv_s = plan.dinv_s;
-  ca.y_s = plan.y_s;
-  ca.face_i = plan.face;
-  ca.face_j = plan.face + nf;
   ca.pf_lo = plan.pf;
   ca.pf_up = plan.pf + ca.pf_n;
-  ca.ctr = plan.ctr;
-  ca.dummy = plan.dummy;
+  plan.ready = 1;
+  return 0;
+}
+
+int build_column_plan_stored(ColumnPlan& plan, const Grid3& g, const CoefArrays& co, bool wrap,
+                             const float* dinv) {
+  free_column_plan(plan);
+  ColArgs& ca = plan.a;
+  ca.mode = kStored;
+  if (plan_columns(plan, g, IluBlocks{g.a, g.b, g.c, wrap ? 1 : 0}, g.c) != 0)
+    return no_plan(plan);
+  const int steps = ca.rounds * kCS;
+  const size_t n = (size_t)ca.NI * ca.NJ * steps * 64;
+  if (hipMalloc((void**)&plan.cs, 2 * n * sizeof(float4)) != hipSuccess) return no_plan(plan);
+  const int top = ca.c + ca.skip + kDelay - 1;
+  const unsigned nb = (unsigned)((n + 255) / 256);
+  k_col_gather_stored<<<nb, 256>>>(g, ca.NI, steps, top, n, co.lo_k, co.lo_j, co.lo_i, dinv, 1,
+                                   plan.cs);
+  k_col_gather_stored<<<nb, 256>>>(g, ca.NI, steps, top, n, co.up_k, co.up_j, co.up_i, dinv, 0,
+                                   plan.cs + n);
+  if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+    return no_plan(plan);
+  ca.lo_s = plan.cs;
+  ca.up_s = plan.cs + n;
+  ca.wrap_lo = co.wrap_lo;
+  ca.wrap_up = co.wrap_up;
   plan.ready = 1;
   return 0;
 }
 
 void free_column_plan(ColumnPlan& plan) {
-  void* bufs[] = {plan.order, plan.dinv_s, plan.y_s, plan.face, plan.pf, plan.ctr, plan.dummy};
+  void* bufs[] = {plan.order, plan.dinv_s, plan.y_s, plan.face, plan.pf, plan.ctr, plan.dummy, plan.cs};
   for (void* b : bufs)
     if (b) hipFree(b);
   plan = ColumnPlan();
@@ -662,6 +931,14 @@ void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g
     launch_columns<T, kPhiCut>(ca, m, g, r, z, guard, ap, s);
   else
     launch_columns<T, kPhiAny>(ca, m, g, r, z, guard, ap, s);
+}
+
+void launch_dilu_columns_stored(const ColumnPlan& plan, const Grid3& g, double* x, float* r32,
+                                hipStream_t s) {
+  const ColArgs& ca = plan.a;
+  const int nb = ca.NI * ca.NJ;
+  k_col_fwd_stored<<<nb, kThreads, sizeof(ColLdsStored), s>>>(g, ca, x, r32);
+  k_col_bwd_stored<<<nb, kThreads, sizeof(ColLdsStored), s>>>(g, ca, x);
 }
 
 const unsigned* column_failure_flag(const ColumnPlan& plan) { return plan.ctr + 2; }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "p3d_internal.hpp"
+#include "p3d_kernels.hpp"
 
 namespace p3d {
 
@@ -27,6 +28,10 @@ struct ColArgs {
   unsigned long long* face_j = nullptr;
   const float2* pf_lo = nullptr;  // (FDPH, FDPL) by plane + 21, zero outside
   const float2* pf_up = nullptr;  // (FDPH, FDPU) from plane c + skip - 1 downwards, likewise
+  // stored couplings: {k, j, i, dinv} by step and lane of the forward and the
+  // backward march, and those of the phi wrap (a x b)
+  const float4 *lo_s = nullptr, *up_s = nullptr;
+  const float *wrap_lo = nullptr, *wrap_up = nullptr;
   unsigned* ctr = nullptr;        // stamps of the next forward, backward sweep; failure flag
   void* dummy = nullptr;          // where rows outside the vectors are stored
 };
@@ -40,12 +45,16 @@ struct ColumnPlan {
   float2* pf = nullptr;
   unsigned* ctr = nullptr;
   void* dummy = nullptr;
+  float4* cs = nullptr;  // stored couplings, forward then backward
 };
 
 // dinv: the D-ILU's inverse pivots in natural order; tk_log2: planes per
 // tile of the r and z placement.  Returns 0 when the sweeps can run.
 int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
                       int tk_log2, const float* dinv);
+// The same with stored couplings; co's wrap planes have to outlive the plan.
+int build_column_plan_stored(ColumnPlan& plan, const Grid3& g, const CoefArrays& co, bool wrap,
+                             const float* dinv);
 void free_column_plan(ColumnPlan& plan);
 
 // z = (LU)^-1 r on tile-major r and z, two launches.  ap (tile-major, with
@@ -53,6 +62,11 @@ void free_column_plan(ColumnPlan& plan);
 template <typename T>
 void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g, T* r, T* z,
                          const CgState* guard, const T* ap, hipStream_t s);
+
+// x = (LU)^-1 x on natural order, stored couplings, two launches.  r32 (N
+// floats) receives x as it was, rounded to FP32 as the sweep uses it.
+void launch_dilu_columns_stored(const ColumnPlan& plan, const Grid3& g, double* x, float* r32,
+                                hipStream_t s);
 
 // Device word that is not 0 once a wait of a column sweep ran into its bound.
 const unsigned* column_failure_flag(const ColumnPlan& plan);
