@@ -122,23 +122,25 @@ static void forward(p3d_nn* n) {
   auto W = [&](int i) { return n->wb + n->conv[i].w_off; };
   auto B = [&](int i) { return n->w + n->conv[i].b_off; };
   const Dims3* D = n->D;
-  conv_fwd(D[0], 16, 16, n->x0, W(0), B(0), n->e0, nullptr, true, s);
+  auto layer = [&](int i, const uint16_t* x, uint16_t* y, const uint16_t* e = nullptr,
+                   uint16_t* sum = nullptr) {
+    const ConvSpec& c = n->conv[i];
+    conv_relu(D[c.level], c.Cin, c.Cout, x, W(i), B(i), y, e, sum, s);
+  };
+  layer(0, n->x0, n->e0);
   pool_fwd(D[0], D[1], 16, n->e0, n->p1, s);
-  conv_fwd(D[1], 16, 32, n->p1, W(1), B(1), n->e1, nullptr, true, s);
+  layer(1, n->p1, n->e1);
   pool_fwd(D[1], D[2], 32, n->e1, n->p2, s);
-  conv_fwd(D[2], 32, 64, n->p2, W(2), B(2), n->e2, nullptr, true, s);
+  layer(2, n->p2, n->e2);
   pool_fwd(D[2], D[3], 64, n->e2, n->p3, s);
-  conv_fwd(D[3], 64, 128, n->p3, W(3), B(3), n->e3, nullptr, true, s);
+  layer(3, n->p3, n->e3);
   up_fwd(D[3], D[2], 128, n->e3, n->u2, s);
-  conv_fwd(D[2], 128, 64, n->u2, W(4), B(4), n->d2, nullptr, true, s);
-  add_bf16(D[2].V() * 64, n->d2, n->e2, n->s2, s);
+  layer(4, n->u2, n->d2, n->e2, n->s2);
   up_fwd(D[2], D[1], 64, n->s2, n->u1, s);
-  conv_fwd(D[1], 64, 32, n->u1, W(5), B(5), n->d1, nullptr, true, s);
-  add_bf16(D[1].V() * 32, n->d1, n->e1, n->s1, s);
+  layer(5, n->u1, n->d1, n->e1, n->s1);
   up_fwd(D[1], D[0], 32, n->s1, n->u0, s);
-  conv_fwd(D[0], 32, 16, n->u0, W(6), B(6), n->d0, nullptr, true, s);
-  add_bf16(D[0].V() * 16, n->d0, n->e0, n->s0, s);
-  conv_fwd(D[0], 16, 16, n->s0, W(7), B(7), nullptr, n->out, false, s);
+  layer(6, n->u0, n->d0, n->e0, n->s0);
+  conv_head(D[0], 16, 16, n->s0, W(7), B(7), n->out, s);
 }
 
 static int nchunk_for(const Dims3& d) {
@@ -281,15 +283,18 @@ int p3d_nn_create(p3d_nn** out, int nr, int nt, int np, const double* rh, unsign
               {&n->u2, V2 * 128}, {&n->d2, V2 * 64}, {&n->s2, V2 * 64}, {&n->u1, V1 * 64},
               {&n->d1, V1 * 32}, {&n->s1, V1 * 32}, {&n->u0, V0 * 32}, {&n->d0, V0 * 16},
               {&n->s0, V0 * 16}};
-  for (auto& a : acts)
-    if ((rc = dmalloc(n, (void**)a.p, a.n * 2))) {
+  for (auto& a : acts) {
+    if ((rc = dmalloc(n, (void**)a.p, kZeroFront + a.n * 2))) {
       p3d_nn_destroy(n);
       return rc;
     }
+    hipMemset(*a.p, 0, kZeroFront);
+    *a.p += kZeroFront / 2;
+  }
   struct {
     float** p;
     size_t n;
-  } grads[] = {{&n->out, V0 * 16},   {&n->g_out, V0 * 16}, {&n->g_s0, V0 * 16},
+  } grads[] = {{&n->out, V0},        {&n->g_out, V0 * 16}, {&n->g_s0, V0 * 16},
                {&n->g_t0, V0 * 16},  {&n->g_u0, V0 * 32},  {&n->g_s1, V1 * 32},
                {&n->g_t1, V1 * 32},  {&n->g_u1, V1 * 64},  {&n->g_s2, V2 * 64},
                {&n->g_t2, V2 * 64},  {&n->g_u2, V2 * 128}, {&n->g_e3, V3 * 128},
@@ -477,7 +482,7 @@ int p3d_nn_predict(p3d_nn* n, const double* br0, double* x, double* x_dev) {
     if (hipMalloc((void**)&tmp, V * 8) != hipSuccess) return nfail(P3D_ENOMEM, "allocation failed");
     dst = tmp;
   }
-  head_to_x((int)V, 16, n->out, target_scale(n, bs), dst, n->stream);
+  head_to_x((int)V, n->out, target_scale(n, bs), dst, n->stream);
   if (x) hipMemcpyAsync(x, dst, V * 8, hipMemcpyDeviceToHost, n->stream);
   hipError_t e = hipStreamSynchronize(n->stream);
   if (tmp) hipFree(tmp);

@@ -12,8 +12,16 @@ struct Dims3 {
   size_t V() const { return (size_t)X * Y * Z; }
 };
 
-void conv_fwd(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
-              const float* bias, uint16_t* y, float* yf, bool relu, hipStream_t s);
+// Zero bytes in front of every BF16 tensor that a convolution reads (one
+// voxel's channels at most).
+constexpr size_t kZeroFront = 256;
+
+// y = relu(conv x + bias); with e also sum = y + e (the skip connection)
+void conv_relu(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
+               const float* bias, uint16_t* y, const uint16_t* e, uint16_t* sum, hipStream_t s);
+// y1[v] = channel 0 of conv x + bias (FP32)
+void conv_head(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
+               const float* bias, float* y1, hipStream_t s);
 // dx may be null; gw (27*Cout*Cin), gb (Cout) FP32; part: scratch of
 // nchunk*27*Cout*Cin floats.
 void conv_bwd(const Dims3& d, int Cin, int Cout, const float* dy, const uint16_t* x,
@@ -25,7 +33,6 @@ void pool_bwd(const Dims3& f, const Dims3& c, int C, const float* dy, float* dx,
 void up_fwd(const Dims3& c, const Dims3& f, int C, const uint16_t* x, uint16_t* y,
             hipStream_t s);
 void up_bwd(const Dims3& c, const Dims3& f, int C, const float* dy, float* dx, hipStream_t s);
-void add_bf16(size_t n, const uint16_t* a, const uint16_t* b, uint16_t* y, hipStream_t s);
 void relu_bwd(size_t n, const uint16_t* y, const float* g, const float* g2, float* out,
               hipStream_t s);
 void mse(int V, int C, const float* out, const float* tgt, float* g, float* part, float* loss,
@@ -41,7 +48,7 @@ void features(const Dims3& d, int C, int nt, const double* br0, const float* dec
               hipStream_t s);
 void gather_target(const Dims3& d, int roll, int flip, float sign, const float* src, float* dst,
                    hipStream_t s);
-void head_to_x(int V, int C, const float* out, double scale, double* xo, hipStream_t s);
+void head_to_x(int V, const float* out, double scale, double* xo, hipStream_t s);
 void prolong(int af, int bf, int cf, int nrc, int ntc, int npc, const double* phic,
              const int* ir, const double* wr, const int* it, const double* wt, const int* ip,
              const double* wp, double* xf, hipStream_t s);

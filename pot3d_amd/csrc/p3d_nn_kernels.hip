@@ -1,5 +1,5 @@
 // Kernels of the warm-start network: 3x3x3 convolutions as implicit GEMMs
-// on the gfx950 matrix cores (v_mfma_f32_16x16x16_bf16: BF16 operands,
+// on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16: BF16 operands,
 // FP32 accumulation), average pooling, nearest upsampling, skip additions,
 // ReLU, the MSE loss and Adam.
 //
@@ -9,11 +9,14 @@
 // are kept in FP32 (Adam state) with a BF16 copy [tap][c_out][c_in] for the
 // matrix cores.  The z axis (phi) is periodic, x and y are zero-padded.
 //
-// MFMA 16x16x16 operand layout (lane l of a wave64):
-//   A (16 x 16, M x K): lane holds A[l%16][4*(l/16) .. 4*(l/16)+3]
-//   B (16 x 16, K x N): lane holds B[4*(l/16) .. 4*(l/16)+3][l%16]
-//   D (16 x 16, M x N): lane holds D[4*(l/16) .. 4*(l/16)+3][l%16]
-// (checked on the device against a host matmul by p3d_nn_mfma_check).
+// MFMA 16x16x32 operand layout (lane l of a wave64): A row l%16 and B column
+// l%16, each with the eight k of group l/16 (the order of the k does not
+// matter as long as A and B agree); D (16 x 16): lane holds D[4*(l/16) ..
+// 4*(l/16)+3][l%16].  p3d_nn_mfma_check compares the 16x16x16 form, whose
+// groups hold four k, with a host matmul.
+//
+// Every BF16 tensor is preceded by kZeroFront zero bytes (the allocation's
+// first ones): a tap that falls outside the grid reads those.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -23,6 +26,8 @@ namespace p3d {
 namespace nn {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {
@@ -36,6 +41,17 @@ __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint
 __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
+
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ unsigned pack2(float lo, float hi) {
+  return (unsigned)f2bf(lo) | ((unsigned)f2bf(hi) << 16);
+}
+// the two BF16 values of a word
+__device__ __forceinline__ float lo2f(unsigned w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float hi2f(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
 
 struct Dims {
   int X, Y, Z;
@@ -62,42 +78,161 @@ __device__ __forceinline__ void coords(const Dims& d, int v, int& x, int& y, int
 
 // ---------------------------------------------------------------------------
 // y[v][co] = act( sum_t sum_ci x[nb(v,t)][ci] w[t][co][ci] + bias[co] )
-// grid (ceil(V/64), Cout/16), block 256: each wave computes 16 voxels x 16
-// output channels.
+// One wave: MT x 16 voxels times NB x 16 output channels; grid (voxels / (64
+// MT), Cout / (16 NB)), block 256.  The weights are the MFMA's A operand and
+// the voxels its B operand, so a lane ends with four channels of one voxel.
+// K runs over 32 channels of a tap; with 16 channels over two taps at a time
+// (lanes 0-31 the even, 32-63 the odd one; the 28th tap is empty).
+//
+// What bounds it: the voxel operand, 16 bytes a lane read from L1/L2 once per
+// tap and 32 channels (27 times the tensor), and the index arithmetic before
+// it.  MT tiles share a weight fragment and give the loads of one step
+// something to overlap with.  The eight convolutions of a forward pass at
+// 51x91x181: 1123 us with one 16 x 16 tile a wave and 8-byte operands, 394 us
+// so.
+struct ConvOut {
+  uint16_t* y;        // BF16 result (after the ReLU), or null
+  const uint16_t* e;  // BF16 skip input, or null
+  uint16_t* s;        // with e: the BF16 sum y + e
+  float* yf;          // FP32 result, all channels, or null
+  float* y1;          // FP32 result, channel 0 alone, or null
+  const float* bias;  // or null
+  int relu;
+};
+
+template <int CIN, int NB, int MT>
 __global__ void __launch_bounds__(256)
-    k_conv_fwd(Dims d, int Cin, int Cout, const uint16_t* __restrict__ x,
-               const uint16_t* __restrict__ w, const float* __restrict__ bias,
-               uint16_t* __restrict__ y, float* __restrict__ yf, int relu) {
+    k_conv(Dims d, int Cout, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+           ConvOut o) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int v0 = (blockIdx.x * 4 + wave) * 16;
-  const int co0 = blockIdx.y * 16;
-  const int m = lane & 15, kb = lane >> 4;
-  const int v = v0 + m;
-  int vx = 0, vy = 0, vz = 0;
-  const bool valid = v < d.V;
-  if (valid) coords(d, v, vx, vy, vz);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int ncb = Cin / 16;
-  for (int t = 0; t < 27; t++) {
-    const int vn = valid ? neighbour(d, vx, vy, vz, t, 1) : -1;
-    const uint16_t* wt = w + ((size_t)t * Cout + co0 + m) * Cin + 4 * kb;
-    for (int cb = 0; cb < ncb; cb++) {
-      bf16x4 a = {0, 0, 0, 0};
-      if (vn >= 0) a = *(const bf16x4*)(x + (size_t)vn * Cin + cb * 16 + 4 * kb);
-      const bf16x4 b = *(const bf16x4*)(wt + cb * 16);
-      acc = mfma16(a, b, acc);
+  const int m = lane & 15, kb = lane >> 4, h = kb >> 1;
+  // a contiguous range of voxels per XCD (workgroups go round the 8 XCDs):
+  // a tensor's neighbouring planes then meet in one L2
+  const int per = (int)gridDim.x / 8;
+  const int blk = (int)blockIdx.x < 8 * per
+                      ? ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3)
+                      : (int)blockIdx.x;
+  const int v0 = (blk * 4 + wave) * (16 * MT);
+  const int co0 = blockIdx.y * (16 * NB);
+  constexpr unsigned kQ = CIN / 8;  // 16-byte words of a voxel
+  const u32x4* xq = (const u32x4*)x - kZeroFront / 16;
+  const unsigned lane_q = kZeroFront / 16 + (CIN == 16 ? (unsigned)(kb & 1) : (unsigned)kb);
+  const unsigned XQ = kQ * (unsigned)d.X, PQ = kQ * (unsigned)d.X * (unsigned)d.Y;
+  unsigned base[MT], zlo[MT], zhi[MT];
+  bool in[MT], xm[MT], xp[MT], ym[MT], yp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; t++) {
+    const int v = v0 + t * 16 + m;
+    int vx = 0, vy = 0, vz = 0;
+    in[t] = v < d.V;
+    if (in[t]) coords(d, v, vx, vy, vz);
+    base[t] = lane_q + kQ * (unsigned)(in[t] ? v : 0);
+    zlo[t] = vz > 0 ? 0u - PQ : PQ * (unsigned)(d.Z - 1);
+    zhi[t] = vz < d.Z - 1 ? PQ : 0u - PQ * (unsigned)(d.Z - 1);
+    xm[t] = in[t] && vx > 0;
+    xp[t] = in[t] && vx < d.X - 1;
+    ym[t] = vy > 0;
+    yp[t] = vy < d.Y - 1;
+  }
+  // index and validity of tap t (a constant) for tile q
+  auto tap_ok = [&](int q, int t) {
+    const int dx = t % 3, dy = (t / 3) % 3;
+    const bool vx = dx == 0 ? xm[q] : (dx == 2 ? xp[q] : in[q]);
+    return t < 27 && vx && (dy == 0 ? ym[q] : (dy == 2 ? yp[q] : true));
+  };
+  auto tap_off = [&](int q, int t) {
+    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9;
+    return (unsigned)(dx * (int)kQ) + (unsigned)dy * XQ +
+           (dz == 0 ? zlo[q] : (dz == 2 ? zhi[q] : 0u));
+  };
+  f32x4 acc[NB][MT];
+#pragma unroll
+  for (int n = 0; n < NB; n++)
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[n][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  if constexpr (CIN == 16) {
+    const u32x4* wq = (const u32x4*)w + (size_t)(co0 + m) * kQ + (kb & 1);
+    const size_t wt = (size_t)Cout * kQ;
+#pragma unroll
+    for (int s = 0; s < 14; s++) {
+      u32x4 av[NB], bv[MT];
+#pragma unroll
+      for (int n = 0; n < NB; n++) {
+        const u32x4* p = wq + (size_t)n * 16 * kQ;
+        av[n] = p[wt * (size_t)(h && s < 13 ? 2 * s + 1 : 2 * s)];
+        if (s == 13 && h) av[n] = zero;
+      }
+#pragma unroll
+      for (int t = 0; t < MT; t++) {
+        const bool ok = h ? tap_ok(t, 2 * s + 1) : tap_ok(t, 2 * s);
+        const unsigned off = h ? tap_off(t, 2 * s + 1) : tap_off(t, 2 * s);
+        bv[t] = xq[ok ? base[t] + off : lane_q - kZeroFront / 16];
+      }
+#pragma unroll
+      for (int n = 0; n < NB; n++)
+#pragma unroll
+        for (int t = 0; t < MT; t++) acc[n][t] = mfma32(av[n], bv[t], acc[n][t]);
+    }
+  } else {
+    const u32x4* wq = (const u32x4*)w + (size_t)(co0 + m) * kQ + kb;
+    const size_t wt = (size_t)Cout * kQ;
+#pragma unroll 1
+    for (int dz = 0; dz < 3; dz++) {
+      unsigned bz[MT];
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+        bz[t] = base[t] + (dz == 0 ? zlo[t] : (dz == 2 ? zhi[t] : 0u));
+      const u32x4* wz = wq + wt * (size_t)(9 * dz);
+#pragma unroll
+      for (int r = 0; r < 9; r++) {
+        unsigned idx[MT];
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+          idx[t] = tap_ok(t, r) ? bz[t] + (unsigned)((r % 3 - 1) * (int)kQ) +
+                                      (unsigned)(r / 3 - 1) * XQ
+                                : lane_q - kZeroFront / 16;
+#pragma unroll
+        for (int c = 0; c < CIN / 32; c++) {
+          u32x4 av[NB], bv[MT];
+#pragma unroll
+          for (int n = 0; n < NB; n++) av[n] = wz[wt * (size_t)r + (size_t)n * 16 * kQ + 4 * c];
+#pragma unroll
+          for (int t = 0; t < MT; t++) bv[t] = xq[idx[t] + 4u * c];
+#pragma unroll
+          for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[n][t] = mfma32(av[n], bv[t], acc[n][t]);
+        }
+      }
     }
   }
-  const int co = co0 + m;
-  const float bv = bias ? bias[co] : 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int vo = v0 + 4 * kb + i;
-    if (vo < d.V) {
-      float val = acc[i] + bv;
-      if (relu && val < 0.f) val = 0.f;
-      if (y) y[(size_t)vo * Cout + co] = f2bf(val);
-      if (yf) yf[(size_t)vo * Cout + co] = val;
+  for (int n = 0; n < NB; n++) {
+    const int co = co0 + n * 16 + 4 * kb;
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+    if (o.bias) bias = *(const f32x4*)(o.bias + co);
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      const int v = v0 + t * 16 + m;
+      if (v >= d.V) continue;
+      f32x4 r = acc[n][t] + bias;
+      if (o.relu)
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = r[i] < 0.f ? 0.f : r[i];
+      const size_t at = (size_t)v * Cout + co;
+      if (o.y) {
+        const uint2 y = make_uint2(pack2(r[0], r[1]), pack2(r[2], r[3]));
+        *(uint2*)(o.y + at) = y;
+        if (o.e) {
+          const uint2 e = *(const uint2*)(o.e + at);
+          *(uint2*)(o.s + at) =
+              make_uint2(pack2(lo2f(y.x) + lo2f(e.x), hi2f(y.x) + hi2f(e.x)),
+                         pack2(lo2f(y.y) + lo2f(e.y), hi2f(y.y) + hi2f(e.y)));
+        }
+      }
+      if (o.yf) *(f32x4*)(o.yf + at) = r;
+      if (o.y1 && co == 0) o.y1[v] = r[0];
     }
   }
 }
@@ -212,25 +347,36 @@ __device__ __forceinline__ int child_count(const Dims& f, int px, int py, int pz
   return nx * ny * nz;
 }
 
+// (both forward kernels: one thread per voxel and 8 channels)
 __global__ void k_pool_fwd(Dims f, Dims c, int C, const uint16_t* __restrict__ x,
                            uint16_t* __restrict__ y) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)c.V * C) return;
-  const int ch = (int)(e % C), v = (int)(e / C);
+  const int Q = C / 8;
+  if (e >= (size_t)c.V * Q) return;
+  const int q = (int)(e % Q), v = (int)(e / Q);
   int px, py, pz;
   coords(c, v, px, py, pz);
-  float s = 0.f;
+  float s[8] = {};
   int n = 0;
   for (int dz = 0; dz < 2; dz++)
     for (int dy = 0; dy < 2; dy++)
       for (int dx = 0; dx < 2; dx++) {
         const int X = 2 * px + dx, Y = 2 * py + dy, Z = 2 * pz + dz;
         if (X < f.X && Y < f.Y && Z < f.Z) {
-          s += bf2f(x[((size_t)X + f.X * (Y + (size_t)f.Y * Z)) * C + ch]);
+          const u32x4 w = ((const u32x4*)x)[((size_t)X + f.X * (Y + (size_t)f.Y * Z)) * Q + q];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            s[2 * i] += lo2f(w[i]);
+            s[2 * i + 1] += hi2f(w[i]);
+          }
           n++;
         }
       }
-  y[e] = f2bf(s / (float)n);
+  const float fn = (float)n;
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; i++) o[i] = pack2(s[2 * i] / fn, s[2 * i + 1] / fn);
+  ((u32x4*)y)[e] = o;
 }
 
 __global__ void k_pool_bwd(Dims f, Dims c, int C, const float* __restrict__ dy,
@@ -248,11 +394,13 @@ __global__ void k_pool_bwd(Dims f, Dims c, int C, const float* __restrict__ dy,
 __global__ void k_up_fwd(Dims c, Dims f, int C, const uint16_t* __restrict__ x,
                          uint16_t* __restrict__ y) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)f.V * C) return;
-  const int ch = (int)(e % C), v = (int)(e / C);
+  const int Q = C / 8;
+  if (e >= (size_t)f.V * Q) return;
+  const int q = (int)(e % Q), v = (int)(e / Q);
   int X, Y, Z;
   coords(f, v, X, Y, Z);
-  y[e] = x[((size_t)(X / 2) + c.X * ((Y / 2) + (size_t)c.Y * (Z / 2))) * C + ch];
+  ((u32x4*)y)[e] =
+      ((const u32x4*)x)[((size_t)(X / 2) + c.X * ((Y / 2) + (size_t)c.Y * (Z / 2))) * Q + q];
 }
 
 __global__ void k_up_bwd(Dims c, Dims f, int C, const float* __restrict__ dy,
@@ -273,13 +421,6 @@ __global__ void k_up_bwd(Dims c, Dims f, int C, const float* __restrict__ dy,
   dx[e] = s;
 }
 
-// y = a + b (BF16), the skip connection
-__global__ void k_add_bf16(size_t n, const uint16_t* __restrict__ a,
-                           const uint16_t* __restrict__ b, uint16_t* __restrict__ y) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) y[e] = f2bf(bf2f(a[e]) + bf2f(b[e]));
-}
-
 // ReLU backward through the post-activation y, summing two incoming
 // gradients: out = (g + g2) * (y > 0)   (g2 may be null; out may alias g)
 __global__ void k_relu_bwd(size_t n, const uint16_t* __restrict__ y, const float* g,
@@ -290,8 +431,8 @@ __global__ void k_relu_bwd(size_t n, const uint16_t* __restrict__ y, const float
   out[e] = bf2f(y[e]) > 0.f ? v : 0.f;
 }
 
-// loss partials and gradient of L = mean_v (out[v][0] - t[v])^2 (out FP32,
-// C channels; only channel 0 is the prediction)
+// loss partials and gradient of L = mean_v (out[v] - t[v])^2 (out FP32, the
+// head's channel 0; its other channels have no gradient)
 __global__ void __launch_bounds__(256)
     k_mse(int V, int C, const float* __restrict__ out, const float* __restrict__ tgt,
           float* __restrict__ g, float* __restrict__ part) {
@@ -299,7 +440,7 @@ __global__ void __launch_bounds__(256)
   const int v = blockIdx.x * 256 + threadIdx.x;
   float l = 0.f;
   if (v < V) {
-    const float dlt = out[(size_t)v * C] - tgt[v];
+    const float dlt = out[v] - tgt[v];
     l = dlt * dlt;
     g[(size_t)v * C] = 2.f * dlt / (float)V;
     for (int c = 1; c < C; c++) g[(size_t)v * C + c] = 0.f;
@@ -362,11 +503,9 @@ __global__ void k_features(Dims d, int C, int nt, const double* __restrict__ br0
   const int js = flip ? d.Y - 1 - j : j;
   const int ks = k + roll < d.Z ? k + roll : k + roll - d.Z;
   const float b = (float)br0[(size_t)(js + 1) + (size_t)nt * (ks + 1)] * inv_bscale;
-  uint16_t* o = x0 + (size_t)v * C;
-  o[0] = f2bf(b * decay[i]);
-  o[1] = f2bf(b);
-  o[2] = f2bf(rpos[i]);
-  for (int c = 3; c < C; c++) o[c] = 0;
+  u32x4* o = (u32x4*)(x0 + (size_t)v * C);
+  o[0] = u32x4{pack2(b * decay[i], b), (unsigned)f2bf(rpos[i]), 0u, 0u};
+  for (int c = 1; c < C / 8; c++) o[c] = u32x4{0u, 0u, 0u, 0u};
 }
 
 // Training target of a rotated/reflected sample: dst(i,j,k) = sign *
@@ -382,11 +521,11 @@ __global__ void k_gather_target(Dims d, int roll, int flip, float sign,
   dst[v] = sign * src[i + d.X * (js + d.Y * ks)];
 }
 
-// x (FP64, packed) = scale * out[v][0]
-__global__ void k_head_to_x(int V, int C, const float* __restrict__ out, double scale,
+// x (FP64, packed) = scale * out[v]
+__global__ void k_head_to_x(int V, const float* __restrict__ out, double scale,
                             double* __restrict__ xo) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < V) xo[v] = scale * (double)out[(size_t)v * C];
+  if (v < V) xo[v] = scale * (double)out[v];
 }
 
 // Trilinear prolongation of a padded coarse field phi_c(nrc,ntc,npc) to the
@@ -438,11 +577,49 @@ __global__ void k_mfma_check(const uint16_t* __restrict__ A, const uint16_t* __r
 // host launchers
 static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-void conv_fwd(const Dims3& d3, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
-              const float* bias, uint16_t* y, float* yf, bool relu, hipStream_t s) {
-  Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
-  dim3 grid(nblk(d.V, 64), Cout / 16);
-  k_conv_fwd<<<grid, 256, 0, s>>>(d, Cin, Cout, x, w, bias, y, yf, relu ? 1 : 0);
+template <int CIN, int NB>
+static void conv_mt(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
+                    const ConvOut& o, hipStream_t s) {
+  const unsigned gy = Cout / (16 * NB);
+  // tiles per wave: as many as leave a few waves to every SIMD (1024 of them)
+  if (d.V >= 200000)
+    k_conv<CIN, NB, 4><<<dim3(nblk(d.V, 256), gy), 256, 0, s>>>(d, Cout, x, w, o);
+  else if (d.V >= 50000)
+    k_conv<CIN, NB, 2><<<dim3(nblk(d.V, 128), gy), 256, 0, s>>>(d, Cout, x, w, o);
+  else
+    k_conv<CIN, NB, 1><<<dim3(nblk(d.V, 64), gy), 256, 0, s>>>(d, Cout, x, w, o);
+}
+
+template <int CIN>
+static void conv_nb(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
+                    const ConvOut& o, hipStream_t s) {
+  if (Cout % 32 == 0 && d.V >= 10000)
+    conv_mt<CIN, 2>(d, Cout, x, w, o, s);
+  else
+    conv_mt<CIN, 1>(d, Cout, x, w, o, s);
+}
+
+static void conv(const Dims3& d3, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
+                 const ConvOut& o, hipStream_t s) {
+  const Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
+  if (Cin == 16)
+    conv_nb<16>(d, Cout, x, w, o, s);
+  else if (Cin == 32)
+    conv_nb<32>(d, Cout, x, w, o, s);
+  else if (Cin == 64)
+    conv_nb<64>(d, Cout, x, w, o, s);
+  else
+    conv_nb<128>(d, Cout, x, w, o, s);
+}
+
+void conv_relu(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
+               const float* bias, uint16_t* y, const uint16_t* e, uint16_t* sum, hipStream_t s) {
+  conv(d, Cin, Cout, x, w, ConvOut{y, e, sum, nullptr, nullptr, bias, 1}, s);
+}
+
+void conv_head(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
+               const float* bias, float* y1, hipStream_t s) {
+  conv(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0}, s);
 }
 
 void conv_bwd(const Dims3& d3, int Cin, int Cout, const float* dy, const uint16_t* x,
@@ -466,7 +643,7 @@ void conv_bwd(const Dims3& d3, int Cin, int Cout, const float* dy, const uint16_
 void pool_fwd(const Dims3& f3, const Dims3& c3, int C, const uint16_t* x, uint16_t* y,
               hipStream_t s) {
   Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
-  k_pool_fwd<<<nblk((size_t)c.V * C, 256), 256, 0, s>>>(f, c, C, x, y);
+  k_pool_fwd<<<nblk((size_t)c.V * (C / 8), 256), 256, 0, s>>>(f, c, C, x, y);
 }
 void pool_bwd(const Dims3& f3, const Dims3& c3, int C, const float* dy, float* dx,
               hipStream_t s) {
@@ -476,15 +653,12 @@ void pool_bwd(const Dims3& f3, const Dims3& c3, int C, const float* dy, float* d
 void up_fwd(const Dims3& c3, const Dims3& f3, int C, const uint16_t* x, uint16_t* y,
             hipStream_t s) {
   Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
-  k_up_fwd<<<nblk((size_t)f.V * C, 256), 256, 0, s>>>(c, f, C, x, y);
+  k_up_fwd<<<nblk((size_t)f.V * (C / 8), 256), 256, 0, s>>>(c, f, C, x, y);
 }
 void up_bwd(const Dims3& c3, const Dims3& f3, int C, const float* dy, float* dx,
             hipStream_t s) {
   Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
   k_up_bwd<<<nblk((size_t)c.V * C, 256), 256, 0, s>>>(c, f, C, dy, dx);
-}
-void add_bf16(size_t n, const uint16_t* a, const uint16_t* b, uint16_t* y, hipStream_t s) {
-  k_add_bf16<<<nblk(n, 256), 256, 0, s>>>(n, a, b, y);
 }
 void relu_bwd(size_t n, const uint16_t* y, const float* g, const float* g2, float* out,
               hipStream_t s) {
@@ -519,8 +693,8 @@ void gather_target(const Dims3& d3, int roll, int flip, float sign, const float*
   Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
   k_gather_target<<<nblk(d.V, 256), 256, 0, s>>>(d, roll, flip, sign, src, dst);
 }
-void head_to_x(int V, int C, const float* out, double scale, double* xo, hipStream_t s) {
-  k_head_to_x<<<nblk(V, 256), 256, 0, s>>>(V, C, out, scale, xo);
+void head_to_x(int V, const float* out, double scale, double* xo, hipStream_t s) {
+  k_head_to_x<<<nblk(V, 256), 256, 0, s>>>(V, out, scale, xo);
 }
 void prolong(int af, int bf, int cf, int nrc, int ntc, int npc, const double* phic,
              const int* ir, const double* wr, const int* it, const double* wt, const int* ip,
