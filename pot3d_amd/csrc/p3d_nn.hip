@@ -85,12 +85,13 @@ struct p3d_nn {
   // activations (BF16)
   uint16_t *x0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *u2, *d2, *s2, *u1, *d1, *s1, *u0, *d0, *s0;
   float* out = nullptr;
-  // gradients (FP32)
-  float *g_out, *g_s0, *g_t0, *g_u0, *g_s1, *g_t1, *g_u1, *g_s2, *g_t2, *g_u2, *g_e3, *g_p3,
-      *g_e2, *g_p2, *g_e1, *g_p1, *g_e0;
-  float* part = nullptr;  // weight-gradient partials
-  size_t part_n = 0;
-  float* lpart = nullptr;  // loss partials
+  // gradients of the convolutions' inputs and of the skip sums (FP32), and of
+  // one convolution's output (BF16)
+  float *g_s0, *g_u0, *g_s1, *g_u1, *g_s2, *g_u2, *g_e3, *g_p3, *g_p2, *g_p1;
+  uint16_t* dy = nullptr;
+  uint16_t* wt = nullptr;  // flipped weights (BF16)
+  float* part = nullptr;   // weight-gradient partials
+  float *lpart = nullptr, *bpart = nullptr;  // loss and bias-gradient partials
   float* loss = nullptr;   // device scalar
   // features
   float *decay = nullptr, *rpos = nullptr;
@@ -101,6 +102,7 @@ struct p3d_nn {
   std::vector<double> ds_bs;  // per-sample input scale
   std::vector<float*> ds_t;
   float* tgt = nullptr;  // current target (FP32, /phiscale)
+  double* x64 = nullptr;  // solution of a single pair, as it was given
   // training augmentation by exact symmetries of the discrete problem:
   // rotation in phi (uniform phi mesh), reflection in theta (mesh symmetric
   // about the equator), sign (the solution is linear in br0)
@@ -143,53 +145,50 @@ static void forward(p3d_nn* n) {
   conv_head(D[0], 16, 16, n->s0, W(7), B(7), n->out, s);
 }
 
-static int nchunk_for(const Dims3& d) {
-  int nc = (int)((d.V() + 2047) / 2048);
-  return nc < 1 ? 1 : nc;
-}
-
+// From dy, the gradient of the head's output (and GB(7) already there).
 static void backward(p3d_nn* n) {
   hipStream_t s = n->stream;
-  auto W = [&](int i) { return n->wb + n->conv[i].w_off; };
-  auto GW = [&](int i) { return n->g + n->conv[i].w_off; };
-  auto GB = [&](int i) { return n->g + n->conv[i].b_off; };
+  ConvTable ct;
+  ct.n = (int)n->conv.size();
+  for (int i = 0; i < ct.n; i++)
+    ct.e[i] = {n->conv[i].Cin, n->conv[i].Cout, n->conv[i].w_off};
+  flip_weights(ct, n->wb, n->wt, s);
   const Dims3* D = n->D;
-  const size_t V0 = D[0].V(), V1 = D[1].V(), V2 = D[2].V(), V3 = D[3].V();
-  // head: out = conv(s0)
-  conv_bwd(D[0], 16, 16, n->g_out, n->s0, W(7), n->g_s0, GW(7), GB(7), n->part,
-           nchunk_for(D[0]), s);
+  // convolution i: input x, gradient of the output in dy; dx may be null
+  auto conv = [&](int i, const uint16_t* x, float* dx) {
+    const ConvSpec& c = n->conv[i];
+    conv_bwd(D[c.level], c.Cin, c.Cout, n->dy, x, n->wt + c.w_off, dx, n->g + c.w_off, n->part,
+             s);
+  };
+  // its ReLU (output y), from the gradient ga and that of y's pooling
+  auto relu = [&](int i, const uint16_t* y, const float* ga, const float* gp) {
+    const ConvSpec& c = n->conv[i];
+    relu_bwd(D[c.level], D[c.level < 3 ? c.level + 1 : 3], c.Cout, y, ga, gp, n->dy, n->bpart,
+             n->g + c.b_off, s);
+  };
+  conv(7, n->s0, n->g_s0);
   // s0 = relu(conv(u0)) + e0
-  relu_bwd(V0 * 16, n->d0, n->g_s0, nullptr, n->g_t0, s);
-  conv_bwd(D[0], 32, 16, n->g_t0, n->u0, W(6), n->g_u0, GW(6), GB(6), n->part, nchunk_for(D[0]),
-           s);
+  relu(6, n->d0, n->g_s0, nullptr);
+  conv(6, n->u0, n->g_u0);
   up_bwd(D[1], D[0], 32, n->g_u0, n->g_s1, s);
   // s1 = relu(conv(u1)) + e1
-  relu_bwd(V1 * 32, n->d1, n->g_s1, nullptr, n->g_t1, s);
-  conv_bwd(D[1], 64, 32, n->g_t1, n->u1, W(5), n->g_u1, GW(5), GB(5), n->part, nchunk_for(D[1]),
-           s);
+  relu(5, n->d1, n->g_s1, nullptr);
+  conv(5, n->u1, n->g_u1);
   up_bwd(D[2], D[1], 64, n->g_u1, n->g_s2, s);
   // s2 = relu(conv(u2)) + e2
-  relu_bwd(V2 * 64, n->d2, n->g_s2, nullptr, n->g_t2, s);
-  conv_bwd(D[2], 128, 64, n->g_t2, n->u2, W(4), n->g_u2, GW(4), GB(4), n->part,
-           nchunk_for(D[2]), s);
+  relu(4, n->d2, n->g_s2, nullptr);
+  conv(4, n->u2, n->g_u2);
   up_bwd(D[3], D[2], 128, n->g_u2, n->g_e3, s);
   // e3 = relu(conv(p3))
-  relu_bwd(V3 * 128, n->e3, n->g_e3, nullptr, n->g_e3, s);
-  conv_bwd(D[3], 64, 128, n->g_e3, n->p3, W(3), n->g_p3, GW(3), GB(3), n->part,
-           nchunk_for(D[3]), s);
-  pool_bwd(D[2], D[3], 64, n->g_p3, n->g_e2, s);
-  // e2 feeds pool (g_e2) and the skip of s2 (g_s2)
-  relu_bwd(V2 * 64, n->e2, n->g_e2, n->g_s2, n->g_e2, s);
-  conv_bwd(D[2], 32, 64, n->g_e2, n->p2, W(2), n->g_p2, GW(2), GB(2), n->part, nchunk_for(D[2]),
-           s);
-  pool_bwd(D[1], D[2], 32, n->g_p2, n->g_e1, s);
-  relu_bwd(V1 * 32, n->e1, n->g_e1, n->g_s1, n->g_e1, s);
-  conv_bwd(D[1], 16, 32, n->g_e1, n->p1, W(1), n->g_p1, GW(1), GB(1), n->part, nchunk_for(D[1]),
-           s);
-  pool_bwd(D[0], D[1], 16, n->g_p1, n->g_e0, s);
-  relu_bwd(V0 * 16, n->e0, n->g_e0, n->g_s0, n->g_e0, s);
-  conv_bwd(D[0], 16, 16, n->g_e0, n->x0, W(0), nullptr, GW(0), GB(0), n->part, nchunk_for(D[0]),
-           s);
+  relu(3, n->e3, n->g_e3, nullptr);
+  conv(3, n->p3, n->g_p3);
+  // e2, e1, e0 feed a pooling and a skip sum
+  relu(2, n->e2, n->g_s2, n->g_p3);
+  conv(2, n->p2, n->g_p2);
+  relu(1, n->e1, n->g_s1, n->g_p2);
+  conv(1, n->p1, n->g_p1);
+  relu(0, n->e0, n->g_s0, n->g_p1);
+  conv(0, n->x0, nullptr);
 }
 
 static void make_features(p3d_nn* n, const double* br_dev, double bs, int roll = 0,
@@ -256,7 +255,7 @@ int p3d_nn_create(p3d_nn** out, int nr, int nt, int np, const double* rh, unsign
   const size_t P = n->nparam;
   if ((rc = dmalloc(n, (void**)&n->w, P * 4)) || (rc = dmalloc(n, (void**)&n->g, P * 4)) ||
       (rc = dmalloc(n, (void**)&n->m1, P * 4)) || (rc = dmalloc(n, (void**)&n->m2, P * 4)) ||
-      (rc = dmalloc(n, (void**)&n->wb, P * 2))) {
+      (rc = dmalloc(n, (void**)&n->wb, P * 2)) || (rc = dmalloc(n, (void**)&n->wt, P * 2))) {
     p3d_nn_destroy(n);
     return rc;
   }
@@ -282,7 +281,8 @@ int p3d_nn_create(p3d_nn** out, int nr, int nt, int np, const double* rh, unsign
               {&n->p2, V2 * 32}, {&n->e2, V2 * 64}, {&n->p3, V3 * 64}, {&n->e3, V3 * 128},
               {&n->u2, V2 * 128}, {&n->d2, V2 * 64}, {&n->s2, V2 * 64}, {&n->u1, V1 * 64},
               {&n->d1, V1 * 32}, {&n->s1, V1 * 32}, {&n->u0, V0 * 32}, {&n->d0, V0 * 16},
-              {&n->s0, V0 * 16}};
+              {&n->s0, V0 * 16},
+              {&n->dy, std::max({V0 * 16, V1 * 32, V2 * 64, V3 * 128})}};
   for (auto& a : acts) {
     if ((rc = dmalloc(n, (void**)a.p, kZeroFront + a.n * 2))) {
       p3d_nn_destroy(n);
@@ -294,29 +294,26 @@ int p3d_nn_create(p3d_nn** out, int nr, int nt, int np, const double* rh, unsign
   struct {
     float** p;
     size_t n;
-  } grads[] = {{&n->out, V0},        {&n->g_out, V0 * 16}, {&n->g_s0, V0 * 16},
-               {&n->g_t0, V0 * 16},  {&n->g_u0, V0 * 32},  {&n->g_s1, V1 * 32},
-               {&n->g_t1, V1 * 32},  {&n->g_u1, V1 * 64},  {&n->g_s2, V2 * 64},
-               {&n->g_t2, V2 * 64},  {&n->g_u2, V2 * 128}, {&n->g_e3, V3 * 128},
-               {&n->g_p3, V3 * 64},  {&n->g_e2, V2 * 64},  {&n->g_p2, V2 * 32},
-               {&n->g_e1, V1 * 32},  {&n->g_p1, V1 * 16},  {&n->g_e0, V0 * 16},
-               {&n->tgt, V0},        {&n->lpart, V0 / 256 + 2}, {&n->loss, 4}};
+  } grads[] = {{&n->out, V0},       {&n->g_s0, V0 * 16}, {&n->g_u0, V0 * 32},
+               {&n->g_s1, V1 * 32}, {&n->g_u1, V1 * 64}, {&n->g_s2, V2 * 64},
+               {&n->g_u2, V2 * 128}, {&n->g_e3, V3 * 128}, {&n->g_p3, V3 * 64},
+               {&n->g_p2, V2 * 32}, {&n->g_p1, V1 * 16}, {&n->tgt, V0},
+               {(float**)&n->x64, V0 * 2}, {&n->lpart, kSumBlocks},
+               {&n->bpart, kSumBlocks * 128}, {&n->loss, 4}};
   for (auto& a : grads)
     if ((rc = dmalloc(n, (void**)a.p, a.n * 4))) {
       p3d_nn_destroy(n);
       return rc;
     }
-  // weight-gradient partials: the largest nchunk*27*Cout*Cin over layers
+  // weight-gradient partials: the largest over the layers
   size_t pn = 0;
-  for (const ConvSpec& cs : n->conv) {
-    const size_t need = (size_t)nchunk_for(n->D[cs.level]) * 27 * cs.Cin * cs.Cout;
-    if (need > pn) pn = need;
-  }
+  for (const ConvSpec& cs : n->conv)
+    pn = std::max(pn, (size_t)wgrad_chunks(n->D[cs.level], cs.Cin, cs.Cout) * 27 * cs.Cin *
+                          cs.Cout);
   if ((rc = dmalloc(n, (void**)&n->part, pn * 4))) {
     p3d_nn_destroy(n);
     return rc;
   }
-  n->part_n = pn;
   // radial feature tables on the interior shells: (r0/r)^2 and (r-r0)/(r1-r0)
   std::vector<float> dec(n->a), rp(n->a);
   const double r0 = 0.5 * (rh[0] + rh[1]), r1 = 0.5 * (rh[nr - 2] + rh[nr - 1]);
@@ -394,14 +391,13 @@ int p3d_nn_add_sample(p3d_nn* n, const double* br0, const double* x) {
 int p3d_nn_loss_grad(p3d_nn* n, const double* br0, const double* x, double* loss, float* grads) {
   if (!n || !br0 || !x || !loss) return nfail(P3D_EINVAL, "null argument");
   const size_t nb = (size_t)n->nt * (n->c + 2), V = n->D[0].V();
-  std::vector<float> t(V);
   const double bs = sample_scale(n, br0), ts = target_scale(n, bs);
-  for (size_t v = 0; v < V; v++) t[v] = (float)(x[v] / ts);
   hipMemcpyAsync(n->br_dev, br0, nb * 8, hipMemcpyHostToDevice, n->stream);
-  hipMemcpyAsync(n->tgt, t.data(), V * 4, hipMemcpyHostToDevice, n->stream);
+  hipMemcpyAsync(n->x64, x, V * 8, hipMemcpyHostToDevice, n->stream);
   make_features(n, n->br_dev, bs);
   forward(n);
-  mse((int)V, 16, n->out, n->tgt, n->g_out, n->lpart, n->loss, n->stream);
+  mse((int)V, n->out, nullptr, n->x64, ts, n->dy, n->lpart, n->bpart, n->loss,
+      n->g + n->conv[7].b_off, n->stream);
   backward(n);
   float l = 0.f;
   hipMemcpyAsync(&l, n->loss, 4, hipMemcpyDeviceToHost, n->stream);
@@ -444,7 +440,8 @@ int p3d_nn_train(p3d_nn* n, int nsteps, double lr, unsigned seed, float* losses)
     }
     make_features(n, n->ds_br[q], bs, roll, flip);
     forward(n);
-    mse(V, 16, n->out, tq, n->g_out, n->lpart, dloss + it, n->stream);
+    mse(V, n->out, tq, nullptr, 1.0, n->dy, n->lpart, n->bpart, dloss + it,
+        n->g + n->conv[7].b_off, n->stream);
     backward(n);
     n->step++;
     adam(n->nparam, n->w, n->g, n->m1, n->m2, (float)lr, 0.9f, 0.999f, 1e-8f, n->step, n->wb,

@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "p3d_nn.hpp"
 
 namespace p3d {
@@ -58,17 +60,7 @@ struct Dims {
   int V;
 };
 
-// neighbour of (x,y,z) at tap t = (dx+1) + 3*(dy+1) + 9*(dz+1), or -1
-__device__ __forceinline__ int neighbour(const Dims& d, int x, int y, int z, int t, int sign) {
-  const int dx = (t % 3 - 1) * sign, dy = ((t / 3) % 3 - 1) * sign, dz = (t / 9 - 1) * sign;
-  const int xn = x + dx, yn = y + dy;
-  if (xn < 0 || xn >= d.X || yn < 0 || yn >= d.Y) return -1;
-  int zn = z + dz;
-  if (zn < 0) zn += d.Z;
-  if (zn >= d.Z) zn -= d.Z;
-  return xn + d.X * (yn + d.Y * zn);
-}
-
+// Tap t = (dx+1) + 3*(dy+1) + 9*(dz+1).
 __device__ __forceinline__ void coords(const Dims& d, int v, int& x, int& y, int& z) {
   x = v % d.X;
   const int r = v / d.X;
@@ -237,106 +229,174 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// dx[v][ci] = sum_t sum_co dy[nb(v,-t)][co] w[t][co][ci]   (FP32 out)
-__global__ void __launch_bounds__(256)
-    k_conv_bwd_data(Dims d, int Cin, int Cout, const float* __restrict__ dy,
-                    const uint16_t* __restrict__ w, float* __restrict__ dx) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int v0 = (blockIdx.x * 4 + wave) * 16;
-  const int ci0 = blockIdx.y * 16;
-  const int m = lane & 15, kb = lane >> 4;
-  const int v = v0 + m;
-  int vx = 0, vy = 0, vz = 0;
-  const bool valid = v < d.V;
-  if (valid) coords(d, v, vx, vy, vz);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int ncb = Cout / 16;
-  for (int t = 0; t < 27; t++) {
-    const int vn = valid ? neighbour(d, vx, vy, vz, t, -1) : -1;
-    for (int cb = 0; cb < ncb; cb++) {
-      bf16x4 a = {0, 0, 0, 0};
-      if (vn >= 0) {
-        const float* src = dy + (size_t)vn * Cout + cb * 16 + 4 * kb;
-#pragma unroll
-        for (int q = 0; q < 4; q++) a[q] = (short)f2bf(src[q]);
-      }
-      bf16x4 b;
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        b[q] = (short)w[((size_t)t * Cout + cb * 16 + 4 * kb + q) * Cin + ci0 + m];
-      acc = mfma16(a, b, acc);
-    }
-  }
-  const int ci = ci0 + m;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int vo = v0 + 4 * kb + i;
-    if (vo < d.V) dx[(size_t)vo * Cin + ci] = acc[i];
-  }
+// dst[t][ci][co] = src[26-t][co][ci] for every convolution of the parameter
+// buffer: the gradient of a convolution's input is the convolution of the
+// output's gradient with these weights (dx[v][ci] = sum_t sum_co
+// dy[nb(v,-t)][co] w[t][co][ci], and tap 26-t is the opposite of t).
+__global__ void k_flip_weights(ConvTable ct, const uint16_t* __restrict__ src,
+                               uint16_t* __restrict__ dst) {
+  const ConvTable::Entry c = ct.e[blockIdx.y];
+  const int e = blockIdx.x * 256 + threadIdx.x, cc = c.Cin * c.Cout;
+  if (e >= 27 * cc) return;
+  const int t = e / cc, r = e - t * cc, ci = r / c.Cout, co = r - ci * c.Cout;
+  dst[c.w_off + e] = src[c.w_off + (size_t)(26 - t) * cc + (size_t)co * c.Cin + ci];
 }
 
 // Partial weight gradients: part[chunk][t][co][ci] = sum over the chunk's
-// voxels of dy[v][co] x[nb(v,t)][ci].  grid (nchunk, 27, (Cout/16)*(Cin/16)),
-// block 64 (one wave per 16x16 tile).
-__global__ void __launch_bounds__(64)
-    k_conv_bwd_weight(Dims d, int Cin, int Cout, int chunk, const float* __restrict__ dy,
+// voxels of dy[v][co] x[nb(v,t)][ci].  grid (chunks, (Cout/(16 COB)) *
+// (Cin/(16 CIB))), block 256.
+//
+// K of this contraction is the voxels, which neither operand has innermost:
+// 128 (or 96) voxels of dy and, for each of the nine (dy, dz) shifts, the 130 voxels
+// of x that the three dx need are staged in LDS as they lie in memory, and the
+// transposing LDS read (ds_read_b64_tr_b16: sixteen lanes read a 4 x 16 block
+// by rows and receive it by columns) hands the matrix unit its operands.
+// Wave w takes taps w, w + 4, ... and keeps their 16 x 16 results in
+// registers over the whole chunk.  A tap outside the grid reads a row of
+// zeros.
+//
+// What bounds it: the LDS reads, 512 bytes for every four k of a tap, and the
+// index arithmetic before each.  Backward pass at 51x91x181, the eight weight
+// gradients: 4183 us with two-byte loads from memory, 560 us so.
+// voxels per step: 128, 96 where two workgroups would not fit a CU's LDS
+constexpr int wgrad_step(int cib, int cob) { return cib == 2 && cob == 2 ? 96 : 128; }
+
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+__device__ __forceinline__ uint2 lds_read_tr(const uint16_t* p) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)p));
+}
+
+template <int CIB, int COB>
+__global__ void __launch_bounds__(256)
+    k_conv_bwd_weight(Dims d, int Cin, int Cout, int chunk, const uint16_t* __restrict__ dy,
                       const uint16_t* __restrict__ x, float* __restrict__ part) {
-  const int lane = threadIdx.x;
-  const int t = blockIdx.y;
-  const int nci = Cin / 16;
-  const int co0 = (blockIdx.z / nci) * 16, ci0 = (blockIdx.z % nci) * 16;
+  constexpr int XQ = 2 * CIB, YQ = 2 * COB;  // 16-byte words of a row
+  constexpr int kWV = wgrad_step(CIB, COB), kWR = kWV + 2;  // rows of a segment
+  __shared__ u32x4 sx[(9 * kWR + 1) * XQ];   // the last row is zero
+  __shared__ u32x4 sy[kWV * YQ];
+  __shared__ unsigned flag[kWV];  // bit dx + 3 dy: that shift stays in the grid
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = lane & 15, kb = lane >> 4;
+  const int nci = Cin / (16 * CIB);
+  const int co0 = ((int)blockIdx.y / nci) * (16 * COB), ci0 = ((int)blockIdx.y % nci) * (16 * CIB);
   const int vbeg = blockIdx.x * chunk, vend = min(d.V, vbeg + chunk);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int vb = vbeg; vb < vend; vb += 16) {
-    bf16x4 a, b;
+  const int XY = d.X * d.Y;
+  f32x4 acc[7][COB][CIB];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int v = vb + 4 * kb + q;
-      float av = 0.f;
-      short bv = 0;
+  for (int q = 0; q < 7; q++)
+#pragma unroll
+    for (int a = 0; a < COB; a++)
+#pragma unroll
+      for (int b = 0; b < CIB; b++) acc[q][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (tid < XQ) sx[9 * kWR * XQ + tid] = u32x4{0u, 0u, 0u, 0u};
+  const u32x4* xq = (const u32x4*)x + ci0 / 8;
+  const u32x4* yq = (const u32x4*)dy + co0 / 8;
+  for (int v0 = vbeg; v0 < vend; v0 += kWV) {
+    __syncthreads();
+    for (int e = tid; e < kWV * YQ; e += 256) {
+      const int v = v0 + e / YQ;
+      u32x4 w = {0u, 0u, 0u, 0u};
+      if (v < vend) w = yq[(size_t)v * (Cout / 8) + e % YQ];
+      sy[e] = w;
+    }
+    if (tid < kWV) {
+      const int v = v0 + tid;
+      unsigned f = 0;
       if (v < vend) {
-        av = dy[(size_t)v * Cout + co0 + m];
         int vx, vy, vz;
         coords(d, v, vx, vy, vz);
-        const int vn = neighbour(d, vx, vy, vz, t, 1);
-        if (vn >= 0) bv = (short)x[(size_t)vn * Cin + ci0 + m];
+        const unsigned fx = (vx > 0 ? 1u : 0u) | 2u | (vx < d.X - 1 ? 4u : 0u);
+        f = (vy > 0 ? fx : 0u) | fx << 3 | (vy < d.Y - 1 ? fx << 6 : 0u);
       }
-      a[q] = (short)f2bf(av);
-      b[q] = bv;
+      flag[tid] = f;
     }
-    acc = mfma16(a, b, acc);
+    // segment r = (dy+1) + 3 (dz+1): voxels v0 - 1 .. v0 + kWV shifted by it.
+    // Where the shift leaves the grid in y the row is some other voxel's and
+    // not read; in z it is the periodic neighbour's (both are V-periodic)
+#pragma unroll 3
+    for (int r = 0; r < 9; r++) {
+      const int base = v0 - 1 + d.X * (r % 3 - 1) + XY * (r / 3 - 1);
+      for (int e = tid; e < kWR * XQ; e += 256) {
+        int v = base + e / XQ;
+        v = v < 0 ? v + d.V : v;
+        v = v >= d.V ? v - d.V : v;
+        // (a grid of few planes can leave the range even so)
+        v = max(0, min(v, d.V - 1));
+        sx[r * kWR * XQ + e] = xq[(size_t)v * (Cin / 8) + e % XQ];
+      }
+    }
+    __syncthreads();
+    const uint16_t* lx = (const uint16_t*)sx;
+    const uint16_t* ly = (const uint16_t*)sy;
+    const int kr = 4 * kb + (m >> 2), col = (m & 3) * 4;  // this lane's row and part of it
+#pragma unroll 1
+    for (int b = 0; b < kWV / 32; b++) {
+      const int k0 = 32 * b + kr, k1 = k0 + 16;
+      const unsigned f0 = flag[k0], f1 = flag[k1];
+      u32x4 a[COB];
+#pragma unroll
+      for (int q = 0; q < COB; q++) {
+        const uint2 p0 = lds_read_tr(ly + k0 * (YQ * 8) + q * 16 + col);
+        const uint2 p1 = lds_read_tr(ly + k1 * (YQ * 8) + q * 16 + col);
+        a[q] = u32x4{p0.x, p0.y, p1.x, p1.y};
+      }
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        const int t = 4 * q + wave;
+        if (t < 27) {
+          const int bit = t % 9, seg = t / 3;
+          const int row = seg * kWR + t % 3;
+          const int r0 = (f0 >> bit) & 1u ? row + k0 : 9 * kWR;
+          const int r1 = (f1 >> bit) & 1u ? row + k1 : 9 * kWR;
+#pragma unroll
+          for (int c = 0; c < CIB; c++) {
+            const uint2 p0 = lds_read_tr(lx + r0 * (XQ * 8) + c * 16 + col);
+            const uint2 p1 = lds_read_tr(lx + r1 * (XQ * 8) + c * 16 + col);
+            const u32x4 bb = {p0.x, p0.y, p1.x, p1.y};
+#pragma unroll
+            for (int o = 0; o < COB; o++) acc[q][o][c] = mfma32(a[o], bb, acc[q][o][c]);
+          }
+        }
+      }
+    }
   }
   // D[co = 4*kb+i][ci = m]
-  float* out = part + ((size_t)blockIdx.x * 27 + t) * (size_t)Cout * Cin;
+  float* out = part + (size_t)blockIdx.x * 27 * (size_t)Cout * Cin;
 #pragma unroll
-  for (int i = 0; i < 4; i++) out[(size_t)(co0 + 4 * kb + i) * Cin + ci0 + m] = acc[i];
-}
-
-// gw[e] = sum over chunks (fixed order) of part[chunk][e]
-__global__ void k_reduce_chunks(int nchunk, size_t n, const float* __restrict__ part,
-                                float* __restrict__ gw) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  float s = 0.f;
-  for (int c = 0; c < nchunk; c++) s += part[(size_t)c * n + e];
-  gw[e] = s;
-}
-
-// gb[co] = sum_v dy[v][co] (one block per channel, fixed order)
-__global__ void __launch_bounds__(256)
-    k_bias_grad(int V, int C, const float* __restrict__ dy, float* __restrict__ gb) {
-  __shared__ float sh[256];
-  const int co = blockIdx.x;
-  float s = 0.f;
-  for (int v = threadIdx.x; v < V; v += 256) s += dy[(size_t)v * C + co];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
+  for (int q = 0; q < 7; q++) {
+    const int t = 4 * q + wave;
+    if (t < 27)
+#pragma unroll
+      for (int o = 0; o < COB; o++)
+#pragma unroll
+        for (int c = 0; c < CIB; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            out[((size_t)t * Cout + co0 + o * 16 + 4 * kb + i) * Cin + ci0 + c * 16 + m] =
+                acc[q][o][c][i];
   }
-  if (threadIdx.x == 0) gb[co] = sh[0];
+}
+
+// out[e] = sum over chunks (fixed order) of part[chunk][e]: 64 elements a
+// block, 16 threads each (one would read the chunks one after the other: 38
+// us for 381 of them).
+__global__ void __launch_bounds__(1024)
+    k_reduce_chunks(int nchunk, size_t n, const float* __restrict__ part,
+                    float* __restrict__ out) {
+  __shared__ float sh[16][64];
+  const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const size_t e = (size_t)blockIdx.x * 64 + l;
+  float s = 0.f;
+  if (e < n)
+    for (int c = g; c < nchunk; c += 16) s += part[(size_t)c * n + e];
+  sh[g][l] = s;
+  __syncthreads();
+  if (g == 0 && e < n) {
+    float r = 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; q++) r += sh[q][l];
+    out[e] = r;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -347,7 +407,7 @@ __device__ __forceinline__ int child_count(const Dims& f, int px, int py, int pz
   return nx * ny * nz;
 }
 
-// (both forward kernels: one thread per voxel and 8 channels)
+// (one thread per voxel and 8 channels; 4 of the FP32 gradients)
 __global__ void k_pool_fwd(Dims f, Dims c, int C, const uint16_t* __restrict__ x,
                            uint16_t* __restrict__ y) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -379,18 +439,6 @@ __global__ void k_pool_fwd(Dims f, Dims c, int C, const uint16_t* __restrict__ x
   ((u32x4*)y)[e] = o;
 }
 
-__global__ void k_pool_bwd(Dims f, Dims c, int C, const float* __restrict__ dy,
-                           float* __restrict__ dx) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)f.V * C) return;
-  const int ch = (int)(e % C), v = (int)(e / C);
-  int X, Y, Z;
-  coords(f, v, X, Y, Z);
-  const int px = X / 2, py = Y / 2, pz = Z / 2;
-  dx[e] = dy[((size_t)px + c.X * (py + (size_t)c.Y * pz)) * C + ch] /
-          (float)child_count(f, px, py, pz);
-}
-
 __global__ void k_up_fwd(Dims c, Dims f, int C, const uint16_t* __restrict__ x,
                          uint16_t* __restrict__ y) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -406,59 +454,117 @@ __global__ void k_up_fwd(Dims c, Dims f, int C, const uint16_t* __restrict__ x,
 __global__ void k_up_bwd(Dims c, Dims f, int C, const float* __restrict__ dy,
                          float* __restrict__ dx) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (size_t)c.V * C) return;
-  const int ch = (int)(e % C), v = (int)(e / C);
+  const int Q = C / 4;
+  if (e >= (size_t)c.V * Q) return;
+  const int q = (int)(e % Q), v = (int)(e / Q);
   int px, py, pz;
   coords(c, v, px, py, pz);
-  float s = 0.f;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
   for (int dz = 0; dz < 2; dz++)
     for (int dy_ = 0; dy_ < 2; dy_++)
       for (int dx_ = 0; dx_ < 2; dx_++) {
         const int X = 2 * px + dx_, Y = 2 * py + dy_, Z = 2 * pz + dz;
         if (X < f.X && Y < f.Y && Z < f.Z)
-          s += dy[((size_t)X + f.X * (Y + (size_t)f.Y * Z)) * C + ch];
+          s += ((const f32x4*)dy)[((size_t)X + f.X * (Y + (size_t)f.Y * Z)) * Q + q];
       }
-  dx[e] = s;
+  ((f32x4*)dx)[e] = s;
 }
 
-// ReLU backward through the post-activation y, summing two incoming
-// gradients: out = (g + g2) * (y > 0)   (g2 may be null; out may alias g)
-__global__ void k_relu_bwd(size_t n, const uint16_t* __restrict__ y, const float* g,
-                           const float* g2, float* out) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const float v = g[e] + (g2 ? g2[e] : 0.f);
-  out[e] = bf2f(y[e]) > 0.f ? v : 0.f;
-}
-
-// loss partials and gradient of L = mean_v (out[v] - t[v])^2 (out FP32, the
-// head's channel 0; its other channels have no gradient)
+// What a convolution's backward pass starts from: the gradient of its output,
+// g through the ReLU (post-activation y), g = ga (+ gp, the gradient of the
+// average pooling that y feeds, spread over its children), as the BF16 operand
+// of the two contractions, and the bias gradient's partial sums of the FP32
+// values, bpart[block][C].  A thread keeps its 8 channels over all its voxels
+// (C / 8 divides 256).
 __global__ void __launch_bounds__(256)
-    k_mse(int V, int C, const float* __restrict__ out, const float* __restrict__ tgt,
-          float* __restrict__ g, float* __restrict__ part) {
-  __shared__ float sh[256];
-  const int v = blockIdx.x * 256 + threadIdx.x;
-  float l = 0.f;
-  if (v < V) {
-    const float dlt = out[v] - tgt[v];
-    l = dlt * dlt;
-    g[(size_t)v * C] = 2.f * dlt / (float)V;
-    for (int c = 1; c < C; c++) g[(size_t)v * C + c] = 0.f;
+    k_relu_bwd(Dims f, Dims c, int C, const uint16_t* __restrict__ y,
+               const float* __restrict__ ga, const float* __restrict__ gp,
+               uint16_t* __restrict__ dy, float* __restrict__ bpart) {
+  __shared__ float sh[256][9];
+  const int Q = C / 8, q = threadIdx.x % Q;
+  float s[8] = {};
+  const size_t n = (size_t)f.V * Q;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
+    f32x4 g0 = {0.f, 0.f, 0.f, 0.f}, g1 = g0;
+    if (gp) {
+      int X, Y, Z;
+      coords(f, (int)(e / Q), X, Y, Z);
+      const int px = X / 2, py = Y / 2, pz = Z / 2;
+      const f32x4* p =
+          (const f32x4*)(gp + ((size_t)px + c.X * (py + (size_t)c.Y * pz)) * C + 8 * q);
+      const float k = (float)child_count(f, px, py, pz);
+      g0 = p[0] / k;
+      g1 = p[1] / k;
+    }
+    if (ga) {
+      g0 += ((const f32x4*)ga)[2 * e];
+      g1 += ((const f32x4*)ga)[2 * e + 1];
+    }
+    const u32x4 yv = ((const u32x4*)y)[e];
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float a = i % 2 ? hi2f(yv[i / 2]) : lo2f(yv[i / 2]);
+      r[i] = a > 0.f ? (i < 4 ? g0[i] : g1[i - 4]) : 0.f;
+      s[i] += r[i];
+    }
+    ((u32x4*)dy)[e] = u32x4{pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]),
+                            pack2(r[6], r[7])};
   }
-  sh[threadIdx.x] = l;
+#pragma unroll
+  for (int i = 0; i < 8; i++) sh[threadIdx.x][i] = s[i];
+  __syncthreads();
+  if ((int)threadIdx.x < C) {
+    float t = 0.f;
+    for (int r = threadIdx.x / 8; r < 256; r += Q) t += sh[r][threadIdx.x % 8];
+    bpart[(size_t)blockIdx.x * C + threadIdx.x] = t;
+  }
+}
+
+// sum of 256 values, one per thread (fixed order); result in thread 0
+__device__ __forceinline__ float block_sum(float v, float* sh) {
+  __syncthreads();
+  sh[threadIdx.x] = v;
   __syncthreads();
   for (int off = 128; off > 0; off >>= 1) {
     if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  return sh[0];
 }
 
-__global__ void k_sum(int n, const float* __restrict__ part, float* __restrict__ out, float scale) {
-  if (blockIdx.x || threadIdx.x) return;
+// L = mean_v (out[v] - t[v])^2 (out FP32, the head's channel 0; its other 15
+// channels have no gradient): part[block] the loss's partial sums, bpart
+// [block][16] those of the head's bias gradient, dy the gradient as BF16
+// operand.  An FP64 target is divided by its scale here.
+__global__ void __launch_bounds__(256)
+    k_mse(int V, const float* __restrict__ out, const float* __restrict__ tgt,
+          const double* __restrict__ tgt64, double tscale, uint16_t* __restrict__ dy,
+          float* __restrict__ part, float* __restrict__ bpart) {
+  __shared__ float sh[256];
+  float l = 0.f, g = 0.f;
+  for (int v = blockIdx.x * 256 + threadIdx.x; v < V; v += gridDim.x * 256) {
+    const float dlt = out[v] - (tgt64 ? (float)(tgt64[v] / tscale) : tgt[v]);
+    const float gv = 2.f * dlt / (float)V;
+    l += dlt * dlt;
+    g += gv;
+    u32x4* o = (u32x4*)(dy + (size_t)v * 16);
+    o[0] = u32x4{(unsigned)f2bf(gv), 0u, 0u, 0u};
+    o[1] = u32x4{0u, 0u, 0u, 0u};
+  }
+  const float ls = block_sum(l, sh), gs = block_sum(g, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = ls;
+  if (threadIdx.x < 16) bpart[blockIdx.x * 16 + threadIdx.x] = threadIdx.x == 0 ? gs : 0.f;
+}
+
+// *out = scale * sum of part[0..n)
+__global__ void __launch_bounds__(256)
+    k_sum(int n, const float* __restrict__ part, float* __restrict__ out, float scale) {
+  __shared__ float sh[256];
   float s = 0.f;
-  for (int i = 0; i < n; i++) s += part[i];
-  *out = s * scale;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) *out = s * scale;
 }
 
 // Adam (bias-corrected) on FP32 weights; refreshes the BF16 copy when wb.
@@ -481,11 +587,6 @@ __global__ void k_adam(size_t n, float* __restrict__ w, const float* __restrict_
 __global__ void k_to_bf16(size_t n, const float* __restrict__ x, uint16_t* __restrict__ y) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) y[e] = f2bf(x[e]);
-}
-
-__global__ void k_fill_u16(size_t n, uint16_t* p, uint16_t v) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) p[e] = v;
 }
 
 // Input features on the interior grid (a,b,c) from br0(nt,np) (Fortran
@@ -622,33 +723,53 @@ void conv_head(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint1
   conv(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0}, s);
 }
 
-void conv_bwd(const Dims3& d3, int Cin, int Cout, const float* dy, const uint16_t* x,
-              const uint16_t* w, float* dx, float* gw, float* gb, float* part, int nchunk,
-              hipStream_t s) {
-  Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
-  if (dx) {
-    dim3 grid(nblk(d.V, 64), Cin / 16);
-    k_conv_bwd_data<<<grid, 256, 0, s>>>(d, Cin, Cout, dy, w, dx);
-  }
-  int chunk = (d.V + nchunk - 1) / nchunk;
-  chunk = (chunk + 15) / 16 * 16;
-  const int nc = (d.V + chunk - 1) / chunk;
-  dim3 gridw(nc, 27, (Cout / 16) * (Cin / 16));
-  k_conv_bwd_weight<<<gridw, 64, 0, s>>>(d, Cin, Cout, chunk, dy, x, part);
+void flip_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s) {
+  size_t most = 0;
+  for (int i = 0; i < ct.n; i++)
+    most = std::max(most, (size_t)27 * ct.e[i].Cin * ct.e[i].Cout);
+  k_flip_weights<<<dim3(nblk(most, 256), ct.n), 256, 0, s>>>(ct, w, wt);
+}
+
+// Channel blocks of 16 per workgroup of the weight gradient (32 x 32 results
+// per tap fill a wave's registers).
+static int wgrad_block(int C) { return C % 32 == 0 ? 2 : 1; }
+
+// Chunks of voxels of a weight gradient: workgroups for four per CU, of whole
+// steps, and at most 32 MB of partial sums (they are written and read back).
+int wgrad_chunks(const Dims3& d, int Cin, int Cout) {
+  const long V = (long)d.V(), wv = wgrad_step(wgrad_block(Cin), wgrad_block(Cout));
+  const long steps = (V + wv - 1) / wv;
+  const long pairs = (long)(Cin / (16 * wgrad_block(Cin))) * (Cout / (16 * wgrad_block(Cout)));
+  long n = std::min(steps, std::max(1L, 1024 / pairs));
+  n = std::max(1L, std::min(n, (8L << 20) / (27L * Cin * Cout)));
+  const long per = (steps + n - 1) / n;
+  return (int)((steps + per - 1) / per);
+}
+
+void conv_bwd(const Dims3& d3, int Cin, int Cout, const uint16_t* dy, const uint16_t* x,
+              const uint16_t* wt, float* dx, float* gw, float* part, hipStream_t s) {
+  const Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
+  if (dx) conv(d3, Cout, Cin, dy, wt, ConvOut{nullptr, nullptr, nullptr, dx, nullptr, nullptr, 0}, s);
+  const int nc = wgrad_chunks(d3, Cin, Cout);
+  const int bi = wgrad_block(Cin), bo = wgrad_block(Cout), wv = wgrad_step(bi, bo);
+  const int steps = (d.V + wv - 1) / wv, chunk = (steps + nc - 1) / nc * wv;
+  const dim3 grid(nc, (Cin / (16 * bi)) * (Cout / (16 * bo)));
+  if (bi == 1 && bo == 1)
+    k_conv_bwd_weight<1, 1><<<grid, 256, 0, s>>>(d, Cin, Cout, chunk, dy, x, part);
+  else if (bi == 1)
+    k_conv_bwd_weight<1, 2><<<grid, 256, 0, s>>>(d, Cin, Cout, chunk, dy, x, part);
+  else if (bo == 1)
+    k_conv_bwd_weight<2, 1><<<grid, 256, 0, s>>>(d, Cin, Cout, chunk, dy, x, part);
+  else
+    k_conv_bwd_weight<2, 2><<<grid, 256, 0, s>>>(d, Cin, Cout, chunk, dy, x, part);
   const size_t nw = (size_t)27 * Cout * Cin;
-  k_reduce_chunks<<<nblk(nw, 256), 256, 0, s>>>(nc, nw, part, gw);
-  k_bias_grad<<<Cout, 256, 0, s>>>(d.V, Cout, dy, gb);
+  k_reduce_chunks<<<nblk(nw, 64), 1024, 0, s>>>(nc, nw, part, gw);
 }
 
 void pool_fwd(const Dims3& f3, const Dims3& c3, int C, const uint16_t* x, uint16_t* y,
               hipStream_t s) {
   Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
   k_pool_fwd<<<nblk((size_t)c.V * (C / 8), 256), 256, 0, s>>>(f, c, C, x, y);
-}
-void pool_bwd(const Dims3& f3, const Dims3& c3, int C, const float* dy, float* dx,
-              hipStream_t s) {
-  Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
-  k_pool_bwd<<<nblk((size_t)f.V * C, 256), 256, 0, s>>>(f, c, C, dy, dx);
 }
 void up_fwd(const Dims3& c3, const Dims3& f3, int C, const uint16_t* x, uint16_t* y,
             hipStream_t s) {
@@ -658,17 +779,24 @@ void up_fwd(const Dims3& c3, const Dims3& f3, int C, const uint16_t* x, uint16_t
 void up_bwd(const Dims3& c3, const Dims3& f3, int C, const float* dy, float* dx,
             hipStream_t s) {
   Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
-  k_up_bwd<<<nblk((size_t)c.V * C, 256), 256, 0, s>>>(c, f, C, dy, dx);
+  k_up_bwd<<<nblk((size_t)c.V * (C / 4), 256), 256, 0, s>>>(c, f, C, dy, dx);
 }
-void relu_bwd(size_t n, const uint16_t* y, const float* g, const float* g2, float* out,
-              hipStream_t s) {
-  k_relu_bwd<<<nblk(n, 256), 256, 0, s>>>(n, y, g, g2, out);
+// blocks of the kernels that leave partial sums (kSumBlocks at most)
+static unsigned sum_blocks(size_t n) { return (unsigned)std::min<size_t>(nblk(n, 256), kSumBlocks); }
+
+void relu_bwd(const Dims3& f3, const Dims3& c3, int C, const uint16_t* y, const float* ga,
+              const float* gp, uint16_t* dy, float* bpart, float* gb, hipStream_t s) {
+  const Dims f{f3.X, f3.Y, f3.Z, f3.X * f3.Y * f3.Z}, c{c3.X, c3.Y, c3.Z, c3.X * c3.Y * c3.Z};
+  const unsigned nb = sum_blocks((size_t)f.V * (C / 8));
+  k_relu_bwd<<<nb, 256, 0, s>>>(f, c, C, y, ga, gp, dy, bpart);
+  k_reduce_chunks<<<nblk(C, 64), 1024, 0, s>>>((int)nb, (size_t)C, bpart, gb);
 }
-void mse(int V, int C, const float* out, const float* tgt, float* g, float* part, float* loss,
-         hipStream_t s) {
-  const int nb = (int)nblk(V, 256);
-  k_mse<<<nb, 256, 0, s>>>(V, C, out, tgt, g, part);
-  k_sum<<<1, 1, 0, s>>>(nb, part, loss, 1.0f / (float)V);
+void mse(int V, const float* out, const float* tgt, const double* tgt64, double tscale,
+         uint16_t* dy, float* part, float* bpart, float* loss, float* gb, hipStream_t s) {
+  const unsigned nb = sum_blocks(V);
+  k_mse<<<nb, 256, 0, s>>>(V, out, tgt, tgt64, tscale, dy, part, bpart);
+  k_sum<<<1, 256, 0, s>>>((int)nb, part, loss, 1.0f / (float)V);
+  k_reduce_chunks<<<1, 1024, 0, s>>>((int)nb, 16, bpart, gb);
 }
 void adam(size_t n, float* w, const float* g, float* m1, float* m2, float lr, float b1,
           float b2, float eps, int step, uint16_t* wb, hipStream_t s) {
@@ -677,9 +805,6 @@ void adam(size_t n, float* w, const float* g, float* m1, float* m2, float lr, fl
 }
 void to_bf16(size_t n, const float* x, uint16_t* y, hipStream_t s) {
   k_to_bf16<<<nblk(n, 256), 256, 0, s>>>(n, x, y);
-}
-void fill_u16(size_t n, uint16_t* p, uint16_t v, hipStream_t s) {
-  k_fill_u16<<<nblk(n, 256), 256, 0, s>>>(n, p, v);
 }
 void features(const Dims3& d3, int C, int nt, const double* br0, const float* decay,
               const float* rpos, float inv_bscale, int roll, int flip, uint16_t* x0,
