@@ -92,6 +92,41 @@ struct ConvOut {
   int relu;
 };
 
+// The results of a wave: four channels of a voxel per lane and tile.
+template <int NB, int MT>
+__device__ __forceinline__ void conv_store(const Dims& d, int Cout, const ConvOut& o,
+                                           const f32x4 (&acc)[NB][MT], int v0, int co0, int m,
+                                           int kb) {
+#pragma unroll
+  for (int n = 0; n < NB; n++) {
+    const int co = co0 + n * 16 + 4 * kb;
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+    if (o.bias) bias = *(const f32x4*)(o.bias + co);
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      const int v = v0 + t * 16 + m;
+      if (v >= d.V) continue;
+      f32x4 r = acc[n][t] + bias;
+      if (o.relu)
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = r[i] < 0.f ? 0.f : r[i];
+      const size_t at = (size_t)v * Cout + co;
+      if (o.y) {
+        const uint2 y = make_uint2(pack2(r[0], r[1]), pack2(r[2], r[3]));
+        *(uint2*)(o.y + at) = y;
+        if (o.e) {
+          const uint2 e = *(const uint2*)(o.e + at);
+          *(uint2*)(o.s + at) =
+              make_uint2(pack2(lo2f(y.x) + lo2f(e.x), hi2f(y.x) + hi2f(e.x)),
+                         pack2(lo2f(y.y) + lo2f(e.y), hi2f(y.y) + hi2f(e.y)));
+        }
+      }
+      if (o.yf) *(f32x4*)(o.yf + at) = r;
+      if (o.y1 && co == 0) o.y1[v] = r[0];
+    }
+  }
+}
+
 template <int CIN, int NB, int MT>
 __global__ void __launch_bounds__(256)
     k_conv(Dims d, int Cout, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
@@ -199,34 +234,102 @@ __global__ void __launch_bounds__(256)
       }
     }
   }
+  conv_store<NB, MT>(d, Cout, o, acc, v0, co0, m, kb);
+}
+
+// The same for 32 channels and more with the voxels' neighbourhoods staged in
+// LDS: for each dz the 64 MT voxels of the workgroup and one row and one voxel
+// to either side, as they lie in memory, then nine taps from there.  Read
+// straight from memory the 27 taps take each voxel 27 times through L1, which
+// does not hold the neighbourhoods of a CU's workgroups; so it comes in three
+// times (and its edges).  At 51x91x181: 32->16 channels at 780 thousand
+// voxels 104 -> TBD1 us, 64->32 at 101 thousand 101 -> TBD2 us, 128->64 at 13
+// thousand 75 -> TBD3 us.
+// A row's 16-byte words are stored exchanged by the row's number, so that the
+// 16 rows of a read lie in different banks.
+template <int CIN>
+__device__ __forceinline__ int lds_word(int row, int w) {
+  constexpr int Q = CIN / 8;
+  return row * Q + (w ^ ((Q >= 16 ? row : Q == 8 ? row >> 1 : row >> 2) & (Q - 1)));
+}
+
+__host__ __device__ inline int conv_lds_rows(int MT, int X) { return 64 * MT + 2 * X + 2; }
+
+template <int CIN, int NB, int MT>
+__global__ void __launch_bounds__(256)
+    k_conv_lds(Dims d, int Cout, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+               ConvOut o) {
+  constexpr int Q = CIN / 8;
+  extern __shared__ u32x4 sx[];  // conv_lds_rows rows and a row of zeros
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, kb = lane >> 4;
+  const int per = (int)gridDim.x / 8;  // (as in k_conv)
+  const int blk = (int)blockIdx.x < 8 * per
+                      ? ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3)
+                      : (int)blockIdx.x;
+  const int vb = blk * (64 * MT), v0 = vb + wave * (16 * MT);
+  const int co0 = blockIdx.y * (16 * NB);
+  const int rows = conv_lds_rows(MT, d.X), XY = d.X * d.Y;
+  if (tid < Q) sx[rows * Q + tid] = u32x4{0u, 0u, 0u, 0u};
+  unsigned ok[MT];  // bit dx + 3 dy: that shift stays in the grid
 #pragma unroll
-  for (int n = 0; n < NB; n++) {
-    const int co = co0 + n * 16 + 4 * kb;
-    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-    if (o.bias) bias = *(const f32x4*)(o.bias + co);
-#pragma unroll
-    for (int t = 0; t < MT; t++) {
-      const int v = v0 + t * 16 + m;
-      if (v >= d.V) continue;
-      f32x4 r = acc[n][t] + bias;
-      if (o.relu)
-#pragma unroll
-        for (int i = 0; i < 4; i++) r[i] = r[i] < 0.f ? 0.f : r[i];
-      const size_t at = (size_t)v * Cout + co;
-      if (o.y) {
-        const uint2 y = make_uint2(pack2(r[0], r[1]), pack2(r[2], r[3]));
-        *(uint2*)(o.y + at) = y;
-        if (o.e) {
-          const uint2 e = *(const uint2*)(o.e + at);
-          *(uint2*)(o.s + at) =
-              make_uint2(pack2(lo2f(y.x) + lo2f(e.x), hi2f(y.x) + hi2f(e.x)),
-                         pack2(lo2f(y.y) + lo2f(e.y), hi2f(y.y) + hi2f(e.y)));
-        }
-      }
-      if (o.yf) *(f32x4*)(o.yf + at) = r;
-      if (o.y1 && co == 0) o.y1[v] = r[0];
+  for (int t = 0; t < MT; t++) {
+    const int v = v0 + t * 16 + m;
+    ok[t] = 0;
+    if (v < d.V) {
+      int vx, vy, vz;
+      coords(d, v, vx, vy, vz);
+      const unsigned fx = (vx > 0 ? 1u : 0u) | 2u | (vx < d.X - 1 ? 4u : 0u);
+      ok[t] = (vy > 0 ? fx : 0u) | fx << 3 | (vy < d.Y - 1 ? fx << 6 : 0u);
     }
   }
+  f32x4 acc[NB][MT];
+#pragma unroll
+  for (int n = 0; n < NB; n++)
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[n][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const u32x4* xq = (const u32x4*)x;
+  const u32x4* wq = (const u32x4*)w + (size_t)(co0 + m) * Q + kb;
+  const size_t wt = (size_t)Cout * Q;
+#pragma unroll 1
+  for (int dz = 0; dz < 3; dz++) {
+    if (dz) __syncthreads();
+    // rows vb - X - 1 + XY (dz - 1) on: where they leave the plane or the
+    // grid in x or y no tap reads them; in z they are V-periodic (a grid of
+    // few planes can leave the range even so)
+    const int base = vb - d.X - 1 + XY * (dz - 1);
+    for (int e = tid; e < rows * Q; e += 256) {
+      const int r = e / Q, q = e % Q;
+      int v = base + r;
+      v = v < 0 ? v + d.V : v;
+      v = v >= d.V ? v - d.V : v;
+      v = max(0, min(v, d.V - 1));
+      sx[lds_word<CIN>(r, q)] = xq[(size_t)v * Q + q];
+    }
+    __syncthreads();
+    const u32x4* wz = wq + wt * (size_t)(9 * dz);
+#pragma unroll
+    for (int r = 0; r < 9; r++) {
+      const int shift = d.X + 1 + (r % 3 - 1) + (r / 3 - 1) * d.X;
+      int row[MT];
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+        row[t] = (ok[t] >> r) & 1u ? (wave * MT + t) * 16 + m + shift : rows;
+#pragma unroll
+      for (int c = 0; c < CIN / 32; c++) {
+        u32x4 av[NB], bv[MT];
+#pragma unroll
+        for (int n = 0; n < NB; n++) av[n] = wz[wt * (size_t)r + (size_t)n * 16 * Q + 4 * c];
+#pragma unroll
+        for (int t = 0; t < MT; t++) bv[t] = sx[lds_word<CIN>(row[t], 4 * c + kb)];
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+          for (int t = 0; t < MT; t++) acc[n][t] = mfma32(av[n], bv[t], acc[n][t]);
+      }
+    }
+  }
+  conv_store<NB, MT>(d, Cout, o, acc, v0, co0, m, kb);
 }
 
 // dst[t][ci][co] = src[26-t][co][ci] for every convolution of the parameter
@@ -685,17 +788,31 @@ __global__ void k_mfma_check(const uint16_t* __restrict__ A, const uint16_t* __r
 // host launchers
 static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+template <int CIN, int NB, int MT>
+static void conv_launch(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
+                        const ConvOut& o, hipStream_t s) {
+  const dim3 grid(nblk(d.V, 64 * MT), Cout / (16 * NB));
+  if constexpr (CIN >= 32) {
+    // three workgroups per CU, or the r axis is too long for whole rows
+    const size_t lds = (size_t)(conv_lds_rows(MT, d.X) + 1) * CIN * 2;
+    if (lds <= 52 * 1024) {
+      k_conv_lds<CIN, NB, MT><<<grid, 256, lds, s>>>(d, Cout, x, w, o);
+      return;
+    }
+  }
+  k_conv<CIN, NB, MT><<<grid, 256, 0, s>>>(d, Cout, x, w, o);
+}
+
 template <int CIN, int NB>
 static void conv_mt(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
                     const ConvOut& o, hipStream_t s) {
-  const unsigned gy = Cout / (16 * NB);
   // tiles per wave: as many as leave a few waves to every SIMD (1024 of them)
   if (d.V >= 200000)
-    k_conv<CIN, NB, 4><<<dim3(nblk(d.V, 256), gy), 256, 0, s>>>(d, Cout, x, w, o);
+    conv_launch<CIN, NB, 4>(d, Cout, x, w, o, s);
   else if (d.V >= 50000)
-    k_conv<CIN, NB, 2><<<dim3(nblk(d.V, 128), gy), 256, 0, s>>>(d, Cout, x, w, o);
+    conv_launch<CIN, NB, 2>(d, Cout, x, w, o, s);
   else
-    k_conv<CIN, NB, 1><<<dim3(nblk(d.V, 64), gy), 256, 0, s>>>(d, Cout, x, w, o);
+    conv_launch<CIN, NB, 1>(d, Cout, x, w, o, s);
 }
 
 template <int CIN>
