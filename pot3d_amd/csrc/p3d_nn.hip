@@ -89,7 +89,7 @@ struct p3d_nn {
   // one convolution's output (BF16)
   float *g_s0, *g_u0, *g_s1, *g_u1, *g_s2, *g_u2, *g_e3, *g_p3, *g_p2, *g_p1;
   uint16_t* dy = nullptr;
-  uint16_t* wt = nullptr;  // flipped weights (BF16)
+  uint16_t* wt = nullptr;  // transposed weights (BF16)
   float* part = nullptr;   // weight-gradient partials
   float *lpart = nullptr, *bpart = nullptr;  // loss and bias-gradient partials
   float* loss = nullptr;   // device scalar
@@ -152,7 +152,7 @@ static void backward(p3d_nn* n) {
   ct.n = (int)n->conv.size();
   for (int i = 0; i < ct.n; i++)
     ct.e[i] = {n->conv[i].Cin, n->conv[i].Cout, n->conv[i].w_off};
-  flip_weights(ct, n->wb, n->wt, s);
+  transpose_weights(ct, n->wb, n->wt, s);
   const Dims3* D = n->D;
   // convolution i: input x, gradient of the output in dy; dx may be null
   auto conv = [&](int i, const uint16_t* x, float* dx) {

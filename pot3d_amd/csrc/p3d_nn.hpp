@@ -32,9 +32,9 @@ struct ConvTable {
 };
 // wt: the BF16 weights for the gradients of the convolutions' inputs, placed
 // as w
-void flip_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s);
+void transpose_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s);
 // dx (FP32, may be null) and gw (27*Cout*Cin, FP32) from the BF16 gradient dy
-// of the output (kZeroFront bytes before it); wt: flipped weights; part:
+// of the output (kZeroFront bytes before it); wt: transposed weights; part:
 // scratch of wgrad_chunks*27*Cout*Cin floats
 int wgrad_chunks(const Dims3& d, int Cin, int Cout);
 void conv_bwd(const Dims3& d, int Cin, int Cout, const uint16_t* dy, const uint16_t* x,

@@ -90,6 +90,7 @@ struct ConvOut {
   float* y1;          // FP32 result, channel 0 alone, or null
   const float* bias;  // or null
   int relu;
+  int dir;            // 1, or -1: the taps' shifts mirrored (input gradients)
 };
 
 // The results of a wave: four channels of a voxel per lane and tile.
@@ -144,7 +145,8 @@ __global__ void __launch_bounds__(256)
   constexpr unsigned kQ = CIN / 8;  // 16-byte words of a voxel
   const u32x4* xq = (const u32x4*)x - kZeroFront / 16;
   const unsigned lane_q = kZeroFront / 16 + (CIN == 16 ? (unsigned)(kb & 1) : (unsigned)kb);
-  const unsigned XQ = kQ * (unsigned)d.X, PQ = kQ * (unsigned)d.X * (unsigned)d.Y;
+  const bool fw = o.dir > 0;
+  const unsigned XQ = (unsigned)o.dir * kQ * (unsigned)d.X, PQ = kQ * (unsigned)d.X * (unsigned)d.Y;
   unsigned base[MT], zlo[MT], zhi[MT];
   bool in[MT], xm[MT], xp[MT], ym[MT], yp[MT];
 #pragma unroll
@@ -154,12 +156,14 @@ __global__ void __launch_bounds__(256)
     in[t] = v < d.V;
     if (in[t]) coords(d, v, vx, vy, vz);
     base[t] = lane_q + kQ * (unsigned)(in[t] ? v : 0);
-    zlo[t] = vz > 0 ? 0u - PQ : PQ * (unsigned)(d.Z - 1);
-    zhi[t] = vz < d.Z - 1 ? PQ : 0u - PQ * (unsigned)(d.Z - 1);
-    xm[t] = in[t] && vx > 0;
-    xp[t] = in[t] && vx < d.X - 1;
-    ym[t] = vy > 0;
-    yp[t] = vy < d.Y - 1;
+    const unsigned zl = vz > 0 ? 0u - PQ : PQ * (unsigned)(d.Z - 1);
+    const unsigned zh = vz < d.Z - 1 ? PQ : 0u - PQ * (unsigned)(d.Z - 1);
+    zlo[t] = fw ? zl : zh;
+    zhi[t] = fw ? zh : zl;
+    xm[t] = in[t] && (fw ? vx > 0 : vx < d.X - 1);
+    xp[t] = in[t] && (fw ? vx < d.X - 1 : vx > 0);
+    ym[t] = fw ? vy > 0 : vy < d.Y - 1;
+    yp[t] = fw ? vy < d.Y - 1 : vy > 0;
   }
   // index and validity of tap t (a constant) for tile q
   auto tap_ok = [&](int q, int t) {
@@ -169,7 +173,7 @@ __global__ void __launch_bounds__(256)
   };
   auto tap_off = [&](int q, int t) {
     const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9;
-    return (unsigned)(dx * (int)kQ) + (unsigned)dy * XQ +
+    return (unsigned)(dx * o.dir * (int)kQ) + (unsigned)dy * XQ +
            (dz == 0 ? zlo[q] : (dz == 2 ? zhi[q] : 0u));
   };
   f32x4 acc[NB][MT];
@@ -216,7 +220,7 @@ __global__ void __launch_bounds__(256)
         unsigned idx[MT];
 #pragma unroll
         for (int t = 0; t < MT; t++)
-          idx[t] = tap_ok(t, r) ? bz[t] + (unsigned)((r % 3 - 1) * (int)kQ) +
+          idx[t] = tap_ok(t, r) ? bz[t] + (unsigned)((r % 3 - 1) * o.dir * (int)kQ) +
                                       (unsigned)(r / 3 - 1) * XQ
                                 : lane_q - kZeroFront / 16;
 #pragma unroll
@@ -243,8 +247,8 @@ __global__ void __launch_bounds__(256)
 // straight from memory the 27 taps take each voxel 27 times through L1, which
 // does not hold the neighbourhoods of a CU's workgroups; so it comes in three
 // times (and its edges).  At 51x91x181: 32->16 channels at 780 thousand
-// voxels 104 -> TBD1 us, 64->32 at 101 thousand 101 -> TBD2 us, 128->64 at 13
-// thousand 75 -> TBD3 us.
+// voxels 104 -> 60 us, 64->32 at 101 thousand 101 -> 60 us, 128->64 at 13
+// thousand 75 -> 56 us.
 // A row's 16-byte words are stored exchanged by the row's number, so that the
 // 16 rows of a read lie in different banks.
 template <int CIN>
@@ -279,8 +283,11 @@ __global__ void __launch_bounds__(256)
     if (v < d.V) {
       int vx, vy, vz;
       coords(d, v, vx, vy, vz);
-      const unsigned fx = (vx > 0 ? 1u : 0u) | 2u | (vx < d.X - 1 ? 4u : 0u);
-      ok[t] = (vy > 0 ? fx : 0u) | fx << 3 | (vy < d.Y - 1 ? fx << 6 : 0u);
+      const bool fw = o.dir > 0;
+      const unsigned fx = (vx > 0 ? (fw ? 1u : 4u) : 0u) | 2u |
+                          (vx < d.X - 1 ? (fw ? 4u : 1u) : 0u);
+      ok[t] = (vy > 0 ? fx << (fw ? 0 : 6) : 0u) | fx << 3 |
+              (vy < d.Y - 1 ? fx << (fw ? 6 : 0) : 0u);
     }
   }
   f32x4 acc[NB][MT];
@@ -294,23 +301,34 @@ __global__ void __launch_bounds__(256)
 #pragma unroll 1
   for (int dz = 0; dz < 3; dz++) {
     if (dz) __syncthreads();
-    // rows vb - X - 1 + XY (dz - 1) on: where they leave the plane or the
+    // rows vb - X - 1 + XY (dz - 1) on (mirrored: 1 - dz): where they leave the plane or the
     // grid in x or y no tap reads them; in z they are V-periodic (a grid of
     // few planes can leave the range even so)
-    const int base = vb - d.X - 1 + XY * (dz - 1);
-    for (int e = tid; e < rows * Q; e += 256) {
-      const int r = e / Q, q = e % Q;
-      int v = base + r;
-      v = v < 0 ? v + d.V : v;
-      v = v >= d.V ? v - d.V : v;
-      v = max(0, min(v, d.V - 1));
-      sx[lds_word<CIN>(r, q)] = xq[(size_t)v * Q + q];
+    const int base = vb - d.X - 1 + XY * (dz - 1) * o.dir;
+    // six loads of a thread in flight at a time
+    constexpr int kB = 6;
+    for (int e0 = tid; e0 < rows * Q; e0 += 256 * kB) {
+      u32x4 b[kB];
+#pragma unroll
+      for (int u = 0; u < kB; u++) {
+        const int e = min(e0 + 256 * u, rows * Q - 1);
+        int v = base + e / Q;
+        v = v < 0 ? v + d.V : v;
+        v = v >= d.V ? v - d.V : v;
+        v = max(0, min(v, d.V - 1));
+        b[u] = xq[(size_t)v * Q + e % Q];
+      }
+#pragma unroll
+      for (int u = 0; u < kB; u++) {
+        const int e = e0 + 256 * u;
+        if (e < rows * Q) sx[lds_word<CIN>(e / Q, e % Q)] = b[u];
+      }
     }
     __syncthreads();
     const u32x4* wz = wq + wt * (size_t)(9 * dz);
 #pragma unroll
     for (int r = 0; r < 9; r++) {
-      const int shift = d.X + 1 + (r % 3 - 1) + (r / 3 - 1) * d.X;
+      const int shift = d.X + 1 + ((r % 3 - 1) + (r / 3 - 1) * d.X) * o.dir;
       int row[MT];
 #pragma unroll
       for (int t = 0; t < MT; t++)
@@ -332,17 +350,17 @@ __global__ void __launch_bounds__(256)
   conv_store<NB, MT>(d, Cout, o, acc, v0, co0, m, kb);
 }
 
-// dst[t][ci][co] = src[26-t][co][ci] for every convolution of the parameter
+// dst[t][ci][co] = src[t][co][ci] for every convolution of the parameter
 // buffer: the gradient of a convolution's input is the convolution of the
-// output's gradient with these weights (dx[v][ci] = sum_t sum_co
-// dy[nb(v,-t)][co] w[t][co][ci], and tap 26-t is the opposite of t).
-__global__ void k_flip_weights(ConvTable ct, const uint16_t* __restrict__ src,
-                               uint16_t* __restrict__ dst) {
+// output's gradient with these weights and mirrored shifts (dx[v][ci] = sum_t
+// sum_co dy[nb(v,-t)][co] w[t][co][ci], added in that order).
+__global__ void k_transpose_weights(ConvTable ct, const uint16_t* __restrict__ src,
+                                    uint16_t* __restrict__ dst) {
   const ConvTable::Entry c = ct.e[blockIdx.y];
   const int e = blockIdx.x * 256 + threadIdx.x, cc = c.Cin * c.Cout;
   if (e >= 27 * cc) return;
   const int t = e / cc, r = e - t * cc, ci = r / c.Cout, co = r - ci * c.Cout;
-  dst[c.w_off + e] = src[c.w_off + (size_t)(26 - t) * cc + (size_t)co * c.Cin + ci];
+  dst[c.w_off + e] = src[c.w_off + (size_t)t * cc + (size_t)co * c.Cin + ci];
 }
 
 // Partial weight gradients: part[chunk][t][co][ci] = sum over the chunk's
@@ -358,9 +376,11 @@ __global__ void k_flip_weights(ConvTable ct, const uint16_t* __restrict__ src,
 // registers over the whole chunk.  A tap outside the grid reads a row of
 // zeros.
 //
-// What bounds it: the LDS reads, 512 bytes for every four k of a tap, and the
-// index arithmetic before each.  Backward pass at 51x91x181, the eight weight
-// gradients: 4183 us with two-byte loads from memory, 560 us so.
+// What bounds it: memory latency of a step, then the LDS reads, 512 bytes for
+// every four k of a tap, and the index arithmetic before each.  So the next
+// step's values are asked for before the taps of this one.  The eight weight
+// gradients of a backward pass at 51x91x181: 4183 us with two-byte loads from
+// memory, 560 us staged step by step, 312 us so.
 // voxels per step: 128, 96 where two workgroups would not fit a CU's LDS
 constexpr int wgrad_step(int cib, int cob) { return cib == 2 && cob == 2 ? 96 : 128; }
 
@@ -394,41 +414,52 @@ __global__ void __launch_bounds__(256)
   if (tid < XQ) sx[9 * kWR * XQ + tid] = u32x4{0u, 0u, 0u, 0u};
   const u32x4* xq = (const u32x4*)x + ci0 / 8;
   const u32x4* yq = (const u32x4*)dy + co0 / 8;
+  // The next step's values, on their way to registers while this one's taps
+  // are added.  Segment r = (dy+1) + 3 (dz+1): voxels v0 - 1 .. v0 + kWV
+  // shifted by it.  Where the shift leaves the grid in y the row is some other
+  // voxel's and not read; in z it is the periodic neighbour's (both are
+  // V-periodic; a grid of few planes can leave the range even so)
+  constexpr int NX = (9 * kWR * XQ + 255) / 256, NY = (kWV * YQ + 255) / 256;
+  u32x4 bx[NX], by[NY];
+  unsigned bf = 0;
+  auto load = [&](int v0) {
+#pragma unroll
+    for (int u = 0; u < NX; u++) {
+      const int e = min(tid + 256 * u, 9 * kWR * XQ - 1);
+      const int r = e / (kWR * XQ), k = e - r * (kWR * XQ);
+      int v = v0 - 1 + d.X * (r % 3 - 1) + XY * (r / 3 - 1) + k / XQ;
+      v = v < 0 ? v + d.V : v;
+      v = v >= d.V ? v - d.V : v;
+      v = max(0, min(v, d.V - 1));
+      bx[u] = xq[(size_t)v * (Cin / 8) + k % XQ];
+    }
+#pragma unroll
+    for (int u = 0; u < NY; u++) {
+      const int e = tid + 256 * u, v = v0 + e / YQ;
+      by[u] = u32x4{0u, 0u, 0u, 0u};
+      if (v < vend && e < kWV * YQ) by[u] = yq[(size_t)v * (Cout / 8) + e % YQ];
+    }
+    const int v = v0 + tid;
+    bf = 0;
+    if (v < vend) {
+      int vx, vy, vz;
+      coords(d, v, vx, vy, vz);
+      const unsigned fx = (vx > 0 ? 1u : 0u) | 2u | (vx < d.X - 1 ? 4u : 0u);
+      bf = (vy > 0 ? fx : 0u) | fx << 3 | (vy < d.Y - 1 ? fx << 6 : 0u);
+    }
+  };
+  if (vbeg < vend) load(vbeg);
   for (int v0 = vbeg; v0 < vend; v0 += kWV) {
     __syncthreads();
-    for (int e = tid; e < kWV * YQ; e += 256) {
-      const int v = v0 + e / YQ;
-      u32x4 w = {0u, 0u, 0u, 0u};
-      if (v < vend) w = yq[(size_t)v * (Cout / 8) + e % YQ];
-      sy[e] = w;
-    }
-    if (tid < kWV) {
-      const int v = v0 + tid;
-      unsigned f = 0;
-      if (v < vend) {
-        int vx, vy, vz;
-        coords(d, v, vx, vy, vz);
-        const unsigned fx = (vx > 0 ? 1u : 0u) | 2u | (vx < d.X - 1 ? 4u : 0u);
-        f = (vy > 0 ? fx : 0u) | fx << 3 | (vy < d.Y - 1 ? fx << 6 : 0u);
-      }
-      flag[tid] = f;
-    }
-    // segment r = (dy+1) + 3 (dz+1): voxels v0 - 1 .. v0 + kWV shifted by it.
-    // Where the shift leaves the grid in y the row is some other voxel's and
-    // not read; in z it is the periodic neighbour's (both are V-periodic)
-#pragma unroll 3
-    for (int r = 0; r < 9; r++) {
-      const int base = v0 - 1 + d.X * (r % 3 - 1) + XY * (r / 3 - 1);
-      for (int e = tid; e < kWR * XQ; e += 256) {
-        int v = base + e / XQ;
-        v = v < 0 ? v + d.V : v;
-        v = v >= d.V ? v - d.V : v;
-        // (a grid of few planes can leave the range even so)
-        v = max(0, min(v, d.V - 1));
-        sx[r * kWR * XQ + e] = xq[(size_t)v * (Cin / 8) + e % XQ];
-      }
-    }
+#pragma unroll
+    for (int u = 0; u < NX; u++)
+      if (tid + 256 * u < 9 * kWR * XQ) sx[tid + 256 * u] = bx[u];
+#pragma unroll
+    for (int u = 0; u < NY; u++)
+      if (tid + 256 * u < kWV * YQ) sy[tid + 256 * u] = by[u];
+    if (tid < kWV) flag[tid] = bf;
     __syncthreads();
+    if (v0 + kWV < vend) load(v0 + kWV);
     const uint16_t* lx = (const uint16_t*)sx;
     const uint16_t* ly = (const uint16_t*)sy;
     const int kr = 4 * kb + (m >> 2), col = (m & 3) * 4;  // this lane's row and part of it
@@ -491,6 +522,7 @@ __global__ void __launch_bounds__(1024)
   const size_t e = (size_t)blockIdx.x * 64 + l;
   float s = 0.f;
   if (e < n)
+#pragma unroll 8
     for (int c = g; c < nchunk; c += 16) s += part[(size_t)c * n + e];
   sh[g][l] = s;
   __syncthreads();
@@ -839,19 +871,19 @@ static void conv(const Dims3& d3, int Cin, int Cout, const uint16_t* x, const ui
 
 void conv_relu(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
                const float* bias, uint16_t* y, const uint16_t* e, uint16_t* sum, hipStream_t s) {
-  conv(d, Cin, Cout, x, w, ConvOut{y, e, sum, nullptr, nullptr, bias, 1}, s);
+  conv(d, Cin, Cout, x, w, ConvOut{y, e, sum, nullptr, nullptr, bias, 1, 1}, s);
 }
 
 void conv_head(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
                const float* bias, float* y1, hipStream_t s) {
-  conv(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0}, s);
+  conv(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0, 1}, s);
 }
 
-void flip_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s) {
+void transpose_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s) {
   size_t most = 0;
   for (int i = 0; i < ct.n; i++)
     most = std::max(most, (size_t)27 * ct.e[i].Cin * ct.e[i].Cout);
-  k_flip_weights<<<dim3(nblk(most, 256), ct.n), 256, 0, s>>>(ct, w, wt);
+  k_transpose_weights<<<dim3(nblk(most, 256), ct.n), 256, 0, s>>>(ct, w, wt);
 }
 
 // Channel blocks of 16 per workgroup of the weight gradient (32 x 32 results
@@ -873,7 +905,9 @@ int wgrad_chunks(const Dims3& d, int Cin, int Cout) {
 void conv_bwd(const Dims3& d3, int Cin, int Cout, const uint16_t* dy, const uint16_t* x,
               const uint16_t* wt, float* dx, float* gw, float* part, hipStream_t s) {
   const Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
-  if (dx) conv(d3, Cout, Cin, dy, wt, ConvOut{nullptr, nullptr, nullptr, dx, nullptr, nullptr, 0}, s);
+  if (dx)
+    conv(d3, Cout, Cin, dy, wt,
+         ConvOut{nullptr, nullptr, nullptr, dx, nullptr, nullptr, 0, -1}, s);
   const int nc = wgrad_chunks(d3, Cin, Cout);
   const int bi = wgrad_block(Cin), bo = wgrad_block(Cout), wv = wgrad_step(bi, bo);
   const int steps = (d.V + wv - 1) / wv, chunk = (steps + nc - 1) / nc * wv;
