@@ -121,8 +121,8 @@ KERNELS = [
     ("pcg_iteration_fp64 (graph replay)", 3, 106, 8),
     ("stencil_fp64 (k_stencil_lds<double>)", 0, 8, 8),
     ("stencil_fp32 (k_stencil_lds<float>)", 1, 4, 4),
-    ("ilu_apply_fp64 (k_tile_fwd+k_tile_bwd<double>)", 2, 32, 0),
-    ("ilu_apply_fp32 (k_tile_fwd+k_tile_bwd<float>)", 7, 24, 0),
+    ("ilu_apply_fp64 (k_col_fwd+k_col_bwd<double>)", 2, 32, 0),
+    ("ilu_apply_fp32 (column or tile sweeps, float)", 7, 24, 0),
     # r, ap read, r written (runs where the sweeps do not take it)
     ("cg_update_fp64 (k_cg_update<double>)", 4, 24, 0),
     # p, z read, p written, and the solution once per 4 iterations:
