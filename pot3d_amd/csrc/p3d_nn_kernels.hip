@@ -73,6 +73,7 @@ __device__ __forceinline__ void coords(const Dims& d, int v, int& x, int& y, int
 // One wave: MT x 16 voxels times NB x 16 output channels; grid (voxels / (64
 // MT), Cout / (16 NB)), block 256.  The weights are the MFMA's A operand and
 // the voxels its B operand, so a lane ends with four channels of one voxel.
+// DIR -1 mirrors the taps' shifts (input gradients).
 // K runs over 32 channels of a tap; with 16 channels over two taps at a time
 // (lanes 0-31 the even, 32-63 the odd one; the 28th tap is empty).
 //
@@ -90,7 +91,6 @@ struct ConvOut {
   float* y1;          // FP32 result, channel 0 alone, or null
   const float* bias;  // or null
   int relu;
-  int dir;            // 1, or -1: the taps' shifts mirrored (input gradients)
 };
 
 // The results of a wave: four channels of a voxel per lane and tile.
@@ -128,7 +128,7 @@ __device__ __forceinline__ void conv_store(const Dims& d, int Cout, const ConvOu
   }
 }
 
-template <int CIN, int NB, int MT>
+template <int CIN, int NB, int MT, int DIR>
 __global__ void __launch_bounds__(256)
     k_conv(Dims d, int Cout, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
            ConvOut o) {
@@ -145,8 +145,8 @@ __global__ void __launch_bounds__(256)
   constexpr unsigned kQ = CIN / 8;  // 16-byte words of a voxel
   const u32x4* xq = (const u32x4*)x - kZeroFront / 16;
   const unsigned lane_q = kZeroFront / 16 + (CIN == 16 ? (unsigned)(kb & 1) : (unsigned)kb);
-  const bool fw = o.dir > 0;
-  const unsigned XQ = (unsigned)o.dir * kQ * (unsigned)d.X, PQ = kQ * (unsigned)d.X * (unsigned)d.Y;
+  constexpr bool fw = DIR > 0;
+  const unsigned XQ = (unsigned)DIR * kQ * (unsigned)d.X, PQ = kQ * (unsigned)d.X * (unsigned)d.Y;
   unsigned base[MT], zlo[MT], zhi[MT];
   bool in[MT], xm[MT], xp[MT], ym[MT], yp[MT];
 #pragma unroll
@@ -173,7 +173,7 @@ __global__ void __launch_bounds__(256)
   };
   auto tap_off = [&](int q, int t) {
     const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9;
-    return (unsigned)(dx * o.dir * (int)kQ) + (unsigned)dy * XQ +
+    return (unsigned)(dx * DIR * (int)kQ) + (unsigned)dy * XQ +
            (dz == 0 ? zlo[q] : (dz == 2 ? zhi[q] : 0u));
   };
   f32x4 acc[NB][MT];
@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256)
         unsigned idx[MT];
 #pragma unroll
         for (int t = 0; t < MT; t++)
-          idx[t] = tap_ok(t, r) ? bz[t] + (unsigned)((r % 3 - 1) * o.dir * (int)kQ) +
+          idx[t] = tap_ok(t, r) ? bz[t] + (unsigned)((r % 3 - 1) * DIR * (int)kQ) +
                                       (unsigned)(r / 3 - 1) * XQ
                                 : lane_q - kZeroFront / 16;
 #pragma unroll
@@ -259,7 +259,7 @@ __device__ __forceinline__ int lds_word(int row, int w) {
 
 __host__ __device__ inline int conv_lds_rows(int MT, int X) { return 64 * MT + 2 * X + 2; }
 
-template <int CIN, int NB, int MT>
+template <int CIN, int NB, int MT, int DIR>
 __global__ void __launch_bounds__(256)
     k_conv_lds(Dims d, int Cout, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                ConvOut o) {
@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(256)
     if (v < d.V) {
       int vx, vy, vz;
       coords(d, v, vx, vy, vz);
-      const bool fw = o.dir > 0;
+      constexpr bool fw = DIR > 0;
       const unsigned fx = (vx > 0 ? (fw ? 1u : 4u) : 0u) | 2u |
                           (vx < d.X - 1 ? (fw ? 4u : 1u) : 0u);
       ok[t] = (vy > 0 ? fx << (fw ? 0 : 6) : 0u) | fx << 3 |
@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(256)
     // rows vb - X - 1 + XY (dz - 1) on (mirrored: 1 - dz): where they leave the plane or the
     // grid in x or y no tap reads them; in z they are V-periodic (a grid of
     // few planes can leave the range even so)
-    const int base = vb - d.X - 1 + XY * (dz - 1) * o.dir;
+    const int base = vb - d.X - 1 + XY * (dz - 1) * DIR;
     // six loads of a thread in flight at a time
     constexpr int kB = 6;
     for (int e0 = tid; e0 < rows * Q; e0 += 256 * kB) {
@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(256)
     const u32x4* wz = wq + wt * (size_t)(9 * dz);
 #pragma unroll
     for (int r = 0; r < 9; r++) {
-      const int shift = d.X + 1 + ((r % 3 - 1) + (r / 3 - 1) * d.X) * o.dir;
+      const int shift = d.X + 1 + ((r % 3 - 1) + (r / 3 - 1) * d.X) * DIR;
       int row[MT];
 #pragma unroll
       for (int t = 0; t < MT; t++)
@@ -820,7 +820,7 @@ __global__ void k_mfma_check(const uint16_t* __restrict__ A, const uint16_t* __r
 // host launchers
 static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-template <int CIN, int NB, int MT>
+template <int DIR, int CIN, int NB, int MT>
 static void conv_launch(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
                         const ConvOut& o, hipStream_t s) {
   const dim3 grid(nblk(d.V, 64 * MT), Cout / (16 * NB));
@@ -828,55 +828,56 @@ static void conv_launch(const Dims& d, int Cout, const uint16_t* x, const uint16
     // three workgroups per CU, or the r axis is too long for whole rows
     const size_t lds = (size_t)(conv_lds_rows(MT, d.X) + 1) * CIN * 2;
     if (lds <= 52 * 1024) {
-      k_conv_lds<CIN, NB, MT><<<grid, 256, lds, s>>>(d, Cout, x, w, o);
+      k_conv_lds<CIN, NB, MT, DIR><<<grid, 256, lds, s>>>(d, Cout, x, w, o);
       return;
     }
   }
-  k_conv<CIN, NB, MT><<<grid, 256, 0, s>>>(d, Cout, x, w, o);
+  k_conv<CIN, NB, MT, DIR><<<grid, 256, 0, s>>>(d, Cout, x, w, o);
 }
 
-template <int CIN, int NB>
+template <int DIR, int CIN, int NB>
 static void conv_mt(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
                     const ConvOut& o, hipStream_t s) {
   // tiles per wave: as many as leave a few waves to every SIMD (1024 of them)
   if (d.V >= 200000)
-    conv_launch<CIN, NB, 4>(d, Cout, x, w, o, s);
+    conv_launch<DIR, CIN, NB, 4>(d, Cout, x, w, o, s);
   else if (d.V >= 50000)
-    conv_launch<CIN, NB, 2>(d, Cout, x, w, o, s);
+    conv_launch<DIR, CIN, NB, 2>(d, Cout, x, w, o, s);
   else
-    conv_launch<CIN, NB, 1>(d, Cout, x, w, o, s);
+    conv_launch<DIR, CIN, NB, 1>(d, Cout, x, w, o, s);
 }
 
-template <int CIN>
+template <int DIR, int CIN>
 static void conv_nb(const Dims& d, int Cout, const uint16_t* x, const uint16_t* w,
                     const ConvOut& o, hipStream_t s) {
   if (Cout % 32 == 0 && d.V >= 10000)
-    conv_mt<CIN, 2>(d, Cout, x, w, o, s);
+    conv_mt<DIR, CIN, 2>(d, Cout, x, w, o, s);
   else
-    conv_mt<CIN, 1>(d, Cout, x, w, o, s);
+    conv_mt<DIR, CIN, 1>(d, Cout, x, w, o, s);
 }
 
+template <int DIR>
 static void conv(const Dims3& d3, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
                  const ConvOut& o, hipStream_t s) {
   const Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
   if (Cin == 16)
-    conv_nb<16>(d, Cout, x, w, o, s);
+    conv_nb<DIR, 16>(d, Cout, x, w, o, s);
   else if (Cin == 32)
-    conv_nb<32>(d, Cout, x, w, o, s);
+    conv_nb<DIR, 32>(d, Cout, x, w, o, s);
   else if (Cin == 64)
-    conv_nb<64>(d, Cout, x, w, o, s);
+    conv_nb<DIR, 64>(d, Cout, x, w, o, s);
   else
-    conv_nb<128>(d, Cout, x, w, o, s);
+    conv_nb<DIR, 128>(d, Cout, x, w, o, s);
 }
 
 void conv_relu(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
                const float* bias, uint16_t* y, const uint16_t* e, uint16_t* sum, hipStream_t s) {
-  conv(d, Cin, Cout, x, w, ConvOut{y, e, sum, nullptr, nullptr, bias, 1, 1}, s);
+  conv<1>(d, Cin, Cout, x, w, ConvOut{y, e, sum, nullptr, nullptr, bias, 1}, s);
 }
 
 void conv_head(const Dims3& d, int Cin, int Cout, const uint16_t* x, const uint16_t* w,
                const float* bias, float* y1, hipStream_t s) {
-  conv(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0, 1}, s);
+  conv<1>(d, Cin, Cout, x, w, ConvOut{nullptr, nullptr, nullptr, nullptr, y1, bias, 0}, s);
 }
 
 void transpose_weights(const ConvTable& ct, const uint16_t* w, uint16_t* wt, hipStream_t s) {
@@ -906,8 +907,8 @@ void conv_bwd(const Dims3& d3, int Cin, int Cout, const uint16_t* dy, const uint
               const uint16_t* wt, float* dx, float* gw, float* part, hipStream_t s) {
   const Dims d{d3.X, d3.Y, d3.Z, d3.X * d3.Y * d3.Z};
   if (dx)
-    conv(d3, Cout, Cin, dy, wt,
-         ConvOut{nullptr, nullptr, nullptr, dx, nullptr, nullptr, 0, -1}, s);
+    conv<-1>(d3, Cout, Cin, dy, wt,
+             ConvOut{nullptr, nullptr, nullptr, dx, nullptr, nullptr, 0}, s);
   const int nc = wgrad_chunks(d3, Cin, Cout);
   const int bi = wgrad_block(Cin), bo = wgrad_block(Cout), wv = wgrad_step(bi, bo);
   const int steps = (d.V + wv - 1) / wv, chunk = (steps + nc - 1) / nc * wv;
