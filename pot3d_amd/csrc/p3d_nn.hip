@@ -298,7 +298,7 @@ int p3d_nn_create(p3d_nn** out, int nr, int nt, int np, const double* rh, unsign
                {&n->g_s1, V1 * 32}, {&n->g_u1, V1 * 64}, {&n->g_s2, V2 * 64},
                {&n->g_u2, V2 * 128}, {&n->g_e3, V3 * 128}, {&n->g_p3, V3 * 64},
                {&n->g_p2, V2 * 32}, {&n->g_p1, V1 * 16}, {&n->tgt, V0},
-               {(float**)&n->x64, V0 * 2}, {&n->lpart, kSumBlocks},
+               {(float**)&n->x64, V0 * 2}, {&n->lpart, V0 / 256 + 1},
                {&n->bpart, kSumBlocks * 128}, {&n->loss, 4}};
   for (auto& a : grads)
     if ((rc = dmalloc(n, (void**)a.p, a.n * 4))) {

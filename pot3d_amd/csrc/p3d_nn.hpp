@@ -51,8 +51,8 @@ constexpr int kSumBlocks = 1024;
 void relu_bwd(const Dims3& f, const Dims3& c, int C, const uint16_t* y, const float* ga,
               const float* gp, uint16_t* dy, float* bpart, float* gb, hipStream_t s);
 // loss = mean (out - t)^2, t = tgt or tgt64 / tscale, its BF16 gradient for the
-// head's 16 channels and their bias gradient gb; part: kSumBlocks, bpart:
-// 16*kSumBlocks
+// head's 16 channels and their bias gradient gb; part: one per 256 voxels,
+// bpart: 16*kSumBlocks
 void mse(int V, const float* out, const float* tgt, const double* tgt64, double tscale,
          uint16_t* dy, float* part, float* bpart, float* loss, float* gb, hipStream_t s);
 void adam(size_t n, float* w, const float* g, float* m1, float* m2, float lr, float b1,

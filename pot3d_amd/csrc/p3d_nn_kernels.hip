@@ -656,49 +656,84 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// sum of 256 values, one per thread (fixed order); result in thread 0
+// sum of 256 values, one per thread, pairing those 128, 64, ... 1 apart; result
+// in thread 0.  sh: 256 floats that no other sum since the last barrier used.
 __device__ __forceinline__ float block_sum(float v, float* sh) {
+  const int t = (int)threadIdx.x;
+  sh[t] = v;
   __syncthreads();
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
+  float s = 0.f;
+  if (t < 64) {
+    s = (sh[t] + sh[t + 128]) + (sh[t + 64] + sh[t + 192]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
   }
-  return sh[0];
+  return s;
 }
 
 // L = mean_v (out[v] - t[v])^2 (out FP32, the head's channel 0; its other 15
-// channels have no gradient): part[block] the loss's partial sums, bpart
+// channels have no gradient): part the loss's partial sums, one per 256
+// consecutive voxels whatever the grid of blocks (k_sum_in_order), bpart
 // [block][16] those of the head's bias gradient, dy the gradient as BF16
 // operand.  An FP64 target is divided by its scale here.
 __global__ void __launch_bounds__(256)
     k_mse(int V, const float* __restrict__ out, const float* __restrict__ tgt,
           const double* __restrict__ tgt64, double tscale, uint16_t* __restrict__ dy,
           float* __restrict__ part, float* __restrict__ bpart) {
-  __shared__ float sh[256];
-  float l = 0.f, g = 0.f;
-  for (int v = blockIdx.x * 256 + threadIdx.x; v < V; v += gridDim.x * 256) {
-    const float dlt = out[v] - (tgt64 ? (float)(tgt64[v] / tscale) : tgt[v]);
-    const float gv = 2.f * dlt / (float)V;
-    l += dlt * dlt;
-    g += gv;
-    u32x4* o = (u32x4*)(dy + (size_t)v * 16);
-    o[0] = u32x4{(unsigned)f2bf(gv), 0u, 0u, 0u};
-    o[1] = u32x4{0u, 0u, 0u, 0u};
+  __shared__ float sh[3][256];
+  const int groups = (V + 255) / 256;
+  float g = 0.f;
+  int b = 0;
+  for (int q = blockIdx.x; q < groups; q += gridDim.x, b ^= 1) {
+    const int v = q * 256 + (int)threadIdx.x;
+    float l = 0.f;
+    if (v < V) {
+      const float dlt = out[v] - (tgt64 ? (float)(tgt64[v] / tscale) : tgt[v]);
+      const float gv = 2.f * dlt / (float)V;
+      l = dlt * dlt;
+      g += gv;
+      u32x4* o = (u32x4*)(dy + (size_t)v * 16);
+      o[0] = u32x4{(unsigned)f2bf(gv), 0u, 0u, 0u};
+      o[1] = u32x4{0u, 0u, 0u, 0u};
+    }
+    const float ls = block_sum(l, sh[b]);
+    if (threadIdx.x == 0) part[q] = ls;
   }
-  const float ls = block_sum(l, sh), gs = block_sum(g, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = ls;
+  const float gs = block_sum(g, sh[2]);
   if (threadIdx.x < 16) bpart[blockIdx.x * 16 + threadIdx.x] = threadIdx.x == 0 ? gs : 0.f;
 }
 
-// *out = scale * sum of part[0..n)
+// *out = scale * (part[0] + part[1] + ... in this order).  The loss is this sum
+// over its groups of 256 voxels, so its order belongs to the result (a tree
+// over 1024 blocks' sums moved it by up to 2e-6 of itself).  One lane adds, out
+// of LDS, what all have loaded: one load after the other from memory took 141
+// us for the 3050 groups of 51x91x181.
 __global__ void __launch_bounds__(256)
-    k_sum(int n, const float* __restrict__ part, float* __restrict__ out, float scale) {
-  __shared__ float sh[256];
+    k_sum_in_order(int n, const float* __restrict__ part, float* __restrict__ out, float scale) {
+  constexpr int kC = 4096;
+  __shared__ f32x4 sh[kC / 4];
   float s = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
-  s = block_sum(s, sh);
+  for (int n0 = 0; n0 < n; n0 += kC) {
+#pragma unroll
+    for (int u = 0; u < kC; u += 256) {
+      const int i = n0 + u + (int)threadIdx.x;
+      ((float*)sh)[u + threadIdx.x] = i < n ? part[i] : 0.f;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int m = min(kC, n - n0), m4 = m / 4;
+#pragma unroll 8
+      for (int e = 0; e < m4; e++) {
+        const f32x4 v = sh[e];
+        s += v[0];
+        s += v[1];
+        s += v[2];
+        s += v[3];
+      }
+      for (int e = 4 * m4; e < m; e++) s += ((const float*)sh)[e];
+    }
+    __syncthreads();
+  }
   if (threadIdx.x == 0) *out = s * scale;
 }
 
@@ -954,7 +989,7 @@ void mse(int V, const float* out, const float* tgt, const double* tgt64, double 
          uint16_t* dy, float* part, float* bpart, float* loss, float* gb, hipStream_t s) {
   const unsigned nb = sum_blocks(V);
   k_mse<<<nb, 256, 0, s>>>(V, out, tgt, tgt64, tscale, dy, part, bpart);
-  k_sum<<<1, 256, 0, s>>>((int)nb, part, loss, 1.0f / (float)V);
+  k_sum_in_order<<<1, 256, 0, s>>>((V + 255) / 256, part, loss, 1.0f / (float)V);
   k_reduce_chunks<<<1, 1024, 0, s>>>((int)nb, 16, bpart, gb);
 }
 void adam(size_t n, float* w, const float* g, float* m1, float* m2, float lr, float b1,
