@@ -225,6 +225,22 @@ __device__ __forceinline__ int st_load_int(const int* f) {
 __device__ __forceinline__ double st_load(const double* f) {
   return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// What the epilogues read of the state, all loads under way together.
+__device__ __forceinline__ CgState st_snapshot(const CgState* st) {
+  CgState c;
+  c.bdotb = st_load(&st->bdotb);
+  c.rdotr = st_load(&st->rdotr);
+  c.rdotr_old = st_load(&st->rdotr_old);
+  c.rr = st_load(&st->rr);
+  c.bb = st_load(&st->bb);
+  c.epscg = st_load(&st->epscg);
+  c.hist = __hip_atomic_load(&st->hist, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  c.hist_cap = st_load_int(&st->hist_cap);
+  c.ncg = st_load_int(&st->ncg);
+  c.ncgmax = st_load_int(&st->ncgmax);
+  c.stop_mode = st_load_int(&st->stop_mode);
+  return c;
+}
 
 // Reduction slots used by the "last block finishes" pattern.
 struct Reduce {

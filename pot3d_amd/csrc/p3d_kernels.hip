@@ -140,7 +140,7 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
   __syncthreads();
   CgState c;  // for the epilogue, loaded while the count-in is under way
   if (threadIdx.x == 0) {
-    if (st) c = *st;
+    if (st) c = st_snapshot(st);
 #pragma unroll
     for (int q = 0; q < NV; q++) {
       double s = 0.0;
