@@ -21,9 +21,11 @@
 // for columns of lower workgroup number.  Workgroups start in that order on
 // every XCD, so the lowest unfinished one is always running or next to run
 // and never waits for one that is not.  Only other kernels that wait
-// themselves could keep it from starting; every wait is bounded (kSpinMax
-// polls, then a flag that ends all other waits), and the solver starts the
-// call over with the tile schedules.
+// themselves could keep it from starting; every wait is bounded (kPolls polls,
+// then a flag that ends all other waits), and the solver starts the call over
+// with the tile schedules.  P3D_COLUMN_POLLS in the environment sets another
+// bound for the plans built from then on (0: a wait gives up once it has
+// polled in vain), so that this path can be tested.
 //
 // Per-point arithmetic and order are those of p3d_sweep.hip: the same bits.
 //
@@ -35,6 +37,8 @@
 // What bounds it: the chain, as above.  One call of the drop-in interface,
 // tiles and columns: 333 and 85 us at 20x31x60, 1429 and 167 us at 51x91x181,
 // 3448 and 368 us at 101x181x361, 7.06 and 0.87 ms at 151x301x601.
+#include <stdlib.h>
+
 #include <type_traits>
 #include <vector>
 
@@ -54,7 +58,7 @@ constexpr int kDelay = 7 + 7 * kJ;       // steps between a column's first and l
 constexpr int kFront = kCS;              // rows before row 0 of dinv_s and y_s
 constexpr int kRing = 64;                // steps whose values a column holds in LDS
 constexpr int kThreads = 256;            // four waves: march, in, out, faces
-constexpr unsigned kSpinMax = 1u << 20;  // polls of one wait (about a second)
+constexpr unsigned kPolls = 1u << 20;    // polls of one wait (about a second)
 
 #define P3D_DPP(v, ctrl) __builtin_amdgcn_mov_dpp((v), (ctrl), 0xf, 0xf, true)
 
@@ -305,7 +309,7 @@ __device__ __forceinline__ void faces(const ColArgs& ca, const ColCtx& x, ColLds
   const u64* pi = ca.face_i + (has_i ? x.col + d : x.col) * fs + (kCU + 7) * 8 + x.lane;
   const u64* pj = ca.face_j + (has_j ? x.col + d * ca.NI : x.col) * fs + (kCU + 7 * kJ) * 8 + x.lane;
   const unsigned mi = has_i ? ~0u : 0u, mj = has_j ? ~0u : 0u, stamp = x.stamp;
-  unsigned* abort = ca.ctr + 2;
+  unsigned* abort = ca.failed;
   bool dead = false;
   u64 wi[kCP], wj[kCP];
   auto load = [&](int p, int n) {
@@ -324,8 +328,8 @@ __device__ __forceinline__ void faces(const ColArgs& ca, const ColCtx& x, ColLds
         // this chunk and the next ones, which were asked for even earlier
 #pragma unroll
         for (int q = 0; q < kFP; q++) load((p + q) % kCP, n + q);
-        if ((++spins & 1023u) == 0) {
-          const bool stop = spins >= kSpinMax;
+        const bool stop = ++spins >= ca.polls;
+        if (stop || (spins & 1023u) == 0) {
           if (stop && x.lane == 0)
             __hip_atomic_store(abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           if (stop || __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -786,8 +790,11 @@ namespace {
 // What both kinds of plan share: the columns and steps of the grid, and the
 // device memory that does not depend on where the couplings come from.
 // Returns 0, or 1 when a buffer cannot be had (the caller frees the plan).
-int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int planes) {
+int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int planes,
+                 unsigned* failed) {
   ColArgs& ca = plan.a;
+  const char* polls = getenv("P3D_COLUMN_POLLS");
+  ca.polls = polls ? (unsigned)strtoul(polls, nullptr, 10) : kPolls;
   ca.NI = (g.a + 7) / 8;
   ca.NJ = (g.b + 7) / 8;
   ca.c = g.c;
@@ -825,6 +832,7 @@ int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int plan
   ca.face_i = plan.face;
   ca.face_j = plan.face + nf;
   ca.ctr = plan.ctr;
+  ca.failed = failed ? failed : plan.ctr + 2;
   ca.dummy = plan.dummy;
   return ok ? 0 : 1;
 }
@@ -838,7 +846,7 @@ int no_plan(ColumnPlan& plan) {
 }  // namespace
 
 int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
-                      int tk_log2, const float* dinv) {
+                      int tk_log2, const float* dinv, unsigned* failed) {
   free_column_plan(plan);
   ColArgs& ca = plan.a;
   ca.tk_log2 = tk_log2;
@@ -860,7 +868,7 @@ int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const I
   ca.mode = !uniform ? kPhiAny : (bl.bk < g.c ? kPhiCut : kPhiUniform);
   ca.u_d = dph[0];
   ca.u_k = dpl[0];
-  if (plan_columns(plan, g, bl, planes) != 0) return no_plan(plan);
+  if (plan_columns(plan, g, bl, planes, failed) != 0) return no_plan(plan);
   if (col_lds(ca) > kColLdsMax) return no_plan(plan);
   std::vector<float2> lo(ca.pf_n, make_float2(0.f, 0.f)), up(lo);
   for (int k = 0; k < g.c; k++) {
@@ -893,7 +901,7 @@ int build_column_plan_stored(ColumnPlan& plan, const Grid3& g, const CoefArrays&
   free_column_plan(plan);
   ColArgs& ca = plan.a;
   ca.mode = kStored;
-  if (plan_columns(plan, g, IluBlocks{g.a, g.b, g.c, wrap ? 1 : 0}, g.c) != 0)
+  if (plan_columns(plan, g, IluBlocks{g.a, g.b, g.c, wrap ? 1 : 0}, g.c, nullptr) != 0)
     return no_plan(plan);
   const int steps = ca.rounds * kCS;
   const size_t n = (size_t)ca.NI * ca.NJ * steps * 64;

@@ -32,7 +32,9 @@ struct ColArgs {
   // backward march, and those of the phi wrap (a x b)
   const float4 *lo_s = nullptr, *up_s = nullptr;
   const float *wrap_lo = nullptr, *wrap_up = nullptr;
-  unsigned* ctr = nullptr;        // stamps of the next forward, backward sweep; failure flag
+  unsigned* ctr = nullptr;        // stamps of the next forward, backward sweep
+  unsigned* failed = nullptr;     // set once a wait ran into its bound
+  unsigned polls = 0;             // that bound
   void* dummy = nullptr;          // where rows outside the vectors are stored
 };
 
@@ -49,10 +51,12 @@ struct ColumnPlan {
 };
 
 // dinv: the D-ILU's inverse pivots in natural order; tk_log2: planes per
-// tile of the r and z placement.  Returns 0 when the sweeps can run.
+// tile of the r and z placement; failed: device word that is set once a wait
+// runs into its bound.  Returns 0 when the sweeps can run.
 int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
-                      int tk_log2, const float* dinv);
-// The same with stored couplings; co's wrap planes have to outlive the plan.
+                      int tk_log2, const float* dinv, unsigned* failed);
+// The same with stored couplings; co's wrap planes have to outlive the plan,
+// whose word column_failure_flag is.
 int build_column_plan_stored(ColumnPlan& plan, const Grid3& g, const CoefArrays& co, bool wrap,
                              const float* dinv);
 void free_column_plan(ColumnPlan& plan);
@@ -68,7 +72,8 @@ void launch_dilu_columns(const ColumnPlan& plan, const Metric& m, const Grid3& g
 void launch_dilu_columns_stored(const ColumnPlan& plan, const Grid3& g, double* x, float* r32,
                                 hipStream_t s);
 
-// Device word that is not 0 once a wait of a column sweep ran into its bound.
+// The plan's own device word, not 0 once a wait of its sweeps ran into its bound
+// (build_column_plan_stored).
 const unsigned* column_failure_flag(const ColumnPlan& plan);
 
 }  // namespace p3d

@@ -203,6 +203,7 @@ struct CgState {
   // the current group, and the buffer holding the current search direction
   double alpha_hist[4];
   int p_cur;
+  unsigned col_failed;  // a wait of a column sweep ran into its bound
 };
 
 // Iterations per update of the FP64 solution (the p update's group; directions of a group live in kXBatch rotating buffers).

@@ -394,6 +394,9 @@ void external_lu_solver(double* x) {
       // a wait ran into its bound: x as it was (in the FP32 that the sweeps
       // work in), and from now on the tiles
       free_column_plan(G.col);
+      fprintf(stderr, " external_lu_solver: column sweeps: a wait ran into its bound; tile "
+                      "schedules from here on\n");
+      fflush(stderr);
       k_widen<<<(unsigned)(((size_t)G.N + 255) / 256), 256, 0, G.stream>>>(G.yv, dx, (size_t)G.N);
       trisolve_tiles(dx);
     }

@@ -142,6 +142,14 @@ static int dalloc(void** p, size_t bytes) {
   return P3D_OK;
 }
 
+// Captured iterations hold the launches of the options they were captured with.
+static void drop_graphs(p3d_solver* s) {
+  for (int q = 0; q < 3; q++) {
+    if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
+    s->gexec[q] = nullptr;
+  }
+}
+
 template <typename A, typename B>
 __global__ void k_convert(uint32_t n, const A* __restrict__ src, B* __restrict__ dst) {
   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -230,10 +238,7 @@ static int update_tilemap(p3d_solver* s) {
   if (t.on == s->tm.on && t.TNI == s->tm.TNI && t.TNJ == s->tm.TNJ && t.tk_log2 == s->tm.tk_log2)
     return P3D_OK;
   HIPCHK(hipStreamSynchronize(s->stream));
-  for (int q = 0; q < 3; q++) {
-    if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-    s->gexec[q] = nullptr;
-  }
+  drop_graphs(s);
   s->tm = t;
   if (t.on) {
     int dev = 0, ncu = 0;
@@ -268,10 +273,28 @@ static int ensure_hist(p3d_solver* s, int ncgmax) {
   return P3D_OK;
 }
 
+// Waits for the stream and copies the control state to the host.  A column
+// sweep that gave up waiting leaves its mark there: what the call computed
+// since it last looked is void, whatever the rest of the state says, and it
+// starts over with the tile schedules (kStartOver; the vectors' entries outside
+// the grid are zero again).  So every read of the state after a sweep, and
+// before anything is made of its results, is this one.
+static constexpr int kStartOver = -1;
 static int read_state(p3d_solver* s) {
   HIPCHK(hipMemcpyAsync(s->st_host, s->st, sizeof(CgState), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
-  return P3D_OK;
+  if (!s->st_host->col_failed) return P3D_OK;
+  drop_graphs(s);
+  free_column_plan(s->col);
+  s->st_host->col_failed = 0;
+  HIPCHK(hipMemsetAsync(&s->st->col_failed, 0, sizeof(unsigned), s->stream));
+  for (double* v : {s->r, s->z, s->ap})
+    HIPCHK(hipMemsetAsync(v, 0, s->nvec * sizeof(double), s->stream));
+  for (float* v : {s->r32, s->z32, s->ap32})
+    if (v) HIPCHK(hipMemsetAsync(v, 0, s->nvec * sizeof(float), s->stream));
+  fprintf(stderr, "[p3d] column sweeps: a wait ran into its bound; tile schedules from here on\n");
+  fflush(stderr);
+  return kStartOver;
 }
 
 // ---------------------------------------------------------------------------
@@ -301,7 +324,7 @@ static bool columns_on(const p3d_solver* s) { return columns_wanted(s) && s->col
 static void ensure_columns(p3d_solver* s) {
   if (!columns_wanted(s) || s->col_tried) return;
   s->col_tried = true;
-  build_column_plan(s->col, s->m, s->g, s->blocks, s->tm.tk_log2, s->dinv);
+  build_column_plan(s->col, s->m, s->g, s->blocks, s->tm.tk_log2, s->dinv, &s->st->col_failed);
 }
 
 // Whether the FP32 ILU apply can take the residual update (see cg_iteration).
@@ -509,28 +532,6 @@ static void print_history(p3d_solver* s, int ncghist) {
   fflush(stdout);
 }
 
-// Whether a column sweep gave up waiting (two threads' sweeps that crowd each
-// other out of the device can do that): its results are void, and the call
-// starts over with the tile schedules (kStartOver).  copy_column_flag goes with the other copies of a
-// result to the host, check_columns after the stream has been waited for.
-static constexpr int kStartOver = -1;
-static void copy_column_flag(p3d_solver* s) {
-  unsigned* f = (unsigned*)(s->out_host + 6);
-  *f = 0;
-  if (columns_on(s))
-    (void)hipMemcpyAsync(f, column_failure_flag(s->col), sizeof *f, hipMemcpyDeviceToHost,
-                         s->stream);
-}
-static int check_columns(p3d_solver* s) {
-  if (*(const unsigned*)(s->out_host + 6) == 0) return P3D_OK;
-  for (int q = 0; q < 3; q++) {
-    if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-    s->gexec[q] = nullptr;
-  }
-  free_column_plan(s->col);
-  return kStartOver;
-}
-
 static int true_residual(p3d_solver* s, double* rr, double* bb) {
   // ap = b - A x (FP64), reductions into out[0] (r.r), out[2] (b.b)
   launch_pole_sums<double>(s->m, s->g, s->x, s->pole_part, s->stream);
@@ -540,11 +541,10 @@ static int true_residual(p3d_solver* s, double* rr, double* bb) {
                       s->out + 2, false, s->stream);
   HIPCHK(hipMemcpyAsync(s->out_host, s->out, 4 * sizeof(double), hipMemcpyDeviceToHost,
                         s->stream));
-  copy_column_flag(s);
   HIPCHK(hipStreamSynchronize(s->stream));
   *rr = s->out_host[0];
   *bb = s->out_host[2];
-  return check_columns(s);
+  return P3D_OK;
 }
 
 static int status_rc(int done) {
@@ -844,8 +844,7 @@ const char* p3d_last_error(void) { return g_err.c_str(); }
 int p3d_destroy(p3d_solver* s) {
   if (!s) return P3D_OK;
   if (s->stream) hipStreamSynchronize(s->stream);
-  for (int t = 0; t < 3; t++)
-    if (s->gexec[t]) hipGraphExecDestroy(s->gexec[t]);
+  drop_graphs(s);
   void* bufs[] = {s->tables, s->ftables, s->mesh, s->br0, s->br1, s->x, s->r, s->p, s->ap, s->z, s->b,
                   s->yv, s->dinv, s->x32, s->r32, s->p32, s->ap32, s->z32, s->pole_part,
                   s->st, s->hist, s->red.partial, s->red.counter, s->out, s->phi, s->sums,
@@ -1033,6 +1032,7 @@ int p3d_create(p3d_solver** out, int nr, int nt, int np, const double* r, const 
   if ((rc = dalloc((void**)&s->br0, sizeof(double) * nt * np))) return bail(rc);
   if ((rc = dalloc((void**)&s->pole_part, sizeof(double) * 2 * kPoleSegs * a))) return bail(rc);
   if ((rc = dalloc((void**)&s->st, sizeof(CgState)))) return bail(rc);
+  hipMemset(s->st, 0, sizeof(CgState));
   if (hipHostMalloc((void**)&s->st_host, sizeof(CgState), 0) != hipSuccess)
     return bail(fail(P3D_ENOMEM, "hipHostMalloc failed"));
   if (hipHostMalloc((void**)&s->out_host, 8 * sizeof(double), 0) != hipSuccess)
@@ -1117,10 +1117,7 @@ static IluBlocks ilu_blocks(const p3d_solver* s) {
 static int rebuild_ilu(p3d_solver* s, bool refactor) {
   HIPCHK(hipStreamSynchronize(s->stream));
   drop_columns(s);
-  for (int t = 0; t < 3; t++) {
-    if (s->gexec[t]) hipGraphExecDestroy(s->gexec[t]);
-    s->gexec[t] = nullptr;
-  }
+  drop_graphs(s);
   if (refactor) {
     s->blocks = ilu_blocks(s);
     const int rc = factor_ilu(s);
@@ -1168,10 +1165,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       if (value != 0 && value != 1)
         return fail(P3D_EINVAL, "P3D_OPT_SWEEP must be 0 or 1");
       s->sweep_mode = (int)value;
-      for (int t = 0; t < 3; t++) {
-        if (s->gexec[t]) hipGraphExecDestroy(s->gexec[t]);
-        s->gexec[t] = nullptr;
-      }
+      drop_graphs(s);
       return update_tilemap(s);
     case P3D_OPT_VERBOSE:
       s->verbose = value != 0;
@@ -1183,10 +1177,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       if (v != s->L.stencil) {
         // captured iterations hold the other kernel
         HIPCHK(hipStreamSynchronize(s->stream));
-        for (int q = 0; q < 3; q++) {
-          if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-          s->gexec[q] = nullptr;
-        }
+        drop_graphs(s);
         s->L.stencil = v;
       }
       break;
@@ -1200,10 +1191,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       if (v != s->fuse_rupd) {
         // captured iterations hold the other kernel sequence
         HIPCHK(hipStreamSynchronize(s->stream));
-        for (int q = 0; q < 3; q++) {
-          if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-          s->gexec[q] = nullptr;
-        }
+        drop_graphs(s);
         s->fuse_rupd = v;
       }
       break;
@@ -1214,10 +1202,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       if (v != s->blk_sweep) {
         // captured iterations hold the other launch sequence
         HIPCHK(hipStreamSynchronize(s->stream));
-        for (int q = 0; q < 3; q++) {
-          if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-          s->gexec[q] = nullptr;
-        }
+        drop_graphs(s);
         s->blk_sweep = v;
         s->sweep.persist = block_sweep_on(s);
       }
@@ -1229,10 +1214,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
       if (v != s->column) {
         // captured iterations hold the other launch sequence
         HIPCHK(hipStreamSynchronize(s->stream));
-        for (int q = 0; q < 3; q++) {
-          if (s->gexec[q]) hipGraphExecDestroy(s->gexec[q]);
-          s->gexec[q] = nullptr;
-        }
+        drop_graphs(s);
         s->column = v;
       }
       break;
@@ -1489,6 +1471,7 @@ int p3d_apply_prec(p3d_solver* s, double* x) {
   if (!s || !x) return fail(P3D_EINVAL, "null argument");
   const size_t nb = sizeof(double) * s->g.N;
   ensure_columns(s);
+  int rc;
   do {
     // x -> r and z -> x through the natural-order staging vector ap
     HIPCHK(hipMemcpyAsync(s->ap, x, nb, hipMemcpyHostToDevice, s->stream));
@@ -1496,9 +1479,9 @@ int p3d_apply_prec(p3d_solver* s, double* x) {
     prec_and_dot<double>(s, s->r, s->z, EPI_NONE, nullptr, false);
     launch_copy<double>(s->g, s->L, s->ap, s->z, s->stream, s->tm, 0);
     HIPCHK(hipGetLastError());
-    copy_column_flag(s);
-    HIPCHK(hipStreamSynchronize(s->stream));
-  } while (check_columns(s) == kStartOver);
+    rc = read_state(s);
+  } while (rc == kStartOver);
+  if (rc) return rc;
   HIPCHK(hipMemcpyAsync(x, s->ap, nb, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
   return P3D_OK;
@@ -1511,9 +1494,7 @@ int p3d_ilu_dinv(p3d_solver* s, float* dinv) {
   return P3D_OK;
 }
 
-int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
-  if (!s || !avg_ms || reps <= 0) return fail(P3D_EINVAL, "bad argument");
-  ensure_columns(s);
+static int time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   if (which == 2 && s->ifprec != 2) return fail(P3D_ESTATE, "no ILU preconditioner");
   if ((which == 7 || which == 11) && s->ifprec != 2)
     return fail(P3D_ESTATE, "no ILU preconditioner");
@@ -1651,9 +1632,20 @@ int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   hipEventDestroy(e0);
   hipEventDestroy(e1);
   HIPCHK(hipGetLastError());
+  if (int rc = read_state(s)) return rc;
   *avg_ms = (double)ms / reps / (grouped ? kXBatch : 1);
   if (which > 11 || which < 0) return fail(P3D_EINVAL, "unknown kernel id %d", which);
   return P3D_OK;
+}
+
+int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
+  if (!s || !avg_ms || reps <= 0) return fail(P3D_EINVAL, "bad argument");
+  ensure_columns(s);
+  int rc;
+  do {
+    rc = time_kernel(s, which, reps, avg_ms);
+  } while (rc == kStartOver);
+  return rc;
 }
 
 }  // extern "C"
