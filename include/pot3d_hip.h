@@ -167,14 +167,21 @@ enum {
                                 launch per diagonal over all blocks; -1
                                 (default) 1 below 2^26 unknowns, else 0.
                                 Same values bit for bit. */
-  P3D_OPT_COLUMN = 19        /* 8x8 columns of one wave: 1 runs each ILU sweep
-                                as one launch, a workgroup per column of
-                                points marching all planes and handing its
+  P3D_OPT_COLUMN = 19        /* 8x8 columns of points: 1 runs each ILU sweep
+                                as one launch, a workgroup per column
+                                marching all planes and handing its
                                 faces to the next columns as it goes; 0 the
                                 tile schedules above; -1 (default) 1, but 0
                                 while P3D_OPT_BLOCK_SWEEP is not -1 and for
                                 block-Jacobi register tiles of 2^22 to 2^25
-                                unknowns.  Same values bit for bit. */
+                                unknowns.  Same values bit for bit.  Calls of
+                                several threads whose columns the device
+                                would not hold together take the tiles, all
+                                but the first.  A sweep that waits about a
+                                second in vain (kept out by another process)
+                                says so on stderr; its call starts over with
+                                the tiles, and the solver keeps to them until
+                                this option is set again. */
 };
 
 /* Creates a solver for one rank's grid (nr,nt,np include the boundary /

@@ -19,13 +19,18 @@
 //
 // Termination: columns are numbered by anti-diagonal, so a column only waits
 // for columns of lower workgroup number.  Workgroups start in that order on
-// every XCD, so the lowest unfinished one is always running or next to run
-// and never waits for one that is not.  Only other kernels that wait
-// themselves could keep it from starting; every wait is bounded (kPolls polls,
-// then a flag that ends all other waits), and the solver starts the call over
-// with the tile schedules.  P3D_COLUMN_POLLS in the environment sets another
-// bound for the plans built from then on (0: a wait gives up once it has
-// polled in vain), so that this path can be tested.
+// every XCD, so of one launch the lowest unfinished one is always running or
+// next to run and never waits for one that is not.  Launches that do not wait
+// end by themselves and give their place back.  Two launches of column sweeps
+// side by side could keep each other out: one holds the places of one XCD and
+// waits for a column on another, whose places the other launch holds likewise.
+// So a call claims room for its columns (columns_claim), and takes the tile
+// schedules where the device would not hold all that are under way together.
+// What is left are other processes on the same device: every wait is bounded
+// (kPolls polls, then a flag that ends all other waits), and the solver starts
+// the call over with the tile schedules.  P3D_COLUMN_POLLS in the environment
+// sets another bound for the plans built from then on (0: a wait gives up once
+// it has polled in vain), so that this path can be tested.
 //
 // Per-point arithmetic and order are those of p3d_sweep.hip: the same bits.
 //
@@ -39,6 +44,7 @@
 // 3448 and 368 us at 101x181x361, 7.06 and 0.87 ms at 151x301x601.
 #include <stdlib.h>
 
+#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -766,6 +772,15 @@ __global__ void k_col_gather_stored(Grid3 g, int NI, int steps, int top, size_t 
   dst[t] = v;
 }
 
+// Room taken by the column sweeps under way, by device.
+constexpr int kDevices = 64;
+std::mutex room_mutex;
+long room_used[kDevices] = {};
+
+// Places that a launch of n columns may need: it goes round the 8 XCDs, so one
+// XCD gets (n + 7) / 8 of them at most.
+long room_of(int n) { return (long)n + 7; }
+
 size_t col_lds(const ColArgs& ca) {
   if (ca.mode == kStored) return sizeof(ColLdsStored);
   return sizeof(ColLds) + (ca.mode == kPhiUniform ? 0 : ca.pf_n * sizeof(float2));
@@ -793,6 +808,10 @@ namespace {
 int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int planes,
                  unsigned* failed) {
   ColArgs& ca = plan.a;
+  if (hipGetDevice(&plan.dev) != hipSuccess ||
+      hipDeviceGetAttribute(&plan.ncu, hipDeviceAttributeMultiprocessorCount, plan.dev) !=
+          hipSuccess)
+    return 1;
   const char* polls = getenv("P3D_COLUMN_POLLS");
   ca.polls = polls ? (unsigned)strtoul(polls, nullptr, 10) : kPolls;
   ca.NI = (g.a + 7) / 8;
@@ -844,6 +863,38 @@ int no_plan(ColumnPlan& plan) {
 }
 
 }  // namespace
+
+// A single launch needs no room of its own (see the head of this file).  Beside
+// others it has to fit at two columns per CU: two fit whatever their kernels
+// (kColLdsMax of 160 KB of LDS each, 256 registers at most, one wave per SIMD),
+// so a column that finds no place finds at least that many resident on every CU
+// of its XCD.
+extern "C" int p3d_columns_claim(int dev, int ncol, int ncu) {
+  if (dev < 0 || dev >= kDevices) return 0;
+  std::lock_guard<std::mutex> lock(room_mutex);
+  long& used = room_used[dev];
+  if (used > 0 && used + room_of(ncol) > 2L * ncu) return 0;
+  used += room_of(ncol);
+  return 1;
+}
+
+extern "C" void p3d_columns_release(int dev, int ncol) {
+  std::lock_guard<std::mutex> lock(room_mutex);
+  room_used[dev] -= room_of(ncol);
+}
+
+bool ColumnUse::claim(const ColumnPlan& plan) {
+  release();
+  if (!plan.ready || !p3d_columns_claim(plan.dev, plan.a.NI * plan.a.NJ, plan.ncu)) return false;
+  dev = plan.dev;
+  ncol = plan.a.NI * plan.a.NJ;
+  return true;
+}
+
+void ColumnUse::release() {
+  if (ncol) p3d_columns_release(dev, ncol);
+  ncol = 0;
+}
 
 int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const IluBlocks& bl,
                       int tk_log2, const float* dinv, unsigned* failed) {

@@ -40,6 +40,7 @@ struct ColArgs {
 
 struct ColumnPlan {
   int ready = 0;
+  int dev = 0, ncu = 0;  // device and its CUs
   ColArgs a;
   int* order = nullptr;
   float *dinv_s = nullptr, *y_s = nullptr;
@@ -60,6 +61,23 @@ int build_column_plan(ColumnPlan& plan, const Metric& m, const Grid3& g, const I
 int build_column_plan_stored(ColumnPlan& plan, const Grid3& g, const CoefArrays& co, bool wrap,
                              const float* dinv);
 void free_column_plan(ColumnPlan& plan);
+
+// Room on the device for the column sweeps of one call, from before its first
+// launch until its last one has ended.  Without it (claim false) the call takes
+// the tile schedules.
+struct ColumnUse {
+  int dev = 0, ncol = 0;
+  bool claim(const ColumnPlan& plan);
+  void release();
+  ColumnUse() = default;
+  ColumnUse(const ColumnUse&) = delete;
+  ColumnUse& operator=(const ColumnUse&) = delete;
+  ~ColumnUse() { release(); }
+};
+
+// What it counts with: columns of launches under way on a device of ncu CUs.
+extern "C" int p3d_columns_claim(int dev, int ncol, int ncu);
+extern "C" void p3d_columns_release(int dev, int ncol);
 
 // z = (LU)^-1 r on tile-major r and z, two launches.  ap (tile-major, with
 // guard): r -= alpha ap first, alpha from guard.

@@ -383,7 +383,8 @@ void external_lu_solver(double* x) {
     check(hipMemcpyAsync(G.xbuf, x, nb, hipMemcpyHostToDevice, G.stream), "copy x");
     dx = G.xbuf;
   }
-  if (G.col.ready) {
+  ColumnUse room;  // (released once the stream has been waited for)
+  if (room.claim(G.col)) {
     launch_dilu_columns_stored(G.col, G.g, dx, G.yv, G.stream);
     check(hipGetLastError(), "trisolve launch");
     unsigned failed = 0;

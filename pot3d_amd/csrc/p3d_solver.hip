@@ -109,6 +109,8 @@ struct p3d_solver {
   bool sweep_ready = false;
   ColumnPlan col;
   bool col_tried = false;  // col is the current plan, or there is none
+  bool col_room = false;   // the call under way has room for its columns
+  bool graph_cols = false;  // gexec hold column sweeps (if they hold any)
   // options
   int stop_mode = 0;
   int mixed = 0;
@@ -286,6 +288,7 @@ static int read_state(p3d_solver* s) {
   if (!s->st_host->col_failed) return P3D_OK;
   drop_graphs(s);
   free_column_plan(s->col);
+  s->col_room = s->graph_cols = false;
   s->st_host->col_failed = 0;
   HIPCHK(hipMemsetAsync(&s->st->col_failed, 0, sizeof(unsigned), s->stream));
   for (double* v : {s->r, s->z, s->ap})
@@ -315,7 +318,9 @@ static bool columns_wanted(const p3d_solver* s) {
                          s->g.N < (1u << 25);
   return !tiles_win;
 }
-static bool columns_on(const p3d_solver* s) { return columns_wanted(s) && s->col.ready; }
+static bool columns_on(const p3d_solver* s) {
+  return columns_wanted(s) && s->col.ready && s->col_room;
+}
 
 // Builds the column sweeps' plan for the current pivots, cut and placement
 // before a call that applies the ILU (every option that changes one of them
@@ -326,6 +331,27 @@ static void ensure_columns(p3d_solver* s) {
   s->col_tried = true;
   build_column_plan(s->col, s->m, s->g, s->blocks, s->tm.tk_log2, s->dinv, &s->st->col_failed);
 }
+
+// Around what a call does with the preconditioner: columns where they are
+// wanted, have a plan and find room on the device beside those of other calls
+// under way; captured iterations of the other schedule are dropped.
+struct PrecUse {
+  p3d_solver* s;
+  ColumnUse room;
+  explicit PrecUse(p3d_solver* solver) : s(solver) {
+    ensure_columns(s);
+    s->col_room = columns_wanted(s) && room.claim(s->col);
+    if (s->col_room != s->graph_cols) {
+      (void)hipStreamSynchronize(s->stream);
+      drop_graphs(s);
+      s->graph_cols = s->col_room;
+    }
+  }
+  ~PrecUse() {
+    if (s->col_room) (void)hipStreamSynchronize(s->stream);  // (an error's early return)
+    s->col_room = false;
+  }
+};
 
 // Whether the FP32 ILU apply can take the residual update (see cg_iteration).
 static bool fuse_rupd_available(const p3d_solver* s) {
@@ -743,7 +769,7 @@ static int solve_mixed_ru(p3d_solver* s, double epscg, int ncgmax) {
 static int solve_core(p3d_solver* s, double epscg, int ncgmax, int ncghist) {
   int rc;
   auto t0 = std::chrono::steady_clock::now();
-  ensure_columns(s);
+  PrecUse use(s);
   memset(&s->stats, 0, sizeof s->stats);
   if (s->guess_check) {
     // a proposed guess that is worse than the reference's zero guess is
@@ -1217,6 +1243,7 @@ int p3d_set_option(p3d_solver* s, int key, double value) {
         drop_graphs(s);
         s->column = v;
       }
+      if (!s->col.ready) s->col_tried = false;  // (also after a wait that ran out)
       break;
     }
     case P3D_OPT_TILE_K:
@@ -1470,7 +1497,7 @@ int p3d_apply_A(p3d_solver* s, const double* x, double* y) {
 int p3d_apply_prec(p3d_solver* s, double* x) {
   if (!s || !x) return fail(P3D_EINVAL, "null argument");
   const size_t nb = sizeof(double) * s->g.N;
-  ensure_columns(s);
+  PrecUse use(s);
   int rc;
   do {
     // x -> r and z -> x through the natural-order staging vector ap
@@ -1640,7 +1667,7 @@ static int time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
 
 int p3d_time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
   if (!s || !avg_ms || reps <= 0) return fail(P3D_EINVAL, "bad argument");
-  ensure_columns(s);
+  PrecUse use(s);
   int rc;
   do {
     rc = time_kernel(s, which, reps, avg_ms);

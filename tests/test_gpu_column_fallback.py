@@ -69,13 +69,18 @@ def test_solve_that_does_not_converge(monkeypatch):
 
 
 def test_single_calls(monkeypatch, capfd):
+    from pot3d_amd import _lib
     mesh = small_mesh(42, 60, 80)
     with _solver(mesh, 0, monkeypatch) as s:
         x = np.random.default_rng(1).standard_normal(s.N)
         ref = s.prec_inv(x)
     with _solver(mesh, 1, monkeypatch) as s:
-        assert np.array_equal(s.prec_inv(x), ref)
-        assert MESSAGE in capfd.readouterr().err
+        for rep in range(3):
+            # the tiles from then on, until the option is set again
+            assert np.array_equal(s.prec_inv(x), ref)
+            assert (MESSAGE in capfd.readouterr().err) == (rep != 1)
+            if rep == 1:
+                s.set_option(_lib.OPT_COLUMN, 1)
     for kid in (2, 3, 7):
         with _solver(mesh, 1, monkeypatch) as s:
             assert s.time_kernel(kid, 1) > 0
