@@ -379,7 +379,12 @@ void external_lu_solver(double* x) {
   double* dx = xv.w == W_HOST ? nullptr : (double*)xv.p;  // kernels work in place
   const size_t nb = (size_t)G.N * sizeof(double);
   if (!dx) {
-    if (!G.xbuf) check(hipMalloc((void**)&G.xbuf, nb), "allocate x");
+    if (!G.xbuf && hipMalloc((void**)&G.xbuf, nb) != hipSuccess) {
+      // the tiles do without the columns' plan
+      (void)hipGetLastError();
+      free_column_plan(G.col);
+      check(hipMalloc((void**)&G.xbuf, nb), "allocate x");
+    }
     check(hipMemcpyAsync(G.xbuf, x, nb, hipMemcpyHostToDevice, G.stream), "copy x");
     dx = G.xbuf;
   }

@@ -138,6 +138,7 @@ struct p3d_solver {
 // ---------------------------------------------------------------------------
 static int dalloc(void** p, size_t bytes) {
   if (hipMalloc(p, bytes ? bytes : 1) != hipSuccess) {
+    (void)hipGetLastError();
     *p = nullptr;
     return fail(P3D_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
   }
@@ -158,19 +159,39 @@ __global__ void k_convert(uint32_t n, const A* __restrict__ src, B* __restrict__
   if (q < n) dst[q] = (B)src[q];
 }
 
-// Memory the FP64 recurrence can do without (its x is then updated in every
-// iteration) is given back before an allocation that cannot fails.
-static int dalloc_or_yield(p3d_solver* s, void** p, size_t bytes) {
-  if (hipMalloc(p, bytes) == hipSuccess) return P3D_OK;
-  (void)hipGetLastError();
-  (void)hipStreamSynchronize(s->stream);
-  for (double*& b : s->pb64) {
-    if (b) hipFree(b);
-    b = nullptr;
+// Gives back memory that the solver can do without, one piece per call: the
+// direction buffers of the FP64 recurrence (its x is then updated in every
+// iteration), then the column sweeps' plan (the tile schedules run).  False
+// when there is none left.
+static bool yield_memory(p3d_solver* s) {
+  (void)hipGetLastError();  // (the failed allocation's)
+  if (s->pb64[0]) {
+    (void)hipStreamSynchronize(s->stream);
+    for (double*& b : s->pb64) {
+      if (b) hipFree(b);
+      b = nullptr;
+    }
+    if (s->gexec[0]) hipGraphExecDestroy(s->gexec[0]);
+    s->gexec[0] = nullptr;
+    return true;
   }
-  if (s->gexec[0]) hipGraphExecDestroy(s->gexec[0]);
-  s->gexec[0] = nullptr;
-  return dalloc(p, bytes);
+  if (s->col.ready) {
+    (void)hipStreamSynchronize(s->stream);
+    drop_graphs(s);
+    free_column_plan(s->col);
+    s->col_room = s->graph_cols = false;
+    return true;
+  }
+  return false;
+}
+
+// Every allocation of a solver that exists: it fails only when there is nothing
+// to give back.
+static int dalloc_or_yield(p3d_solver* s, void** p, size_t bytes) {
+  while (hipMalloc(p, bytes ? bytes : 1) != hipSuccess) {
+    if (!yield_memory(s)) return dalloc(p, bytes);
+  }
+  return P3D_OK;
 }
 
 static int ensure_mixed(p3d_solver* s) {
@@ -269,7 +290,7 @@ static int ensure_hist(p3d_solver* s, int ncgmax) {
   if (s->hist) hipFree(s->hist);
   s->hist = nullptr;
   s->hist_cap = 0;
-  int rc = dalloc((void**)&s->hist, sizeof(double) * want);
+  int rc = dalloc_or_yield(s, (void**)&s->hist, sizeof(double) * want);
   if (rc) return rc;
   s->hist_cap = want;
   return P3D_OK;
@@ -804,6 +825,8 @@ static int solve_core(p3d_solver* s, double epscg, int ncgmax, int ncghist) {
     HIPCHK(hipStreamSynchronize(s->stream));
   } else {
     launch_copy<double>(s->g, s->L, s->r, s->b, s->stream, s->tm, 1);
+    // (the history first: its memory may take that of the direction buffers)
+    if ((rc = ensure_hist(s, ncgmax))) return rc;
     if ((rc = pcg<double>(s, fp64_vecs(s), epscg, ncgmax, s->stop_mode))) return rc;
     print_history(s, ncghist);
     s->stats.ncg = s->st_host->ncg;
@@ -829,9 +852,9 @@ static int solve_core(p3d_solver* s, double epscg, int ncgmax, int ncghist) {
 static int factor_ilu(p3d_solver* s) {
   double* dpiv = nullptr;
   unsigned* bad = nullptr;
-  int rc = dalloc((void**)&dpiv, sizeof(double) * s->g.N);
+  int rc = dalloc_or_yield(s, (void**)&dpiv, sizeof(double) * s->g.N);
   if (rc) return rc;
-  if ((rc = dalloc((void**)&bad, sizeof(unsigned)))) {
+  if ((rc = dalloc_or_yield(s, (void**)&bad, sizeof(unsigned)))) {
     hipFree(dpiv);
     return rc;
   }
@@ -1152,9 +1175,11 @@ static int rebuild_ilu(p3d_solver* s, bool refactor) {
   int dev = 0, ncu = 0;
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const int prc =
-      build_sweep_plan(s->sweep, s->g, ncu, s->tile_k, s->tile_waves, &s->blocks, s->dinv,
-                       s->tile_stage, &s->m);
+  int prc;
+  do {
+    prc = build_sweep_plan(s->sweep, s->g, ncu, s->tile_k, s->tile_waves, &s->blocks, s->dinv,
+                           s->tile_stage, &s->m);
+  } while (prc == 1 && yield_memory(s));  // (1: no memory)
   s->sweep_ready = prc == 0;
   s->sweep.persist = block_sweep_on(s);
   int rc = update_tilemap(s);
@@ -1296,7 +1321,7 @@ int p3d_set_br1(p3d_solver* s, const double* br1) {
     return P3D_OK;
   }
   if (!s->br1) {
-    int rc = dalloc((void**)&s->br1, sizeof(double) * s->nt * s->np);
+    int rc = dalloc_or_yield(s, (void**)&s->br1, sizeof(double) * s->nt * s->np);
     if (rc) return rc;
   }
   HIPCHK(hipMemcpy(s->br1, br1, sizeof(double) * s->nt * s->np, hipMemcpyHostToDevice));
@@ -1393,8 +1418,9 @@ int p3d_history(p3d_solver* s, double* hist, int n) {
 static int ensure_phi(p3d_solver* s) {
   if (s->phi) return P3D_OK;
   int rc;
-  if ((rc = dalloc((void**)&s->phi, sizeof(double) * s->nr * s->nt * s->np))) return rc;
-  if ((rc = dalloc((void**)&s->sums, sizeof(double) * 2 * s->nr))) return rc;
+  if ((rc = dalloc_or_yield(s, (void**)&s->phi, sizeof(double) * s->nr * s->nt * s->np)))
+    return rc;
+  if ((rc = dalloc_or_yield(s, (void**)&s->sums, sizeof(double) * 2 * s->nr))) return rc;
   return P3D_OK;
 }
 
@@ -1428,7 +1454,8 @@ int p3d_energy(p3d_solver* s, const double* phi, double* w, double* br, double* 
                           s->stream));
   if (!s->e_partial) {
     s->eG = s->L.G;
-    if ((rc = dalloc((void**)&s->e_partial, sizeof(double) * 3 * (s->eG + kRedCounters))))
+    if ((rc = dalloc_or_yield(s, (void**)&s->e_partial,
+                              sizeof(double) * 3 * (s->eG + kRedCounters))))
       return rc;
   }
   launch_energy(s->em, nr, nt, np, s->phi, s->e_partial, s->red.counter + 8 * kRedSlotWords,
@@ -1445,7 +1472,7 @@ int p3d_energy(p3d_solver* s, const double* phi, double* w, double* br, double* 
     double *dbr, *dbt, *dbp;
     const size_t nbr = (size_t)(nr - 1) * nt * np, nbt = (size_t)nr * (nt - 1) * np,
                  nbp = (size_t)nr * nt * (np - 1);
-    if ((rc = dalloc((void**)&dbr, sizeof(double) * (nbr + nbt + nbp)))) return rc;
+    if ((rc = dalloc_or_yield(s, (void**)&dbr, sizeof(double) * (nbr + nbt + nbp)))) return rc;
     dbt = dbr + nbr;
     dbp = dbt + nbt;
     launch_getb(s->em, nr, nt, np, s->phi, dbr, dbt, dbp, s->stream);
@@ -1467,8 +1494,8 @@ int p3d_apply_A(p3d_solver* s, const double* x, double* y) {
     // the FP32 operator of the mixed recurrence, natural-order output
     float *xf = nullptr, *yf = nullptr;
     int rc;
-    if ((rc = dalloc((void**)&xf, s->g.N * sizeof(float))) ||
-        (rc = dalloc((void**)&yf, s->g.N * sizeof(float)))) {
+    if ((rc = dalloc_or_yield(s, (void**)&xf, s->g.N * sizeof(float))) ||
+        (rc = dalloc_or_yield(s, (void**)&yf, s->g.N * sizeof(float)))) {
       hipFree(xf);
       return rc;
     }
