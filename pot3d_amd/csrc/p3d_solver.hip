@@ -194,19 +194,20 @@ static int dalloc_or_yield(p3d_solver* s, void** p, size_t bytes) {
   return P3D_OK;
 }
 
+// (A call that found no memory for all of them leaves what it got to the next.)
 static int ensure_mixed(p3d_solver* s) {
-  if (s->x32) return P3D_OK;
+  if (s->z32) return P3D_OK;
   const size_t nb = (size_t)s->g.N * sizeof(float), nv = s->nvec * sizeof(float);
-  int rc;
-  if ((rc = dalloc_or_yield(s, (void**)&s->x32, nb)) ||
-      (rc = dalloc_or_yield(s, (void**)&s->r32, nv)) ||
-      (rc = dalloc_or_yield(s, (void**)&s->p32, nb)) ||
-      (rc = dalloc_or_yield(s, (void**)&s->ap32, nv)) ||
-      (rc = dalloc_or_yield(s, (void**)&s->z32, nv)))
-    return rc;
-  HIPCHK(hipMemsetAsync(s->r32, 0, nv, s->stream));
-  HIPCHK(hipMemsetAsync(s->z32, 0, nv, s->stream));
-  HIPCHK(hipMemsetAsync(s->ap32, 0, nv, s->stream));
+  struct {
+    float** p;
+    size_t bytes;
+  } bufs[] = {{&s->x32, nb}, {&s->r32, nv}, {&s->p32, nb}, {&s->ap32, nv}, {&s->z32, nv}};
+  for (auto& b : bufs) {
+    if (*b.p) continue;
+    const int rc = dalloc_or_yield(s, (void**)b.p, b.bytes);
+    if (rc) return rc;
+    HIPCHK(hipMemsetAsync(*b.p, 0, b.bytes, s->stream));
+  }
   return P3D_OK;
 }
 
@@ -1416,9 +1417,10 @@ int p3d_history(p3d_solver* s, double* hist, int n) {
 }
 
 static int ensure_phi(p3d_solver* s) {
-  if (s->phi) return P3D_OK;
+  if (s->sums) return P3D_OK;
   int rc;
-  if ((rc = dalloc_or_yield(s, (void**)&s->phi, sizeof(double) * s->nr * s->nt * s->np)))
+  if (!s->phi &&
+      (rc = dalloc_or_yield(s, (void**)&s->phi, sizeof(double) * s->nr * s->nt * s->np)))
     return rc;
   if ((rc = dalloc_or_yield(s, (void**)&s->sums, sizeof(double) * 2 * s->nr))) return rc;
   return P3D_OK;

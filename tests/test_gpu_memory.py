@@ -89,6 +89,28 @@ def test_options_in_little_memory():
         assert np.array_equal(a, b)
 
 
+def test_mixed_solve_after_one_without_memory():
+    """A call that finds memory for some of the FP32 vectors only, twice, and
+    then for all."""
+    from pot3d_amd import _lib, solver
+    mesh = small_mesh(152, 202, 402)  # the five vectors take 48 MB each and more
+    out = []
+    for leave in (None, 130 * MB):
+        with solver.Pot3dSolver(mesh, -1.0, 1) as s:
+            s.set_br0(random_br0(mesh, 1))
+            s.set_option(_lib.OPT_MIXED, 2)
+            x = np.zeros(s.N)
+            if leave:
+                with _leave(leave):
+                    for _ in range(2):
+                        with pytest.raises(_lib.Pot3dError) as e:
+                            s.solve(x, None, 1e-9, ncgmax=9)
+                        assert e.value.code == _lib.P3D_ENOMEM
+            s.solve(x, None, 1e-9, ncgmax=9)
+            out.append(x)
+    assert np.array_equal(out[0], out[1])
+
+
 def test_legacy_lu_host_vector_in_little_memory():
     from pot3d_amd import _lib
     L = _lib.load()
