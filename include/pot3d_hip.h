@@ -362,8 +362,9 @@ int p3d_nn_prolong_dev_noalloc(int nrc, int ntc, int npc, const double* phic_dev
                                int cf, const int* ir, const double* wr, const int* it,
                                const double* wt, const int* ip, const double* wp,
                                double* xf_dev);
-/* One 16x16x16 BF16 matrix-core product D = A B (row-major BF16 bits in,
- * FP32 out), for checking the operand layout the network kernels use. */
+/* D = A B of 16x16 matrices (row-major BF16 bits in, FP32 out) by the matrix-
+ * core instruction (16x16x32) and the transposing LDS read that the network
+ * kernels use, for checking their operand layout. */
 int p3d_nn_mfma_check(const unsigned short* A, const unsigned short* B, float* D);
 
 #ifdef __cplusplus

@@ -596,7 +596,7 @@ int p3d_nn_prolong_dev_noalloc(int nrc, int ntc, int npc, const double* phic_dev
   return P3D_OK;
 }
 
-// One 16x16x16 BF16 MFMA: D = A*B (A, B row-major BF16 bits, D FP32).
+// D = A*B of 16x16 matrices on the matrix cores (A, B row-major BF16 bits, D FP32).
 int p3d_nn_mfma_check(const uint16_t* A, const uint16_t* B, float* D) {
   uint16_t *dA = nullptr, *dB = nullptr;
   float* dD = nullptr;

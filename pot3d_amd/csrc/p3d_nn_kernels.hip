@@ -12,8 +12,8 @@
 // MFMA 16x16x32 operand layout (lane l of a wave64): A row l%16 and B column
 // l%16, each with the eight k of group l/16 (the order of the k does not
 // matter as long as A and B agree); D (16 x 16): lane holds D[4*(l/16) ..
-// 4*(l/16)+3][l%16].  p3d_nn_mfma_check compares the 16x16x16 form, whose
-// groups hold four k, with a host matmul.
+// 4*(l/16)+3][l%16].  p3d_nn_mfma_check is there to compare it, and the
+// transposing LDS read, with a host matmul.
 //
 // Every BF16 tensor is preceded by kZeroFront zero bytes (the allocation's
 // first ones): a tap that falls outside the grid reads those.
@@ -39,10 +39,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
   return (uint16_t)(u >> 16);
 }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-
-__device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
 
 __device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
@@ -834,21 +830,25 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// A 16x16x16 MFMA on given matrices (A row-major MxK, B row-major KxN, BF16
-// bits) -> D (FP32, row-major): used to check the operand layout.
-__global__ void k_mfma_check(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                             float* __restrict__ D) {
-  const int l = threadIdx.x;
-  bf16x4 a, b;
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    a[q] = (short)A[(l % 16) * 16 + 4 * (l / 16) + q];
-    b[q] = (short)B[(4 * (l / 16) + q) * 16 + (l % 16)];
-  }
+// D = A B for 16 x 16 matrices (A row-major MxK, B row-major KxN, BF16 bits; D
+// FP32, row-major) as the convolutions and weight gradients form it: 16x16x32
+// products, A's rows as they lie in memory, B through the transposing LDS read.
+// Each half of the 32 k holds the product once, the other one zeros, so D is
+// half their sum.
+__global__ void __launch_bounds__(64)
+    k_mfma_check(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                 float* __restrict__ D) {
+  __shared__ u32x4 sb[32];
+  const int l = threadIdx.x, m = l & 15, kb = l >> 4;
+  if (l < 32) sb[l] = ((const u32x4*)B)[l];
+  __syncthreads();
+  const uint2 a = *(const uint2*)(A + m * 16 + 4 * kb);
+  const uint2 b = lds_read_tr((const uint16_t*)sb + (4 * kb + (m >> 2)) * 16 + (m & 3) * 4);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  acc = mfma16(a, b, acc);
+  acc = mfma32(u32x4{a.x, a.y, 0u, 0u}, u32x4{b.x, b.y, 0u, 0u}, acc);
+  acc = mfma32(u32x4{0u, 0u, a.x, a.y}, u32x4{0u, 0u, b.x, b.y}, acc);
 #pragma unroll
-  for (int i = 0; i < 4; i++) D[(4 * (l / 16) + i) * 16 + (l % 16)] = acc[i];
+  for (int i = 0; i < 4; i++) D[(4 * kb + i) * 16 + m] = 0.5f * acc[i];
 }
 
 // ---------------------------------------------------------------------------
