@@ -1167,64 +1167,40 @@ void launch_r_update(uint32_t n_all, const Launch& Lt, float* r, const float* ap
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     k_p_update(Grid3 g, int G, int prec, const float* __restrict__ dg, T* __restrict__ p,
-               const T* __restrict__ r, const T* __restrict__ z, CgState* st, TileMap tm,
-               double* __restrict__ xs, const double* __restrict__ xscale,
-               unsigned* counter) {
-  // With xs (FP32 recurrence, FP64 solution): first the solution update of
-  // the iteration whose alpha is current, xs += (alpha scale) p_old, once per
-  // iteration, including the iteration that set done (CgState::x_ncg counts
-  // the applied updates; the last workgroup advances it, after every
-  // workgroup has read it); then p = z + beta p_old unless done.
-  const int done = st_done(st);
-  const int ncg = xs ? st_load_int(&st->ncg) : 0;
-  const bool do_x = xs && st_load_int(&st->x_ncg) < ncg;
-  if (done && !do_x) return;
+               const T* __restrict__ r, const T* __restrict__ z, const CgState* st, TileMap tm) {
+  if (st_done(st)) return;
   const uint32_t n1 = g.N;
   const bool diag = prec == PREC_DIAG;
   const T beta = (T)st_load(&st->beta);
-  const double alpha_x = do_x ? st_load(&st->alpha) * *xscale : 0.0;
-  // 16 points per thread in flight, and the p and solution streams read
-  // (and the solution written) non-temporally: neither is reused before it
-  // has left the caches, and keeping them out leaves room for the gathered
-  // z (measured: 1.60 -> 1.27 ms at 214.7 M points)
+  // 16 points per thread in flight, and p read non-temporally: it is not
+  // reused before it has left the caches, and keeping it out leaves room for
+  // the gathered z
   constexpr int kU = 16;
   // grid-stride over runs of kU kBlock points in dispatch order: the
   // workgroups in flight stream one window of the vectors together
   for (uint32_t nb = blockIdx.x * (kU * kBlock) + threadIdx.x; nb < n1;
        nb += (uint32_t)G * (kU * kBlock)) {
     T pv[kU], zv[kU];
-    double xv[kU];
     float dv[kU];
 #pragma unroll
     for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
       pv[u] = zv[u] = (T)0;
-      xv[u] = 0.0;
       dv[u] = 0.f;
       if (n < n1) {
         if (diag) dv[u] = dg[n];
         pv[u] = __builtin_nontemporal_load(p + n);
-        if (do_x) xv[u] = __builtin_nontemporal_load(xs + n);
-        if (!done) zv[u] = (prec == PREC_ILU) ? z[tmap(tm, g, n)] : r[n];
+        zv[u] = (prec == PREC_ILU) ? z[tmap(tm, g, n)] : r[n];
       }
     }
 #pragma unroll
     for (int u = 0; u < kU; u++) {
       const uint32_t n = nb + u * kBlock;
       if (n < n1) {
-        if (do_x) __builtin_nontemporal_store(xv[u] + alpha_x * (double)pv[u], xs + n);
-        if (!done) {
-          const T zn = diag ? (T)dv[u] * zv[u] : zv[u];
-          p[n] = beta * pv[u] + zn;
-        }
+        const T zn = diag ? (T)dv[u] * zv[u] : zv[u];
+        p[n] = beta * pv[u] + zn;
       }
     }
-  }
-  if (do_x) {
-    // only the reads of x_ncg must precede its update
-    __syncthreads();
-    if (threadIdx.x == 0 && count_in(counter, G))
-      __hip_atomic_store(&st->x_ncg, ncg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -1360,10 +1336,10 @@ void launch_p_update_x(const Grid3& g, const Launch& L, int prec, int t, const P
 
 template <typename T>
 void launch_p_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* p,
-                     const T* r, const T* z, CgState* st, hipStream_t s, const TileMap& tm,
-                     double* xs, const double* xscale, unsigned* counter) {
+                     const T* r, const T* z, const CgState* st, hipStream_t s,
+                     const TileMap& tm) {
   const int G = sizeof(T) == 8 && L.Gp > 0 ? L.Gp : L.G;
-  k_p_update<T><<<G, kBlock, 0, s>>>(g, G, prec, dg, p, r, z, st, tm, xs, xscale, counter);
+  k_p_update<T><<<G, kBlock, 0, s>>>(g, G, prec, dg, p, r, z, st, tm);
 }
 
 // s0 = x.y, s1 = u.v
@@ -1976,8 +1952,8 @@ void launch_getb(const EnergyMesh& em, int nr, int nt, int np, const double* phi
                                      const T*, const float*, CgState*, hipStream_t,             \
                                      const TileMap&, double*, const double*, unsigned*);        \
   template void launch_p_update<T>(const Grid3&, const Launch&, int, const float*, T*,          \
-                                   const T*, const T*, CgState*, hipStream_t, const TileMap&,   \
-                                   double*, const double*, unsigned*);                          \
+                                   const T*, const T*, const CgState*, hipStream_t,             \
+                                   const TileMap&);                                             \
   template void launch_dot2<T>(const Grid3&, const Launch&, const T*, const T*, const T*,       \
                                const T*, CgState*, Reduce, int, Epi, double*, bool,             \
                                hipStream_t, const TileMap&);                                    \

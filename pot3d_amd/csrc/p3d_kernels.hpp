@@ -175,14 +175,10 @@ void launch_p_update_x(const Grid3& g, const Launch& L, int prec, int t, const P
 
 // p = z + beta p (z = M^-1 r computed in place for DIAG/NONE, read for ILU).
 // tm: placement of r (cg_update) and z (p_update) (natural by default).
-// With xs (FP32 recurrence, FP64 solution) it first applies the pending
-// solution update xs += (alpha * *xscale) p, once per iteration
-// (CgState::x_ncg; counter: a reduction slot's counter).
 template <typename T>
 void launch_p_update(const Grid3& g, const Launch& L, int prec, const float* dg, T* p,
-                     const T* r, const T* z, CgState* st, hipStream_t s,
-                     const TileMap& tm = TileMap{}, double* xs = nullptr,
-                     const double* xscale = nullptr, unsigned* counter = nullptr);
+                     const T* r, const T* z, const CgState* st, hipStream_t s,
+                     const TileMap& tm = TileMap{});
 
 // Generic fused dot: s0 = x.y, s1 = u.v (v/u may be null), epilogue epi.
 // All four vectors are placed by tm; the sums run in natural point order.
