@@ -510,12 +510,11 @@ __global__ void __launch_bounds__(256)
 // out[e] = sum over chunks (fixed order) of part[chunk][e]: 64 elements a
 // block, 16 threads each (one would read the chunks one after the other: 38
 // us for 381 of them).
-__global__ void __launch_bounds__(1024)
-    k_reduce_chunks(int nchunk, size_t n, const float* __restrict__ part,
-                    float* __restrict__ out) {
-  __shared__ float sh[16][64];
+__device__ __forceinline__ void reduce_chunks(int block, int nchunk, size_t n,
+                                              const float* __restrict__ part,
+                                              float* __restrict__ out, float (*sh)[64]) {
   const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const size_t e = (size_t)blockIdx.x * 64 + l;
+  const size_t e = (size_t)block * 64 + l;
   float s = 0.f;
   if (e < n)
 #pragma unroll 8
@@ -528,6 +527,13 @@ __global__ void __launch_bounds__(1024)
     for (int q = 0; q < 16; q++) r += sh[q][l];
     out[e] = r;
   }
+}
+
+__global__ void __launch_bounds__(1024)
+    k_reduce_chunks(int nchunk, size_t n, const float* __restrict__ part,
+                    float* __restrict__ out) {
+  __shared__ float sh[16][64];
+  reduce_chunks(blockIdx.x, nchunk, n, part, out, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -669,7 +675,7 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
 
 // L = mean_v (out[v] - t[v])^2 (out FP32, the head's channel 0; its other 15
 // channels have no gradient): part the loss's partial sums, one per 256
-// consecutive voxels whatever the grid of blocks (k_sum_in_order), bpart
+// consecutive voxels whatever the grid of blocks (k_loss_sums), bpart
 // [block][16] those of the head's bias gradient, dy the gradient as BF16
 // operand.  An FP64 target is divided by its scale here.
 __global__ void __launch_bounds__(256)
@@ -699,19 +705,26 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x < 16) bpart[blockIdx.x * 16 + threadIdx.x] = threadIdx.x == 0 ? gs : 0.f;
 }
 
-// *out = scale * (part[0] + part[1] + ... in this order).  The loss is this sum
-// over its groups of 256 voxels, so its order belongs to the result (a tree
-// over 1024 blocks' sums moved it by up to 2e-6 of itself).  One lane adds, out
-// of LDS, what all have loaded: one load after the other from memory took 141
-// us for the 3050 groups of 51x91x181.
-__global__ void __launch_bounds__(256)
-    k_sum_in_order(int n, const float* __restrict__ part, float* __restrict__ out, float scale) {
+// What follows k_mse.  Block 0: *loss = scale * (part[0] + part[1] + ... in this
+// order).  The loss is this sum over its groups of 256 voxels, so its order
+// belongs to the result (a tree over 1024 blocks' sums moved it by up to 2e-6
+// of itself).  One lane adds, out of LDS, what all have loaded; the chain of
+// additions bounds it: the 3050 groups of 51x91x181 take 141 us with one load
+// after the other from memory, 15 us so.  Block 1: the head's bias gradient
+// from its nb partial sums.
+__global__ void __launch_bounds__(1024)
+    k_loss_sums(int n, const float* __restrict__ part, float* __restrict__ loss, float scale,
+                int nb, const float* __restrict__ bpart, float* __restrict__ gb) {
   constexpr int kC = 4096;
   __shared__ f32x4 sh[kC / 4];
+  if (blockIdx.x == 1) {
+    reduce_chunks(0, nb, 16, bpart, gb, (float(*)[64])sh);
+    return;
+  }
   float s = 0.f;
   for (int n0 = 0; n0 < n; n0 += kC) {
 #pragma unroll
-    for (int u = 0; u < kC; u += 256) {
+    for (int u = 0; u < kC; u += 1024) {
       const int i = n0 + u + (int)threadIdx.x;
       ((float*)sh)[u + threadIdx.x] = i < n ? part[i] : 0.f;
     }
@@ -730,7 +743,7 @@ __global__ void __launch_bounds__(256)
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = s * scale;
+  if (threadIdx.x == 0) *loss = s * scale;
 }
 
 // Adam (bias-corrected) on FP32 weights; refreshes the BF16 copy when wb.
@@ -989,8 +1002,8 @@ void mse(int V, const float* out, const float* tgt, const double* tgt64, double 
          uint16_t* dy, float* part, float* bpart, float* loss, float* gb, hipStream_t s) {
   const unsigned nb = sum_blocks(V);
   k_mse<<<nb, 256, 0, s>>>(V, out, tgt, tgt64, tscale, dy, part, bpart);
-  k_sum_in_order<<<1, 256, 0, s>>>((V + 255) / 256, part, loss, 1.0f / (float)V);
-  k_reduce_chunks<<<1, 1024, 0, s>>>((int)nb, 16, bpart, gb);
+  k_loss_sums<<<2, 1024, 0, s>>>((V + 255) / 256, part, loss, 1.0f / (float)V, (int)nb, bpart,
+                                 gb);
 }
 void adam(size_t n, float* w, const float* g, float* m1, float* m2, float lr, float b1,
           float b2, float eps, int step, uint16_t* wb, hipStream_t s) {
