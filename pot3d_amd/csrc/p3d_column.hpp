@@ -7,7 +7,10 @@
 
 namespace p3d {
 
-// LDS of one column at most (beyond about 5000 planes: the tile schedules)
+// LDS of one column at most.  Phi factors that are not all equal, or a phi cut,
+// take a table of 8 bytes per plane beside the 34 KB of rows: beyond about 3780
+// planes the tile schedules run.  Equal factors without a cut and stored
+// couplings need no table.
 constexpr size_t kColLdsMax = 64 * 1024;
 
 struct ColArgs {

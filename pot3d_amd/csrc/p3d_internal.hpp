@@ -206,7 +206,8 @@ struct CgState {
   unsigned col_failed;  // a wait of a column sweep ran into its bound
 };
 
-// Iterations per update of the FP64 solution (the p update's group; directions of a group live in kXBatch rotating buffers).
+// Iterations per update of the FP64 solution (the p update's group; directions
+// of a group live in kXBatch rotating buffers).
 constexpr int kXBatch = 4;
 template <typename T>
 struct PBuf {

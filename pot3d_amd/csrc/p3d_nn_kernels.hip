@@ -78,7 +78,8 @@ __device__ __forceinline__ void coords(const Dims& d, int v, int& x, int& y, int
 // it.  MT tiles share a weight fragment and give the loads of one step
 // something to overlap with.  The eight convolutions of a forward pass at
 // 51x91x181: 1123 us with one 16 x 16 tile a wave and 8-byte operands, 394 us
-// so.
+// with this kernel alone, 296 us with k_conv_lds for 32 channels and more and
+// DIR known to the compiler (the three of 16 channels here 38, 38 and 13 us).
 struct ConvOut {
   uint16_t* y;        // BF16 result (after the ReLU), or null
   const uint16_t* e;  // BF16 skip input, or null
@@ -243,8 +244,8 @@ __global__ void __launch_bounds__(256)
 // straight from memory the 27 taps take each voxel 27 times through L1, which
 // does not hold the neighbourhoods of a CU's workgroups; so it comes in three
 // times (and its edges).  At 51x91x181: 32->16 channels at 780 thousand
-// voxels 104 -> 60 us, 64->32 at 101 thousand 101 -> 60 us, 128->64 at 13
-// thousand 75 -> 56 us.
+// voxels 104 -> 63 us, 64->32 at 101 thousand 101 -> 60 us, 128->64 at 13
+// thousand 75 -> 55 us.
 // A row's 16-byte words are stored exchanged by the row's number, so that the
 // 16 rows of a read lie in different banks.
 template <int CIN>
@@ -813,7 +814,7 @@ __global__ void k_head_to_x(int V, const float* __restrict__ out, double scale,
 // coarse padded index and weight of the upper neighbour), phi periodic.
 // One thread per point of a fine plane; its place in the plane by 32-bit
 // arithmetic, the plane by the block (64-bit divisions of a flat index were
-// most of the kernel: 128 us for 149x299x599 points, 94 us so).
+// most of the kernel: 128 us for 149x299x599 points, 98 us so).
 __global__ void __launch_bounds__(256)
     k_prolong(int af, int bf, int cf, int nrc, int ntc, int npc,
                           const double* __restrict__ phic, const int* __restrict__ ir,
