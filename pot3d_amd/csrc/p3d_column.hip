@@ -813,7 +813,7 @@ int plan_columns(ColumnPlan& plan, const Grid3& g, const IluBlocks& bl, int plan
           hipSuccess)
     return 1;
   const char* polls = getenv("P3D_COLUMN_POLLS");
-  ca.polls = polls ? (unsigned)strtoul(polls, nullptr, 10) : kPolls;
+  ca.polls = polls && *polls ? (unsigned)strtoul(polls, nullptr, 10) : kPolls;
   ca.NI = (g.a + 7) / 8;
   ca.NJ = (g.b + 7) / 8;
   ca.c = g.c;

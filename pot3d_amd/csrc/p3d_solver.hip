@@ -1556,13 +1556,14 @@ static int time_kernel(p3d_solver* s, int which, int reps, double* avg_ms) {
     return fail(P3D_ESTATE, "no ILU preconditioner");
   if ((which == 8 || which == 9 || which == 10 || which == 11) && !s->tm.on)
     return fail(P3D_ESTATE, "no tile-major placement (single-wave ILU tile sweeps)");
-  if (which == 11 && !fuse_rupd_available(s))
-    return fail(P3D_ESTATE, "no register-tile ILU sweeps (P3D_OPT_TILE_STAGE 2)");
   if (which == 1 || which == 3 || which >= 7) {
     int rc = ensure_mixed(s);
     if (!rc && which == 8) rc = ensure_pbuf(s);
     if (rc) return rc;
   }
+  // (looked at now: the vectors' memory may have taken the columns' plan)
+  if (which == 11 && !fuse_rupd_available(s))
+    return fail(P3D_ESTATE, "no register-tile ILU sweeps (P3D_OPT_TILE_STAGE 2)");
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));

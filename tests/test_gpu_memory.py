@@ -89,6 +89,21 @@ def test_options_in_little_memory():
         assert np.array_equal(a, b)
 
 
+def test_kernel_timing_that_takes_the_columns_plan():
+    """Timing the residual update in the forward sweep needs the columns (or
+    register tiles): an error where the vectors take their plan's memory."""
+    from pot3d_amd import _lib, solver
+    with solver.Pot3dSolver(small_mesh(152, 202, 402), -1.0, 2) as s:
+        s.prec_inv(np.zeros(s.N))  # builds the plan, about 130 MB
+        with _leave(150 * MB):  # the vectors take 250 MB
+            for _ in range(2):
+                with pytest.raises(_lib.Pot3dError) as e:
+                    s.time_kernel(11, 1)
+                assert e.value.code == _lib.P3D_ESTATE
+        s.set_option(_lib.OPT_COLUMN, -1)
+        assert s.time_kernel(11, 1) > 0
+
+
 def test_mixed_solve_after_one_without_memory():
     """A call that finds memory for some of the FP32 vectors only, twice, and
     then for all."""
