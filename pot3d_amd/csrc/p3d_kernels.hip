@@ -138,9 +138,8 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
     if (lane == 0) sh[q][w] = s;
   }
   __syncthreads();
-  CgState c;  // for the epilogue, loaded while the count-in is under way
+  CgState c;  // for the epilogue
   if (threadIdx.x == 0) {
-    if (st) c = st_snapshot(st);
 #pragma unroll
     for (int q = 0; q < NV; q++) {
       double s = 0.0;
@@ -149,6 +148,8 @@ __device__ void block_finish_bs(double (&v)[NV], double* partial, unsigned* coun
     }
     __hip_atomic_store(counter + (1 + grp) * kRedStride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned prev = arrive(counter);
+    // asked for behind the count-in, which waits for what was asked for before
+    if (st) c = st_snapshot(st);
     amlast = (prev == (unsigned)ngrp - 1);
   }
   __syncthreads();
